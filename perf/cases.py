@@ -1,0 +1,420 @@
+"""Performance cases: the calls a program makes on the RNS-CKKS backend, through its Python binding.
+
+Each case names a parameter set and an operation with its sizes. `prepare` makes what a program
+holds before the call (a context per parameter set, keys, ciphertexts resident on the device),
+`run` is one call or one short chain of calls, and the outputs are the resulting polynomials.
+Residues are uniform below their primes, as those of every ciphertext and key in NTT form are.
+"""
+import math
+import os
+import random
+import sys
+
+import numpy as np
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ckks-train_amd"))
+import ckh  # noqa: E402
+
+# Parameter sets: (log2 N, data prime bits, special prime bits, digits).
+SETS = {
+    "n12": (12, [50] * 6, [60] * 2, 3),             # the smallest ring: development and short circuits
+    "n13": (13, [50] * 6, [60] * 2, 2),             # a shallow circuit with three-prime digits
+    "n13_ntt": (13, [50] * 4, [60], 1),             # the plain transform configuration
+    "n14": (14, [60] + [40] * 5, [60] * 2, 3),      # a 60-bit first prime above 40-bit ones
+    "n15": (15, [50] * 20, [60] * 4, 5),            # matrix-vector products
+    "n16": (16, [50] * 24, [60] * 6, 4),            # the headline key switch
+}
+SCALE = 2.0 ** 40
+SERVED = ("relinearize", "hoisted", "relinearize", "product")  # a served mix, in arrival order
+
+
+def listed():
+    return [
+        # one transform there and back of a four-limb polynomial: the smallest call
+        {"name": "round_trip_n13", "op": "round_trip", "set": "n13_ntt", "limbs": 4},
+        # one key switch in the smallest ring: launches and latency
+        {"name": "switch_n12", "op": "switch", "set": "n12", "limbs": 6},
+        # one multiplication step of a circuit (product, relinearization, rescale), last digit clipped
+        {"name": "product_n14", "op": "product", "set": "n14", "limbs": 5},
+        # one rotation at a level that ends inside a digit
+        {"name": "rotate_n15", "op": "rotate", "set": "n15", "limbs": 13},
+        # one key switch at the top of the headline set: the single-call latency
+        {"name": "switch_n16", "op": "switch", "set": "n16", "limbs": 24},
+        # a minibatch's relinearizations at uneven levels in a small ring
+        {"name": "relin_batch_n13", "op": "relin_batch", "set": "n13", "count": 64, "lo": 2, "hi": 6, "mix": 7},
+        # the headline workload: 256 polynomials of 4 to 24 limbs under one key
+        {"name": "switch_batch_n16", "op": "switch_batch", "set": "n16", "count": 256, "lo": 4, "hi": 24, "mix": 1},
+        # sixteen rotations of one ciphertext sharing a decomposition
+        {"name": "hoisted_n16", "op": "hoisted", "set": "n16", "limbs": 19, "count": 16},
+        # the baby-step giant-step product with 64 plaintext diagonals
+        {"name": "matvec_n15", "op": "matvec", "set": "n15", "limbs": 20, "baby": 32, "giant": 32, "per_block": 2},
+        # a small product with encrypted diagonals, as in training on encrypted weights
+        {"name": "matvec_enc_n14", "op": "matvec_enc", "set": "n14", "limbs": 6, "baby": 4, "giant": 4, "per_block": 4},
+        # two CoeffToSlot stages of a bootstrap
+        {"name": "coeff_to_slot_n15", "op": "coeff_to_slot", "set": "n15", "limbs": 18, "baby": 4, "giant": 4},
+        # a burst of mixed requests through the serving loop
+        {"name": "served_n15", "op": "served", "set": "n15", "count": 24, "lo": 4, "hi": 20, "mix": 5},
+    ]
+
+
+def _log_uniform(rng, lo, hi):
+    return min(hi, max(lo, int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))))
+
+
+def draw(rng):
+    op = rng.choice(["round_trip", "switch", "product", "rotate", "relin_batch", "switch_batch", "hoisted", "matvec",
+                     "matvec_enc", "coeff_to_slot", "served"])
+    if op in ("matvec_enc", "coeff_to_slot"):
+        name = rng.choice(["n13", "n14", "n15"])
+    elif op in ("matvec", "served"):
+        name = rng.choice(["n13", "n14", "n15", "n16"])
+    else:
+        name = rng.choice(["n12", "n13", "n14", "n15", "n16"])
+    top = len(SETS[name][1])
+    case = {"op": op, "set": name}
+    if op == "round_trip":
+        case["limbs"] = rng.randint(1, top)
+    elif op in ("switch", "rotate"):
+        case["limbs"] = rng.randint(1, top)
+    elif op == "product":
+        case["limbs"] = rng.randint(2, top)
+    elif op in ("relin_batch", "switch_batch", "served"):
+        lo = rng.randint(2, max(2, top // 2))
+        hi = rng.randint(lo, top)
+        case.update(count=_log_uniform(rng, 2, 32 if op == "served" else 200), lo=lo, hi=hi, mix=rng.randint(0, 10 ** 6))
+    elif op == "hoisted":
+        case.update(limbs=rng.randint(1, top), count=_log_uniform(rng, 2, 24))
+    elif op == "matvec":
+        baby = rng.choice([4, 8, 16, 32])
+        case.update(limbs=rng.randint(2, top), baby=baby, giant=rng.choice([2, 4, 8, 16]), per_block=rng.randint(1, 4))
+    elif op == "matvec_enc":
+        case.update(limbs=rng.randint(2, min(top, 12)), baby=rng.choice([2, 4, 8]), giant=rng.choice([2, 4]),
+                    per_block=rng.randint(1, 2))
+    else:
+        case.update(limbs=rng.randint(3, top), baby=rng.choice([2, 4]), giant=rng.choice([2, 4]))
+    return case
+
+
+# ---------------------------------------------------------------- sizes
+
+def _batch_limbs(case):
+    r = random.Random(case["mix"])
+    return [r.randint(case["lo"], case["hi"]) for _ in range(case["count"])]
+
+
+def _served_requests(case):
+    """(kind, limbs, rotation steps) per request of the served burst."""
+    r = random.Random(case["mix"])
+    out = []
+    for i in range(case["count"]):
+        kind = SERVED[i % len(SERVED)]
+        limbs = r.randint(max(case["lo"], 2), max(case["hi"], 2))
+        out.append((kind, limbs, sorted(r.sample(range(1, 33), 16)) if kind == "hoisted" else []))
+    return out
+
+
+def _mask(case):
+    """Which of the baby * giant diagonals are present: per_block of every giant block, spread over the baby steps."""
+    baby, giant, per = case["baby"], case["giant"], min(case["per_block"], case["baby"])
+    present = [False] * (baby * giant)
+    for k1 in range(giant):
+        for j in range(per):
+            present[k1 * baby + (k1 + j * baby // per) % baby] = True
+    return present
+
+
+def _product_steps(present, baby, giant, stride, slots):
+    """The rotation steps of a baby-step giant-step product (offset 0), each once."""
+    steps = {k2 * stride for k2 in range(baby) if any(present[k1 * baby + k2] for k1 in range(giant))}
+    steps |= {baby * k1 * stride for k1 in range(giant) if any(present[k1 * baby:(k1 + 1) * baby])}
+    return sorted(s % slots for s in steps if s % slots)
+
+
+# ---------------------------------------------------------------- state
+
+_contexts = {}
+
+
+def _context(name):
+    """The program's context of a parameter set (tables and launch plans), opened once."""
+    if name not in _contexts:
+        log_n, q_bits, p_bits, dnum = SETS[name]
+        q, p = ckh.params_primes(log_n, q_bits, p_bits)
+        _contexts[name] = ckh.Context(log_n, q, p, dnum)
+    return _contexts[name]
+
+
+def _ct(ctx, limbs, seed, comps=2):
+    return ctx.ct_from_polys([ctx.uniform(limbs - 1, seed=seed, stream0=100 * c) for c in range(comps)], SCALE)
+
+
+def _keys(ctx, steps, seed):
+    top = len(ctx.q) - 1
+    return [ctx.ksk_uniform(top, seed=seed + 7 * s, galois=ckh.galois_elt(ctx.log_n, s)) for s in steps]
+
+
+def prepare(case, seed):
+    ctx = _context(case["set"])
+    top, slots = len(ctx.q) - 1, ctx.n // 2
+    base = 1000003 * (seed + 1)
+    op, s = case["op"], {"case": case, "ctx": ctx}
+    if op == "round_trip":
+        s["poly"] = ctx.uniform(case["limbs"] - 1, seed=base, ntt=False)
+    elif op in ("switch", "switch_batch"):
+        limbs = [case["limbs"]] if op == "switch" else _batch_limbs(case)
+        s["key"] = ctx.ksk_uniform(top, seed=base)
+        s["polys"] = [ctx.uniform(n - 1, seed=base + 11 + i) for i, n in enumerate(limbs)]
+    elif op == "relin_batch":
+        s["ev"] = ckh.Evaluator(ctx, ctx.ksk_uniform(top, seed=base))
+        s["cts"] = [_ct(ctx, n, base + 11 + i, 3) for i, n in enumerate(_batch_limbs(case))]
+    elif op == "product":
+        s["ev"] = ckh.Evaluator(ctx, ctx.ksk_uniform(top, seed=base))
+        s["a"], s["b"] = (_ct(ctx, case["limbs"], base + i) for i in (11, 12))
+    elif op == "rotate":
+        s["ev"] = ckh.Evaluator(ctx, None, _keys(ctx, [5], base))
+        s["a"] = _ct(ctx, case["limbs"], base + 11)
+    elif op == "hoisted":
+        s["steps"] = list(range(1, case["count"] + 1))
+        s["ev"] = ckh.Evaluator(ctx, None, _keys(ctx, s["steps"], base))
+        s["a"] = _ct(ctx, case["limbs"], base + 11)
+    elif op in ("matvec", "matvec_enc"):
+        present = _mask(case)
+        keys = _keys(ctx, _product_steps(present, case["baby"], case["giant"], 1, slots), base)
+        relin = ctx.ksk_uniform(top, seed=base + 3) if op == "matvec_enc" else None
+        s["ev"] = ckh.Evaluator(ctx, relin, keys)
+        s["a"] = _ct(ctx, case["limbs"], base + 11)
+        s["entries"] = [None if not p else
+                        ctx.uniform(case["limbs"] - 1, seed=base + 5000 + i) if op == "matvec" else
+                        _ct(ctx, case["limbs"], base + 5000 + i) for i, p in enumerate(present)]
+    elif op == "coeff_to_slot":
+        _prepare_stages(s, case, ctx, base)
+    else:
+        relin = ctx.ksk_uniform(top, seed=base)
+        s["ev"] = ckh.Evaluator(ctx, relin, _keys(ctx, range(1, 33), base))
+        s["server"] = ckh.Server(hbm_budget_bytes=100 * 10 ** 9)
+        kinds = {"relinearize": ckh.OP_RELINEARIZE, "hoisted": ckh.OP_HOISTED_ROTATE, "product": ckh.OP_MUL_RELIN_RESCALE}
+        s["requests"] = []
+        for i, (kind, limbs, steps) in enumerate(_served_requests(case)):
+            a = _ct(ctx, limbs, base + 2 * i + 11, 3 if kind == "relinearize" else 2)
+            b = _ct(ctx, limbs, base + 2 * i + 12) if kind == "product" else None
+            s["requests"].append((kinds[kind], a, b, steps))
+    ctx.synchronize()
+    return s
+
+
+def _stage_shapes(case):
+    d = case["baby"] * case["giant"]
+    return [(case["baby"], case["giant"], 1, 0), (case["baby"], case["giant"], d, 0)]
+
+
+def _prepare_stages(s, case, ctx, base):
+    """Two CoeffToSlot stages with every diagonal present, the last also taking the conjugate."""
+    slots, d = ctx.n // 2, case["baby"] * case["giant"]
+    shapes = _stage_shapes(case)
+    steps = sorted({x for b, g, st, _ in shapes for x in _product_steps([True] * d, b, g, st, slots)})
+    keys = _keys(ctx, steps, base)
+    keys.append(ctx.ksk_uniform(len(ctx.q) - 1, seed=base + 3, galois=ckh.conjugation_elt(ctx.log_n)))
+    ev = s["ev"] = ckh.Evaluator(ctx, None, keys)
+    scale, stages = SCALE, []
+    for k, shape in enumerate(shapes):
+        level = case["limbs"] - 1 - k
+        pt_scale = ev.exact_product_scale(level, SCALE) / scale
+        diags = [ctx.uniform(level, seed=base + 5000 + 100 * k + i) for i in range(d)]
+        second = [ctx.uniform(level, seed=base + 6000 + i) for i in range(d)] if k else None
+        stages.append(ckh.LinearStage(ckh.COEFF_TO_SLOT, level, SCALE, diags, pt_scale, shape, second=second))
+        scale = SCALE
+    s["stages"] = stages
+    s["a"] = _ct(ctx, case["limbs"], base + 11)
+
+
+# ---------------------------------------------------------------- outputs
+
+class Residues(torch.Tensor):
+    """The words of device polynomials or ciphertexts as an int64 tensor. They stay on the device, as in a program
+    that goes on computing with them, and are downloaded when the tensor's values are first used."""
+
+    @staticmethod
+    def __new__(cls, handles, words):
+        return torch.Tensor._make_wrapper_subclass(cls, (words,), dtype=torch.int64, device="cpu")
+
+    def __init__(self, handles, words):
+        self.handles = handles
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        def plain(x):
+            if not isinstance(x, cls):
+                return x
+            return torch.from_numpy(np.concatenate([h.download().ravel() for h in x.handles]).view(np.int64))
+        return func(*[plain(a) for a in args], **{k: plain(v) for k, v in (kwargs or {}).items()})
+
+
+def _polys(ctx, polys, limbs):
+    return Residues(polys, limbs * ctx.n)
+
+
+def _cts(ctx, cts):
+    return Residues(cts, sum(c * (level + 1) for c, level, _ in (ct.info() for ct in cts)) * ctx.n)
+
+
+def run(s):
+    ctx, case = s["ctx"], s["case"]
+    op = case["op"]
+    if op == "round_trip":
+        f = s["poly"].ntt()
+        return [_polys(ctx, [f], case["limbs"]), _polys(ctx, [f.intt()], case["limbs"])]
+    if op == "switch":
+        return [_polys(ctx, [p], case["limbs"]) for p in ctx.key_switch(s["polys"][0], s["key"])]
+    if op == "switch_batch":
+        out = ctx.key_switch_batch(s["polys"], s["key"])
+        total = sum(_batch_limbs(case))
+        return [_polys(ctx, [pair[i] for pair in out], total) for i in range(2)]
+    ev = s["ev"]
+    if op == "relin_batch":
+        return _cts(ctx, ev.relinearize_batch(s["cts"]))
+    if op == "product":
+        return _cts(ctx, [ev.rescale(ev.relinearize(ev.mul_no_relin(s["a"], s["b"])))])
+    if op == "rotate":
+        return _cts(ctx, [ev.rotate(s["a"], 5)])
+    if op == "hoisted":
+        return _cts(ctx, ev.hoisted_rotate(s["a"], s["steps"]))
+    if op == "matvec":
+        return _cts(ctx, [ev.matvec_plain(s["a"], s["entries"], SCALE, case["baby"], case["giant"])])
+    if op == "matvec_enc":
+        return _cts(ctx, [ev.matvec_enc(s["a"], s["entries"], case["baby"], case["giant"])])
+    if op == "coeff_to_slot":
+        return _cts(ctx, list(ev.coeff_to_slot(s["a"], s["stages"])))
+    tickets = [s["server"].submit(kind, ev, a, b, steps) for kind, a, b, steps in s["requests"]]
+    done = [s["server"].poll(t) for t in tickets]
+    assert all(status == 0 for status, _, _, _ in done), done
+    return _cts(ctx, [ct for _, _, outs, _ in done for ct in outs])
+
+
+def exact(case, seed):
+    """Every output is an array of residues, whole numbers that have to be equal."""
+    return None
+
+
+# ---------------------------------------------------------------- work
+
+class _Work:
+    """Limbs read and written once, and modular products, of one call on a parameter set."""
+
+    def __init__(self, name):
+        log_n, q_bits, p_bits, dnum = SETS[name]
+        self.log_n, self.n = log_n, 1 << log_n
+        self.nq, self.k, self.alpha = len(q_bits), len(p_bits), len(q_bits) // dnum
+        self.limbs = 0
+        self.products = 0
+
+    def digits(self, limbs):
+        return -(-limbs // self.alpha)
+
+    def key(self, limbs):
+        self.limbs += 2 * self.digits(limbs) * (limbs + self.k)
+
+    def ntt(self, limbs):
+        self.products += limbs * self.n // 2 * self.log_n
+
+    def decompose(self, limbs):
+        d = self.digits(limbs)
+        targets = d * (limbs + self.k) - limbs
+        self.ntt(limbs + targets)
+        self.products += self.n * (limbs + min(limbs, self.alpha) * targets)
+
+    def apply(self, limbs):
+        self.products += self.n * (2 * self.digits(limbs) * (limbs + self.k) + 2 * self.k + 2 * limbs * (self.k + 1))
+        self.ntt(2 * (self.k + limbs))
+
+    def switch(self, limbs):
+        self.decompose(limbs)
+        self.apply(limbs)
+
+    def rescale(self, limbs, comps=2):
+        self.ntt(comps * limbs)
+        self.products += comps * 2 * (limbs - 1) * self.n
+
+    def total(self):
+        return {"bytes": 8 * self.n * self.limbs, "flops": 2 * self.products}
+
+
+def work(case):
+    w, op = _Work(case["set"]), case["op"]
+    n = case.get("limbs", 0)
+    if op == "round_trip":
+        w.limbs = 3 * n
+        w.ntt(2 * n)
+    elif op in ("switch", "switch_batch", "relin_batch"):
+        each = [n] if op == "switch" else _batch_limbs(case)
+        w.key(max(each))
+        for x in each:
+            w.limbs += 3 * x + (2 * x if op == "relin_batch" else 0)
+            w.switch(x)
+    elif op == "product":
+        w.key(n)
+        w.limbs += 4 * n + 2 * (n - 1)
+        w.switch(n)
+        w.rescale(n)
+        w.products += 4 * n * w.n
+    elif op in ("rotate", "hoisted"):
+        count = case.get("count", 1)
+        w.limbs += 2 * n + 2 * n * count
+        w.decompose(n)
+        for _ in range(count):
+            w.key(n)
+            w.apply(n)
+    elif op in ("matvec", "matvec_enc"):
+        _work_product(w, case, _mask(case), n, 1 if op == "matvec" else 2)
+        w.limbs += 4 * n
+    elif op == "coeff_to_slot":
+        d = case["baby"] * case["giant"]
+        for k, inputs in enumerate((1, 2)):
+            for i in range(inputs):
+                _work_product(w, dict(case, per_block=case["baby"]), [True] * d, n - k, 1, giants=i == 0)
+            w.rescale(n - k)
+        for x in (n - 1, n - 2):  # the conjugations
+            w.key(x)
+            w.switch(x)
+        w.limbs += 2 * n + 4 * (n - 2)
+    else:
+        requests = _served_requests(case)
+        if any(kind != "hoisted" for kind, _, _ in requests):
+            w.key(max(x for kind, x, _ in requests if kind != "hoisted"))
+        for step in {s for _, _, steps in requests for s in steps}:
+            w.key(max(x for _, x, steps in requests if step in steps))
+        for kind, x, steps in requests:
+            if kind == "hoisted":
+                w.limbs += 2 * x + 2 * x * len(steps)
+                w.decompose(x)
+                for _ in steps:
+                    w.apply(x)
+            elif kind == "relinearize":
+                w.limbs += 5 * x
+                w.switch(x)
+            else:
+                w.limbs += 4 * x + 2 * (x - 1)
+                w.switch(x)
+                w.rescale(x)
+                w.products += 4 * x * w.n
+    return w.total()
+
+
+def _work_product(w, case, present, limbs, comps, giants=True):
+    """One baby-step giant-step product: its diagonals, rotation keys and, encrypted, relinearizations."""
+    baby, giant, nnz = case["baby"], case["giant"], sum(present)
+    babies = sum(1 for k2 in range(1, baby) if any(present[k1 * baby + k2] for k1 in range(giant)))
+    blocks = sum(1 for k1 in range(giant) if any(present[k1 * baby:(k1 + 1) * baby]))
+    w.limbs += nnz * comps * limbs
+    w.products += 2 * comps * nnz * limbs * w.n
+    w.decompose(limbs)
+    for _ in range(babies):
+        w.key(limbs)
+        w.apply(limbs)
+    if comps == 2:
+        w.key(limbs)
+        for _ in range(blocks):
+            w.switch(limbs)
+    for _ in range(blocks - 1 if giants else 0):
+        w.key(limbs)
+        w.switch(limbs)
