@@ -114,6 +114,22 @@ def _served_requests(case):
     return out
 
 
+def _output_limbs(case):
+    """Limbs of each output tensor."""
+    op, n = case["op"], case.get("limbs", 0)
+    if op in ("round_trip", "switch"):
+        return n
+    if op in ("switch_batch", "relin_batch"):
+        return (2 if op == "relin_batch" else 1) * sum(_batch_limbs(case))
+    if op == "product":
+        return 2 * (n - 1)
+    if op == "coeff_to_slot":  # two stages, each a level; re and im
+        return 4 * (n - 2)
+    if op == "served":
+        return sum(2 * (x - 1 if kind == "product" else x) * max(1, len(steps)) for kind, x, steps in _served_requests(case))
+    return 2 * n * case.get("count", 1)
+
+
 def _mask(case):
     """Which of the baby * giant diagonals are present: per_block of every giant block, spread over the baby steps."""
     baby, giant, per = case["baby"], case["giant"], min(case["per_block"], case["baby"])
@@ -158,7 +174,8 @@ def prepare(case, seed):
     ctx = _context(case["set"])
     top, slots = len(ctx.q) - 1, ctx.n // 2
     base = 1000003 * (seed + 1)
-    op, s = case["op"], {"case": case, "ctx": ctx}
+    op = case["op"]
+    s = {"op": op, "ctx": ctx, "words": _output_limbs(case) * ctx.n}
     if op == "round_trip":
         s["poly"] = ctx.uniform(case["limbs"] - 1, seed=base, ntt=False)
     elif op in ("switch", "switch_batch"):
@@ -184,6 +201,7 @@ def prepare(case, seed):
         relin = ctx.ksk_uniform(top, seed=base + 3) if op == "matvec_enc" else None
         s["ev"] = ckh.Evaluator(ctx, relin, keys)
         s["a"] = _ct(ctx, case["limbs"], base + 11)
+        s["baby"], s["giant"] = case["baby"], case["giant"]
         s["entries"] = [None if not p else
                         ctx.uniform(case["limbs"] - 1, seed=base + 5000 + i) if op == "matvec" else
                         _ct(ctx, case["limbs"], base + 5000 + i) for i, p in enumerate(present)]
@@ -250,45 +268,35 @@ class Residues(torch.Tensor):
         return func(*[plain(a) for a in args], **{k: plain(v) for k, v in (kwargs or {}).items()})
 
 
-def _polys(ctx, polys, limbs):
-    return Residues(polys, limbs * ctx.n)
-
-
-def _cts(ctx, cts):
-    return Residues(cts, sum(c * (level + 1) for c, level, _ in (ct.info() for ct in cts)) * ctx.n)
-
-
 def run(s):
-    ctx, case = s["ctx"], s["case"]
-    op = case["op"]
+    op, words = s["op"], s["words"]
     if op == "round_trip":
         f = s["poly"].ntt()
-        return [_polys(ctx, [f], case["limbs"]), _polys(ctx, [f.intt()], case["limbs"])]
+        return [Residues([f], words), Residues([f.intt()], words)]
     if op == "switch":
-        return [_polys(ctx, [p], case["limbs"]) for p in ctx.key_switch(s["polys"][0], s["key"])]
+        return [Residues([p], words) for p in s["ctx"].key_switch(s["polys"][0], s["key"])]
     if op == "switch_batch":
-        out = ctx.key_switch_batch(s["polys"], s["key"])
-        total = sum(_batch_limbs(case))
-        return [_polys(ctx, [pair[i] for pair in out], total) for i in range(2)]
+        out = s["ctx"].key_switch_batch(s["polys"], s["key"])
+        return [Residues([pair[i] for pair in out], words) for i in range(2)]
     ev = s["ev"]
     if op == "relin_batch":
-        return _cts(ctx, ev.relinearize_batch(s["cts"]))
+        return Residues(ev.relinearize_batch(s["cts"]), words)
     if op == "product":
-        return _cts(ctx, [ev.rescale(ev.relinearize(ev.mul_no_relin(s["a"], s["b"])))])
+        return Residues([ev.rescale(ev.relinearize(ev.mul_no_relin(s["a"], s["b"])))], words)
     if op == "rotate":
-        return _cts(ctx, [ev.rotate(s["a"], 5)])
+        return Residues([ev.rotate(s["a"], 5)], words)
     if op == "hoisted":
-        return _cts(ctx, ev.hoisted_rotate(s["a"], s["steps"]))
+        return Residues(ev.hoisted_rotate(s["a"], s["steps"]), words)
     if op == "matvec":
-        return _cts(ctx, [ev.matvec_plain(s["a"], s["entries"], SCALE, case["baby"], case["giant"])])
+        return Residues([ev.matvec_plain(s["a"], s["entries"], SCALE, s["baby"], s["giant"])], words)
     if op == "matvec_enc":
-        return _cts(ctx, [ev.matvec_enc(s["a"], s["entries"], case["baby"], case["giant"])])
+        return Residues([ev.matvec_enc(s["a"], s["entries"], s["baby"], s["giant"])], words)
     if op == "coeff_to_slot":
-        return _cts(ctx, list(ev.coeff_to_slot(s["a"], s["stages"])))
+        return Residues(list(ev.coeff_to_slot(s["a"], s["stages"])), words)
     tickets = [s["server"].submit(kind, ev, a, b, steps) for kind, a, b, steps in s["requests"]]
     done = [s["server"].poll(t) for t in tickets]
     assert all(status == 0 for status, _, _, _ in done), done
-    return _cts(ctx, [ct for _, _, outs, _ in done for ct in outs])
+    return Residues([ct for _, _, outs, _ in done for ct in outs], words)
 
 
 def exact(case, seed):
