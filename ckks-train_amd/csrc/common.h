@@ -22,6 +22,15 @@ CKH_DEV u32 brev32(u32 x) { return __brev(x); }
 // A value the optimizer must treat as unknown (it cannot hoist what is derived from it).
 #define CKH_OPAQUE(x) asm volatile("" : "+v"(x))
 
+// Orders the LDS accesses of one wave before and after it (no instruction: a wave's LDS accesses
+// are performed in order; the fences keep the compiler from moving them across).
+#define CKH_WAVE_SYNC()                                        \
+    do {                                                       \
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); \
+        __builtin_amdgcn_wave_barrier();                       \
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront"); \
+    } while (0)
+
 #include "arith.h"
 
 namespace ckh {

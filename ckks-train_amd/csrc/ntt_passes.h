@@ -23,11 +23,17 @@
 //
 // The includer provides, besides arith.h: glb(p) (a global-memory view of a pointer),
 // load_coherent(p) (a load that sees other workgroups' completed stores), __syncthreads(),
-// threadIdx.x and CKH_OPAQUE(x) (hides a value's origin from the optimizer). The LDS tile is a
-// template parameter (a __shared__ array on the device).
+// CKH_WAVE_SYNC() (orders the LDS accesses of the 64 threads of one wave; where it is not
+// defined, the workgroup's barrier stands in), threadIdx.x and CKH_OPAQUE(x) (hides a value's
+// origin from the optimizer). The LDS tile is a template parameter (a __shared__ array on the
+// device).
 #pragma once
 
 #include "arith.h"
+
+#ifndef CKH_WAVE_SYNC
+#define CKH_WAVE_SYNC() __syncthreads()
+#endif
 
 namespace ckh {
 namespace fast {
@@ -39,6 +45,17 @@ constexpr u32 LDS_WORDS = TILE + TILE / 16;
 
 // Padded LDS index: one spare word per 16 spreads strided accesses over the banks.
 CKH_DEV u32 pad(u32 a) { return a + (a >> 4); }
+
+// Word k (of 16) of thread tid in the coalesced layout of a row pass. A row of at most 256 words
+// belongs to at most 16 adjacent threads, so a wave's 64 threads own 1024 consecutive words of the
+// tile: every LDS exchange of a row pass stays inside one wave, which needs no workgroup barrier
+// (an LDS access of a wave follows its earlier ones), and the coalesced words of a wave are those
+// same 1024. The fused row pass + inner product + finish is bound by latency at 3 waves per SIMD,
+// and waves that do not meet three times per digit overlap one another's loads: 4.64 -> 4.25 ms
+// per 256-switch step at N = 2^16 (and the registers fit without the two spilled sums), 0.746 ->
+// 0.716 ms for 31 rotations at 2^15. The finish of an unfused row pass keeps the workgroup's
+// order of words: with the wave's it was 3-7 % slower (224 against 216 us, 16 rotations).
+CKH_DEV u32 wave_word(u32 tid, u32 k) { return ((tid & ~63u) << 4) + (tid & 63u) + (k << 6); }
 
 // ---------------------------------------------------------------- f64 arithmetic (q < 2^50)
 
@@ -331,7 +348,8 @@ CKH_DEV void fwd_cols(const Ar& ar, const u64* __restrict__ in_p, u64* __restric
 struct NoPre {
     CKH_DEV void operator()() const {}
 };
-template <u32 M, bool F64, class Ar, bool COH = false, class Lds, bool RAW = false, class Pre = NoPre>
+// BLOCK: the closing barrier is the workgroup's, for a caller that reads the tile across its waves.
+template <u32 M, bool F64, class Ar, bool COH = false, class Lds, bool RAW = false, bool BLOCK = false, class Pre = NoPre>
 CKH_DEV void fwd_rows_to_lds(const Ar& ar, const u64* __restrict__ in_p, Lds lds, u32 log_n, u32 tile,
                              u32 tid = threadIdx.x, Pre pre = Pre{}) {
     const auto in = glb(in_p);
@@ -348,7 +366,7 @@ CKH_DEV void fwd_rows_to_lds(const Ar& ar, const u64* __restrict__ in_p, Lds lds
     rows_round1_fwd<Ar>(ar, v, A, row);
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) lds[pad((rr << M) + o + (k << R2))] = ar.to_mid(v[k]);
-    __syncthreads();
+    CKH_WAVE_SYNC();
 #pragma unroll
     for (u32 e = 0; e < 16; ++e) {
         const u32 c = ((((o << U) | (e >> R2)) << R2) | (e & JM));
@@ -357,14 +375,17 @@ CKH_DEV void fwd_rows_to_lds(const Ar& ar, const u64* __restrict__ in_p, Lds lds
     // Round 2: the thread's column c = 16 o + e, so stage A + s uses tab[2^(A+s) + row 2^s +
     // o 2^D + m] with D = s + 4 - M and m = e >> (M - s) < 2^D.
     rows_round2_fwd<M, Ar>(ar, v, A, row, o);
-    __syncthreads();
+    CKH_WAVE_SYNC();
 #pragma unroll
     for (u32 e = 0; e < 16; ++e) {
         const u32 c = ((((o << U) | (e >> R2)) << R2) | (e & JM));
         lds[pad((rr << M) + c)] = RAW ? ar.to_mid(v[e]) : F64 ? ar.fwd_final_f(v[e]) : ar.fwd_final(v[e]);
     }
     pre();
-    __syncthreads();
+    if constexpr (BLOCK)
+        __syncthreads();
+    else
+        CKH_WAVE_SYNC();
 }
 
 template <u32 M, class Ar, bool COH = false, class Lds>
@@ -390,7 +411,7 @@ CKH_DEV void fwd_rows(const Ar& ar, const u64* __restrict__ in, u64* __restrict_
         if constexpr (Ar::F64) {
             // in f64: the transform left unreduced (|.| <= 2.6 q), a - t below 3.6 q, one modular
             // product (|.| <= 1.2 q), the addend, one reduction
-            fwd_rows_to_lds<M, false, Ar, COH, Lds, true>(ar, in, lds, log_n, tile, tid, pre);
+            fwd_rows_to_lds<M, false, Ar, COH, Lds, true, true>(ar, in, lds, log_n, tile, tid, pre);
             const FTw iv = fin->inv_f;
 #pragma unroll
             for (u32 k = 0; k < 16; ++k) {
@@ -399,7 +420,7 @@ CKH_DEV void fwd_rows(const Ar& ar, const u64* __restrict__ in, u64* __restrict_
                 fout[tbase + tid + k * NT] = d2u(fcanon(v, ar.q, ar.qinv));
             }
         } else {
-            fwd_rows_to_lds<M, false, Ar, COH, Lds, false>(ar, in, lds, log_n, tile, tid, pre);
+            fwd_rows_to_lds<M, false, Ar, COH, Lds, false, true>(ar, in, lds, log_n, tile, tid, pre);
 #pragma unroll
             for (u32 k = 0; k < 16; ++k) {
                 u64 v = shoup(sub_mod(av[k], lds[pad(tid + k * NT)], q), inv, inv_s, q);
@@ -412,7 +433,7 @@ CKH_DEV void fwd_rows(const Ar& ar, const u64* __restrict__ in, u64* __restrict_
     fwd_rows_to_lds<M, false, Ar, COH>(ar, in, lds, log_n, tile, tid);
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) {
-        const u32 idx = tid + k * NT;
+        const u32 idx = wave_word(tid, k);
         out[tbase + idx] = lds[pad(idx)];
     }
 }
@@ -428,10 +449,10 @@ CKH_DEV void inv_rows(const Ar& ar, const u64* __restrict__ in_p, u64* __restric
     const u64 tbase = (u64)tile << TL;
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) {
-        const u32 idx = tid + k * NT;
+        const u32 idx = wave_word(tid, k);
         lds[pad(idx)] = in[tbase + idx];
     }
-    __syncthreads();
+    CKH_WAVE_SYNC();
     typename Ar::V v[16];
 #pragma unroll
     for (u32 e = 0; e < 16; ++e) {
@@ -441,13 +462,13 @@ CKH_DEV void inv_rows(const Ar& ar, const u64* __restrict__ in_p, u64* __restric
     // Round 1: c = 16 o + e; stage u uses tab[2^(logN-1-u) + row 2^(M-1-u) + o 2^(3-u) + m],
     // m = e >> (u + 1).
     rows_round1_inv<M, Ar>(ar, v, log_n - M, row, o);
-    __syncthreads();
+    CKH_WAVE_SYNC();
 #pragma unroll
     for (u32 e = 0; e < 16; ++e) {
         const u32 c = ((((o << U) | (e >> R2)) << R2) | (e & JM));
         lds[pad((rr << M) + c)] = ar.to_mid(v[e]);
     }
-    __syncthreads();
+    CKH_WAVE_SYNC();
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) v[k] = ar.from_mid(lds[pad((rr << M) + o + (k << R2))]);
     // Round 2: c = o + (k << R2) with o < 2^R2, so c >> (u + 1) = k >> (u + 1 - R2): stage u
@@ -534,8 +555,8 @@ CKH_DEV void rows_ip_sums(const FpAr& ar, const RowIpJob& J, Lds lds, u32 log_n,
         if (j == J.own_j) {
 #pragma unroll
             for (u32 k = 0; k < 16; ++k) {
-                const double x = u2d(glb(J.own)[tbase + tid + k * NT]);
-                const double b = u2d(kb[tid + k * NT]), a = u2d(ka[tid + k * NT]);
+                const double x = u2d(glb(J.own)[tbase + wave_word(tid, k)]);
+                const double b = u2d(kb[wave_word(tid, k)]), a = u2d(ka[wave_word(tid, k)]);
                 sb[k] += fmulmod(x, b, b * qinv, q);
                 sa[k] += fmulmod(x, a, a * qinv, q);
             }
@@ -546,19 +567,19 @@ CKH_DEV void rows_ip_sums(const FpAr& ar, const RowIpJob& J, Lds lds, u32 log_n,
             auto pre = [&] {
 #pragma unroll
                 for (u32 k = 0; k < 16; ++k) {
-                    kbw[k] = kb[tid + k * NT];
-                    kaw[k] = ka[tid + k * NT];
+                    kbw[k] = kb[wave_word(tid, k)];
+                    kaw[k] = ka[wave_word(tid, k)];
                 }
             };
             fwd_rows_to_lds<M, true, FpAr, false, Lds, true>(ar, J.mid + j * J.mid_stride, lds, log_n, tile, tid, pre);
 #pragma unroll
             for (u32 k = 0; k < 16; ++k) {
-                const double x = bits_f64(lds[pad(tid + k * NT)]);
+                const double x = bits_f64(lds[pad(wave_word(tid, k))]);
                 const double b = u2d(kbw[k]), a = u2d(kaw[k]);
                 sb[k] += fmulmod(x, b, b * qinv, q);
                 sa[k] += fmulmod(x, a, a * qinv, q);
             }
-            __syncthreads();  // the next digit's pass reuses the LDS
+            CKH_WAVE_SYNC();  // the next digit's pass reuses the LDS
         }
         if ((j & 3) == 3) {
 #pragma unroll
@@ -579,8 +600,8 @@ CKH_DEV void rows_ip(const FpAr& ar, const RowIpJob& J, Lds lds, u32 log_n, u32 
     const u32 tid = threadIdx.x;
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) {
-        glb(J.acc_b)[tbase + tid + k * NT] = d2u(fcanon(sb[k], ar.q, ar.qinv));
-        glb(J.acc_a)[tbase + tid + k * NT] = d2u(fcanon(sa[k], ar.q, ar.qinv));
+        glb(J.acc_b)[tbase + wave_word(tid, k)] = d2u(fcanon(sb[k], ar.q, ar.qinv));
+        glb(J.acc_a)[tbase + wave_word(tid, k)] = d2u(fcanon(sa[k], ar.q, ar.qinv));
     }
 }
 
@@ -602,19 +623,19 @@ CKH_DEV void finish_sum(const FpAr& ar, const double (&s)[16], const u64* z, u64
     auto pre = [&] {
         if (add_p) {
 #pragma unroll
-            for (u32 k = 0; k < 16; ++k) dv[k] = glb(add_p)[tbase + tid + k * NT];
+            for (u32 k = 0; k < 16; ++k) dv[k] = glb(add_p)[tbase + wave_word(tid, k)];
         }
     };
     fwd_rows_to_lds<M, false, FpAr, false, Lds, true>(ar, z, lds, log_n, tile, tid, pre);
     const auto out = glb(out_p);
 #pragma unroll
     for (u32 k = 0; k < 16; ++k) {
-        const double d = freduce(s[k], q, qinv) - bits_f64(lds[pad(tid + k * NT)]);
+        const double d = freduce(s[k], q, qinv) - bits_f64(lds[pad(wave_word(tid, k))]);
         double v = fmulmod(d, inv.w, inv.wq, q);
         if (add_p) v = v + u2d(dv[k]);
-        out[tbase + tid + k * NT] = d2u(fcanon(v, q, qinv));
+        out[tbase + wave_word(tid, k)] = d2u(fcanon(v, q, qinv));
     }
-    __syncthreads();  // the next pass reuses the LDS
+    CKH_WAVE_SYNC();  // the next pass reuses the LDS
 }
 
 }  // namespace fast
