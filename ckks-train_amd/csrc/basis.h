@@ -27,10 +27,8 @@ struct ConvTables {
 // For each job: coefficient-form input limbs (reduced) -> converted output limbs (reduced,
 // coefficient form): out_t = [x_c]_r with x_c the centered value of the source residues
 // (BaseConverter::convert_exact of [x + h]_Q minus h mod r).
-// Tuning choices: variant: 0 = vector kernel; 1 = vector kernel with 50-bit targets of 60-bit
-// sources summed as exact f64 pieces (20-bit source pieces times 25-bit constant halves) instead
-// of two modular products per source; 2 = the matrix-core kernel (when ConvTables::mf_ok; else
-// variant 0); tg:
+// Tuning choices: variant: 0 or 1 = vector kernel; 2 = the matrix-core kernel (when
+// ConvTables::mf_ok; else the vector kernel); tg:
 // targets per workgroup of the vector kernels (the sources are read once per group of tg);
 // yform: every job's input limbs are in y form (YForm), for kernels compiled for that input.
 void conv_launch(const ConvTables& t, const ConvJob* jobs, u32 njobs, u32 max_tgt, u32 max_src, u32 variant,

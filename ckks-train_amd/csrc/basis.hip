@@ -10,7 +10,7 @@ namespace ckh {
 
 // One block: 256 coefficients of one job, targets [t0, t0 + tg) of its plan. YF: inputs in y form
 // (a separate instantiation: the per-source product it skips would otherwise hold registers).
-template <u32 MAXS, bool PIECES, bool YF>
+template <u32 MAXS, bool YF>
 __global__ __launch_bounds__(256) void k_conv(ConvTables T, const ConvJob* __restrict__ jobs, u32 tg) {
     const u32 n = 1u << T.log_n;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
@@ -18,7 +18,7 @@ __global__ __launch_bounds__(256) void k_conv(ConvTables T, const ConvJob* __res
     const ConvPlan P = T.plans[job.plan];
     const u32 t0 = blockIdx.z * tg;
     if (t0 >= P.ntgt || c >= n) return;
-    conv_coeff<MAXS, PIECES>(T.src, T.tgt, T.pc, P, job.in, job.out, n, c, t0, min(t0 + tg, P.ntgt), YF);
+    conv_coeff<MAXS>(T.src, T.tgt, T.pc, P, job.in, job.out, n, c, t0, min(t0 + tg, P.ntgt), YF);
 }
 
 // ---------------------------------------------------------------- matrix-core conversion
@@ -44,14 +44,11 @@ __global__ __launch_bounds__(256) void k_conv_mf(ConvTables T, const ConvJob* __
 }
 
 template <u32 MAXS, bool YF>
-static void conv_launch_s(const ConvTables& t, const ConvJob* jobs, u32 njobs, u32 max_tgt, u32 variant, u32 tg,
+static void conv_launch_s(const ConvTables& t, const ConvJob* jobs, u32 njobs, u32 max_tgt, u32 tg,
                           hipStream_t stream) {
     const u32 n = 1u << t.log_n;
     const u32 zt = (max_tgt + tg - 1) / tg;
-    if (variant == 1)
-        hipLaunchKernelGGL((k_conv<MAXS, true, YF>), dim3((n + 255) / 256, njobs, zt), dim3(256), 0, stream, t, jobs, tg);
-    else
-        hipLaunchKernelGGL((k_conv<MAXS, false, YF>), dim3((n + 255) / 256, njobs, zt), dim3(256), 0, stream, t, jobs, tg);
+    hipLaunchKernelGGL((k_conv<MAXS, YF>), dim3((n + 255) / 256, njobs, zt), dim3(256), 0, stream, t, jobs, tg);
 }
 
 template <bool YF>
@@ -67,15 +64,15 @@ static void conv_launch_t(const ConvTables& t, const ConvJob* jobs, u32 njobs, u
     }
     switch (max_src) {
         case 0:
-        case 1: conv_launch_s<1, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 2: conv_launch_s<2, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 3: conv_launch_s<3, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 4: conv_launch_s<4, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 5: conv_launch_s<5, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 6: conv_launch_s<6, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 7: conv_launch_s<7, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        case 8: conv_launch_s<8, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
-        default: conv_launch_s<16, YF>(t, jobs, njobs, max_tgt, variant, tg, stream); break;
+        case 1: conv_launch_s<1, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 2: conv_launch_s<2, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 3: conv_launch_s<3, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 4: conv_launch_s<4, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 5: conv_launch_s<5, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 6: conv_launch_s<6, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 7: conv_launch_s<7, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        case 8: conv_launch_s<8, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
+        default: conv_launch_s<16, YF>(t, jobs, njobs, max_tgt, tg, stream); break;
     }
 }
 

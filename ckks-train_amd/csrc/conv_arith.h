@@ -14,6 +14,13 @@
 // non-modular step: it uses the CPU's exact sequence (round-to-nearest u64->f64 conversion,
 // round-to-nearest product with the host-computed reciprocal, round-to-nearest sum in source
 // order from +0.0, then floor), so every includer compiles it without FMA contraction.
+//
+// Conversions of at most 8 sources (WRAP_SMALL / WRAP_LARGE below) take one quotient for the whole
+// sum T = sum_j y_j c_j + e (-Q) - (Q-1)/2: an f64 sum F of y_j (c_j / r) estimates T / r, and
+// T - k r (k = rint(F)) is formed exactly modulo 2^64 from 32-bit halves, where its small size
+// makes it exact. Per source and target that is three 32 x 32 multiply-adds and one f64 FMA,
+// instead of a modular product each (7 operations), six piece products, or the nine operations of
+// an exact 128-bit sum with its carries.
 #pragma once
 
 #include "arith.h"
@@ -21,6 +28,7 @@
 namespace ckh {
 
 constexpr u32 MAX_SRC = 16;
+constexpr u32 WRAP_SRC = 8;  // sources of the single-quotient form
 
 // One source prime q_j of a conversion from Q = prod q_j.
 struct ConvSrc {
@@ -43,20 +51,34 @@ struct ConvTgt {
     u64 qhat[MAX_SRC];                   // (Q / q_j) mod r
     double qhat_f[MAX_SRC], qhat_q[MAX_SRC];      // f64 path: (Q / q_j) mod r and its quotient by r
     double qhat30_f[MAX_SRC], qhat30_q[MAX_SRC];  // split path: 2^30 (Q / q_j) mod r, quotient by r
-    double half[2][MAX_SRC];  // piece path: (Q / q_j) mod r in 25-bit halves (low, high)
-    FTw p20, p40, p65;        // piece path: 2^20, 2^40, 2^65 mod r (and their quotients by r)
     double qmod_f, qmod_q, hmod_f, rf, rinv;
-    // The correction terms as addends: nq = -Q mod r (e nq = -e Q mod r), nh = -(Q - 1)/2 mod r;
-    // nq_c = nq centered in (-r/2, r/2]; nq_half / nh_half their 25-bit halves (r < 2^50).
-    u64 nq, nh;
-    double nq_c, nq_half[2], nh_half[2];
-    // TGT_INT: r at least 2^50, 128-bit integer sums; TGT_FP: r and every source below 2^50, f64
-    // products of the sources; TGT_SPLIT: r below 2^50 with larger sources, each source split
-    // into 30-bit halves (or, variant 1, 20-bit pieces summed exactly).
-    u32 mode, pad;
+    // nq = -Q mod r (e nq = -e Q mod r), nq_c the same centered in (-r/2, r/2].
+    u64 nq;
+    double nq_c;
+    // Without the single-quotient form: TGT_INT: r at least 2^50, 128-bit integer sums; TGT_FP: r
+    // and every source below 2^50, f64 products of the sources; TGT_SPLIT: r below 2^50 with
+    // larger sources, each source split into 30-bit halves.
+    u32 mode, wrap;
+    // The single-quotient form (wrap): c_j centered in (-r/2, r/2] as a two's complement word and
+    // its quotient by r (WRAP_LARGE: by 2^11 r); -Q mod r likewise; the negated divisor -r
+    // (WRAP_LARGE: -2^11 r) and r itself; the sum's constant and its quotient.
+    u64 cw[WRAP_SRC];
+    double cq[WRAP_SRC];
+    u64 nqw, nr, r, aw;
+    double nqq, aq;
 };
 
 enum : u32 { TGT_INT = 0, TGT_FP = 1, TGT_SPLIT = 2 };
+// WRAP_SMALL: every source below 2^50, any r. The sums run over y_j - 2^49 (the constant takes
+// 2^49 sum_j c_j): the partial sums of F stay below 2^51, their roundings, those of the c_j / r and
+// of the e term add up to less than 0.9 for 6 sources and 1.2 for 8, so with rint |T - k r| < 2 r.
+// WRAP_LARGE: r below 2^50, sources below 2^60: F, in units of 2^11, is off by at most 1.7 with
+// its rounding (8 sources: 2,400 from the sums and their factors, 1,024 from rint, of 4,096), so
+// |T - 2^11 k r| < 2^12 r < 2^62; a second quotient of that remainder by r gives the residue.
+enum : u32 { WRAP_NONE = 0, WRAP_SMALL = 1, WRAP_LARGE = 2 };
+constexpr u64 WRAP_CENTER = 1ull << 49;
+constexpr double WRAP_ROUND = 6755399441055744.0;        // 1.5 2^52: adding it rounds to an integer
+constexpr u64 WRAP_ROUND_BITS = 0x4338000000000000ull;  // its bits
 
 // A conversion: sources [src_first, src_first + nsrc) of the ConvSrc table (their input limbs
 // are src_limb0 + j of the job's input), targets [tgt_first, tgt_first + ntgt) of the ConvTgt
@@ -79,171 +101,181 @@ CKH_DEV double u64_to_f64_rn(u64 v) {
     return hi + lo;
 }
 
-// Coefficient c of one conversion (plan P, input polynomial in_p, output out_p, N = n): the
-// output words of targets [t0, t1). MAXS bounds the plan's sources; PIECES selects the exact
-// f64 piece sums for 50-bit targets of 60-bit sources. Per-target constants are read through
-// cst (the scalar cache on the device); 60-bit targets sum exact 128-bit integer products and
-// reduce once.
-// yform: the input limbs already hold y_j = [x_j + h_j]_{q_j} (Q/q_j)^-1 mod q_j (YForm: an
-// inverse NTT computed it in its last stage).
-template <u32 MAXS, bool PIECES>
-CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeConst* pcs, const ConvPlan& P,
-                        const u64* in_p, u64* out_p, u32 n, u32 c, u32 t0, u32 t1, bool yform) {
-    const auto inp = glb(in_p);
+// The sources of one coefficient: y_j as integers and as f64, and the overflow estimate e.
+template <u32 MAXS>
+struct ConvY {
     u64 y[MAXS];
-    // f64 source: yd = y, yh = 0; integer source: yd / yh = its low / high 30 bits, or (PIECES)
-    // yd / yh / yx = its 20-bit pieces from the low end
-    double yd[MAXS], yh[MAXS], yx[MAXS];
+    double yd[MAXS];
+    u64 e;
+    bool small;  // every source below 2^50
+};
+
+// Reads the sources of coefficient c (absent ones are 0). yform: the input limbs already hold
+// y_j = [x_j + h_j]_{q_j} (Q/q_j)^-1 mod q_j (YForm: an inverse NTT computed it in its last stage).
+template <u32 MAXS, class In>
+CKH_DEV void conv_sources(const ConvSrc* srcs, const ConvPlan& P, In inp, u32 n, u32 c, bool yform, ConvY<MAXS>& Y) {
     double f = 0.0;
-    // the piece path needs every source integer (at most 7: the bracketed sums below 2^53)
-    bool srcs_int = PIECES && MAXS <= 7;
-    for (u32 j = 0; j < P.nsrc && srcs_int; ++j) srcs_int = !cst(srcs + P.src_first + j)->fp;
+    Y.small = true;
+    // every word loaded before any is used: the loads of a coefficient are in flight together
+    u64 xs[MAXS];
+#pragma unroll
+    for (u32 j = 0; j < MAXS; ++j) xs[j] = j < P.nsrc ? (u64)inp[(u64)(P.src_limb0 + j) * n + c] : (u64)0;
 #pragma unroll
     for (u32 j = 0; j < MAXS; ++j) {
-        y[j] = 0;
-        yd[j] = 0.0;
-        yh[j] = 0.0;
-        yx[j] = 0.0;
+        Y.y[j] = 0;
+        Y.yd[j] = 0.0;
         if (j < P.nsrc) {
-            const ConvSrc* s = srcs + P.src_first + j;
-            const u64 x = inp[(u64)(P.src_limb0 + j) * n + c];
+            const auto* s = cst(srcs + P.src_first + j);
+            const u64 x = xs[j];
             if (s->fp) {
                 if (yform) {
-                    yd[j] = u2d(x);
-                    y[j] = x;
+                    Y.y[j] = x;
+                    Y.yd[j] = u2d(x);
                 } else {
                     double sv = u2d(x) + (double)s->h;
                     sv = sv >= s->qf ? sv - s->qf : sv;
                     double v = fmulmod(sv, s->qhinv_f, s->qhinv_q, s->qf);
                     v = v < 0.0 ? v + s->qf : v;
-                    yd[j] = v;
-                    y[j] = d2u(v);
+                    Y.yd[j] = v;
+                    Y.y[j] = d2u(v);
                 }
             } else {
-                y[j] = yform ? x : shoup(add_mod(x, s->h, s->q), s->qhinv, s->qhinv_s, s->q);
-                if (srcs_int) {
-                    yd[j] = (double)(u32)(y[j] & ((1u << 20) - 1));
-                    yh[j] = (double)(u32)((y[j] >> 20) & ((1u << 20) - 1));
-                    yx[j] = (double)(u32)(y[j] >> 40);
-                } else {
-                    yd[j] = (double)(u32)(y[j] & ((1u << 30) - 1));  // low 30 bits, exact
-                    yh[j] = (double)(u32)(y[j] >> 30);                // high 30 bits, exact
-                }
+                Y.y[j] = yform ? x : shoup(add_mod(x, s->h, s->q), s->qhinv, s->qhinv_s, s->q);
+                Y.yd[j] = u64_to_f64_rn(Y.y[j]);
+                Y.small = false;
             }
             if (P.exact) {
-                // f64(y_j): yd already is (y_j < 2^50 converts exactly) for an f64 source
-                const double prod = (s->fp ? yd[j] : u64_to_f64_rn(y[j])) * s->inv;
+                const double prod = Y.yd[j] * s->inv;  // f64(y_j) to nearest, exact below 2^50
                 f = f + prod;
             }
         }
     }
-    const u64 e = P.exact ? (u64)f : 0;  // f >= 0: truncation is floor
-    // With at most 8 sources, e < 8: -e (Q mod r) and -(Q - 1)/2 enter the sums as addends (e nq_c
-    // and the half products are exact) instead of a modular product and two subtractions; every
-    // f64 sum stays an integer below 2^53, which fcanon reduces exactly.
-    const double ed = (double)e;
+    Y.e = P.exact ? (u64)f : 0;  // f >= 0: truncation is floor
+}
+
+// l + (a b mod 2^64) from 32-bit halves: the low product joins l, the crossed ones m (read modulo
+// 2^32: the word is l + m 2^32).
+CKH_DEV void mad_wrap(u64& l, u64& m, u64 a, u64 b) {
+    l += (u64)(u32)a * (u32)b;
+    m += (u64)(u32)a * (u32)(b >> 32);
+    m += (u64)(u32)(a >> 32) * (u32)b;
+}
+CKH_DEV u64 wrap_word(u64 l, u64 m) {
+    CKH_OPAQUE(m);  // else only its low half is summed, as a multiply and an addition per product
+    return l + ((u64)(u32)m << 32);
+}
+
+// x, or x - m when that is not negative (x below 2^63).
+CKH_DEV u64 csub_sign(u64 x, u64 m) {
+    const u64 d = x - m;
+    return (int64_t)d < 0 ? x : d;
+}
+
+// The residue of one target g from the sources of a WRAP_SMALL conversion, y_j given minus 2^49.
+template <u32 MAXS, class Tgt>
+CKH_DEV u64 conv_wrap_small(const Tgt& g, const u64 (&y)[MAXS], const double (&yd)[MAXS], u32 e, double ed) {
+    u64 l = g->aw + (g->r << 1), m = 0;
+    double F = __builtin_fma(ed, g->nqq, g->aq);
+    l += (u64)e * (u32)g->nqw;
+    m += (u64)e * (u32)(g->nqw >> 32);
+#pragma unroll
+    for (u32 j = 0; j < MAXS; ++j) {
+        mad_wrap(l, m, y[j], g->cw[j]);
+        F = __builtin_fma(yd[j], g->cq[j], F);
+    }
+    // rint(F) as the low bits of F + 1.5 2^52 (the constant's own bits are in aw)
+    mad_wrap(l, m, f64_bits(F + WRAP_ROUND), g->nr);
+    // T - k r + 2 r, below 4 r
+    return csub_sign(csub_sign(wrap_word(l, m), g->r << 1), g->r);
+}
+
+// The residue of one target from the sources of a WRAP_LARGE conversion.
+template <u32 MAXS, class Tgt>
+CKH_DEV u64 conv_wrap_large(const Tgt& g, const u64 (&y)[MAXS], const double (&yd)[MAXS], u32 e) {
+    const u64 r = g->r;
+    u64 l = g->aw + (r << 12), m = 0;
+    double F = 0.0;
+    l += (u64)e * (u32)g->nqw;
+    m += (u64)e * (u32)(g->nqw >> 32);
+#pragma unroll
+    for (u32 j = 0; j < MAXS; ++j) {
+        mad_wrap(l, m, y[j], g->cw[j]);
+        F = __builtin_fma(yd[j], g->cq[j], F);
+    }
+    mad_wrap(l, m, f64_bits(F + WRAP_ROUND), g->nr);
+    // U = T - 2^11 k r + 2^12 r in (0, 2^13 r): its quotient by r, rounded down from an estimate
+    // 2^-20 low (so never too large, and too small by one at most for the last 2^-20 of r)
+    const u64 U = wrap_word(l, m);
+    const double ud = __builtin_fma((double)(u32)(U >> 32), 4294967296.0, (double)(u32)U);
+    const double kd = __builtin_fma(ud, g->rinv, -0x1p-20);
+    const u32 k = (u32)kd;  // a negative estimate (U < 2^-20 r) converts to 0
+    return csub_sign(U - (u64)k * r, r);
+}
+
+// Coefficient c of one conversion (plan P, input polynomial in_p, output out_p, N = n): the
+// output words of targets [t0, t1). MAXS bounds the plan's sources. Per-target constants are read
+// through cst (the scalar cache on the device). Bound by VALU before the single-quotient form, now
+// by memory and latency: ModUp conversions of 256 switches at N = 2^16 (50-bit sources) 2.92 ->
+// 1.64 ms, mod_down's (60-bit sources) 2.12 -> 0.98 ms per step.
+template <u32 MAXS, bool = false>
+CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeConst* pcs, const ConvPlan& P,
+                        const u64* in_p, u64* out_p, u32 n, u32 c, u32 t0, u32 t1, bool yform) {
+    ConvY<MAXS> Y;
+    conv_sources<MAXS>(srcs, P, glb(in_p), n, c, yform, Y);
     const auto outp = glb(out_p);
+    const double ed = (double)(u32)Y.e;
+    if constexpr (MAXS <= WRAP_SRC) {
+        if (Y.small) {
+            // y_j - 2^49, an absent source's as well (its constants are 0)
+#pragma unroll
+            for (u32 j = 0; j < MAXS; ++j) {
+                Y.y[j] -= WRAP_CENTER;
+                Y.yd[j] -= (double)WRAP_CENTER;
+            }
+            for (u32 t = t0; t < t1; ++t) {
+                const auto* g = cst(tgts + P.tgt_first + t);
+                st_nt(outp, (u64)g->limb * n + c, conv_wrap_small<MAXS>(g, Y.y, Y.yd, (u32)Y.e, ed));
+            }
+            return;
+        }
+    }
     for (u32 t = t0; t < t1; ++t) {
         const auto* g = cst(tgts + P.tgt_first + t);
         u64 o;
-        if (PIECES && g->mode == TGT_SPLIT && srcs_int) {
-            // y_j = y0 + y1 2^20 + y2 2^40 (20-bit pieces), c_j = c0 + c1 2^25 (25-bit halves):
-            // S_ab = sum_j y_ja c_jb is exact (every product < 2^45, at most 7 terms), and
-            // sum_j y_j c_j = S00 + (32 S01 + S10) 2^20 + (32 S11 + S20) 2^40 + S21 2^65, the two
-            // bracketed sums staying below 2^53.
-            // -(Q - 1)/2 starts the two low sums and e (-Q mod r) is one more term of them (e < 7:
-            // both stay below 7 2^45 + 2^28, the bracketed sums below 2^53)
-            const double r = g->rf, rinv = g->rinv;
-            double s00 = g->nh_half[0], s01 = g->nh_half[1], s10 = 0.0, s11 = 0.0, s20 = 0.0, s21 = 0.0;
-#pragma unroll
-            for (u32 j = 0; j < MAXS; ++j) {
-                const double c0 = g->half[0][j], c1 = g->half[1][j];
-                s00 = __builtin_fma(yd[j], c0, s00);
-                s01 = __builtin_fma(yd[j], c1, s01);
-                s10 = __builtin_fma(yh[j], c0, s10);
-                s11 = __builtin_fma(yh[j], c1, s11);
-                s20 = __builtin_fma(yx[j], c0, s20);
-                s21 = __builtin_fma(yx[j], c1, s21);
-            }
-            s00 = __builtin_fma(ed, g->nq_half[0], s00);
-            s01 = __builtin_fma(ed, g->nq_half[1], s01);
-            const double t1 = __builtin_fma(s01, 32.0, s10), t2 = __builtin_fma(s11, 32.0, s20);
-            double acc = s00 + fmulmod(t1, g->p20.w, g->p20.wq, r);
-            acc = acc + fmulmod(t2, g->p40.w, g->p40.wq, r);
-            acc = acc + fmulmod(s21, g->p65.w, g->p65.wq, r);
-            o = d2u(fcanon(acc, r, rinv));
-        } else if (g->mode == TGT_SPLIT) {
-            // y_j = yh 2^30 + yl: y_j c = yh (2^30 c) + yl c (mod r), four terms between reductions.
+        if (MAXS <= WRAP_SRC && g->wrap == WRAP_LARGE) {
+            o = conv_wrap_large<MAXS>(g, Y.y, Y.yd, (u32)Y.e);
+        } else if (MAXS > WRAP_SRC && g->mode != TGT_INT) {
+            // f64 modular products: the source's own (TGT_FP), or its 30-bit halves
             const double r = g->rf, rinv = g->rinv;
             double acc = -g->hmod_f;
-#pragma unroll
-            for (u32 j = 0; j < MAXS; ++j) {
-                acc = acc + fmulmod(yd[j], g->qhat_f[j], g->qhat_q[j], r);
-                acc = acc + fmulmod(yh[j], g->qhat30_f[j], g->qhat30_q[j], r);
-                if (j & 1) acc = freduce(acc, r, rinv);
-            }
-            if constexpr (MAXS <= 8)
-                acc = __builtin_fma(ed, g->nq_c, acc);
-            else if (P.exact)
-                acc = acc - fmulmod(ed, g->qmod_f, g->qmod_q, r);
-            o = d2u(fcanon(acc, r, rinv));
-        } else if (g->mode == TGT_FP) {
-            const double r = g->rf, rinv = g->rinv;
-            double acc = -g->hmod_f;
-#pragma unroll
-            for (u32 j = 0; j < MAXS; ++j) {
-                acc = acc + fmulmod(yd[j], g->qhat_f[j], g->qhat_q[j], r);
-                if ((j & 3) == 3) acc = freduce(acc, r, rinv);
-            }
-            if constexpr (MAXS <= 8)
-                acc = __builtin_fma(ed, g->nq_c, acc);
-            else if (P.exact)
-                acc = acc - fmulmod(ed, g->qmod_f, g->qmod_q, r);
-            o = d2u(fcanon(acc, r, rinv));
-        } else {
-            const PrimeConst C = pc_int(pcs + g->prime);
-            if constexpr (MAXS <= 7) {
-                // sum_j y_j c_j from 32-bit halves (y_j, c_j < 2^60): y c = y0 c0 + (y0 c1 +
-                // y1 c0) 2^32 + y1 c1 2^64 with y1, c1 < 2^28, so the middle sum stays below
-                // 7 * 2^61 < 2^64 and the high one below 2^59; one 32 x 32 -> 64 multiply per
-                // partial product instead of full 64 x 64 products. The same exact sum, which
-                // starts at -(Q - 1)/2 mod r and takes e (-Q mod r) as one more term (e < 7).
-                u64 l = g->nh, m = 0, h = 0;
-                u32 carry = 0;
+            if (g->mode == TGT_FP) {
 #pragma unroll
                 for (u32 j = 0; j < MAXS; ++j) {
-                    const u64 cj = g->qhat[j];
-                    const u32 y0 = (u32)y[j], y1 = (u32)(y[j] >> 32), c0 = (u32)cj, c1 = (u32)(cj >> 32);
-                    const u64 p = (u64)y0 * c0;
-                    l += p;
-                    carry += l < p ? 1u : 0u;
-                    m += (u64)y0 * c1 + (u64)y1 * c0;
-                    h += (u64)y1 * c1;
-                    // one term at a time: otherwise the compiler forms every term's products
-                    // first and holds them all (92 VGPRs instead of 66 with y-form inputs)
-                    CKH_OPAQUE(l);
-                    CKH_OPAQUE(m);
-                    CKH_OPAQUE(h);
+                    acc = acc + fmulmod(Y.yd[j], g->qhat_f[j], g->qhat_q[j], r);
+                    if ((j & 3) == 3) acc = freduce(acc, r, rinv);
                 }
-                {
-                    const u64 p = (u64)(u32)e * (u32)g->nq;
-                    l += p;
-                    carry += l < p ? 1u : 0u;
-                    m += (u64)(u32)e * (u32)(g->nq >> 32);
-                }
-                const u64 lo = l + (m << 32);
-                const u64 hi = h + carry + (m >> 32) + (lo < l ? 1 : 0);
-                o = reduce128(hi, lo, C);
             } else {
-                Dot60 acc;
 #pragma unroll
-                for (u32 j = 0; j < MAXS; ++j) acc.add(y[j], g->qhat[j]);
-                u64 hi, lo;
-                acc.get(hi, lo);
-                o = reduce128(hi, lo, C);
-                if (P.exact) o = sub_mod(o, shoup(e, g->qmod, g->qmod_s, C.q), C.q);
-                o = sub_mod(o, g->hmod, C.q);
+                for (u32 j = 0; j < MAXS; ++j) {
+                    const double lo = (double)(u32)(Y.y[j] & ((1u << 30) - 1)), hi = (double)(u32)(Y.y[j] >> 30);
+                    acc = acc + fmulmod(lo, g->qhat_f[j], g->qhat_q[j], r);
+                    acc = acc + fmulmod(hi, g->qhat30_f[j], g->qhat30_q[j], r);
+                    if (j & 1) acc = freduce(acc, r, rinv);
+                }
             }
+            if (P.exact) acc = acc - fmulmod(ed, g->qmod_f, g->qmod_q, r);
+            o = d2u(fcanon(acc, r, rinv));
+        } else {
+            // sources of any size to a target of at least 2^50: the exact 128-bit sum
+            const PrimeConst C = pc_int(pcs + g->prime);
+            Dot60 acc;
+#pragma unroll
+            for (u32 j = 0; j < MAXS; ++j) acc.add(Y.y[j], g->qhat[j]);
+            u64 hi, lo;
+            acc.get(hi, lo);
+            o = reduce128(hi, lo, C);
+            if (P.exact) o = sub_mod(o, shoup(Y.e, g->qmod, g->qmod_s, C.q), C.q);
+            o = sub_mod(o, g->hmod, C.q);
         }
         st_nt(outp, (u64)g->limb * n + c, o);
     }

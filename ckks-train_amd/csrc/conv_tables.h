@@ -72,18 +72,7 @@ struct HostConvTables {
                 t.qmod_q = (double)t.qmod / (double)r;
                 t.hmod_f = (double)t.hmod;
                 t.nq = (r - t.qmod % r) % r;
-                t.nh = (r - t.hmod % r) % r;
                 t.nq_c = t.nq > r / 2 ? -(double)(r - t.nq) : (double)t.nq;
-                for (u32 b = 0; b < 2; ++b) {
-                    t.nq_half[b] = (double)((t.nq >> (25 * b)) & ((1u << 25) - 1));
-                    t.nh_half[b] = (double)((t.nh >> (25 * b)) & ((1u << 25) - 1));
-                }
-                if (r < FP_PRIME_BOUND) {
-                    for (auto [sh, dst] : {std::pair<u32, FTw*>{20, &t.p20}, {40, &t.p40}, {65, &t.p65}}) {
-                        const u64 v = hm::pow(2, sh, r);
-                        *dst = {(double)v, (double)v / (double)r};
-                    }
-                }
                 for (size_t j = 0; j < src.size(); ++j) {
                     u64 qh = 1 % r;
                     for (size_t i = 0; i < src.size(); ++i)
@@ -94,14 +83,35 @@ struct HostConvTables {
                     const u64 qh30 = hm::mul(qh, (1ull << 30) % r, r);
                     t.qhat30_f[j] = (double)qh30;
                     t.qhat30_q[j] = (double)qh30 / (double)r;
-                    for (u32 b = 0; b < 2; ++b) t.half[b][j] = (double)((qh >> (25 * b)) & ((1u << 25) - 1));
                 }
+                if (src.size() <= WRAP_SRC && (srcs_fp || r < FP_PRIME_BOUND)) set_wrap(t, src.size(), r, srcs_fp);
                 tgts.push_back(t);
             }
         }
         pl.ntgt = (u32)tg.size();
         plans.push_back(pl);
         return (u32)plans.size() - 1;
+    }
+
+    // The single-quotient form of a target (conv_wrap_small / conv_wrap_large), from its c_j.
+    static void set_wrap(ConvTgt& t, size_t nsrc, u64 r, bool small) {
+        auto centered = [r](u64 v) { return v > r / 2 ? v - r : v; };  // two's complement
+        t.wrap = small ? WRAP_SMALL : WRAP_LARGE;
+        const double unit = small ? (double)r : 2048.0 * (double)r;
+        u64 csum = 0;
+        for (size_t j = 0; j < nsrc; ++j) {
+            t.cw[j] = centered(t.qhat[j]);
+            t.cq[j] = (double)(int64_t)t.cw[j] / unit;
+            csum = (csum + t.qhat[j]) % r;
+        }
+        t.r = r;
+        t.nr = (small ? 0 : 0 - (r << 10)) - (small ? r : r << 10);  // -r, or -2^11 r modulo 2^64
+        t.nqw = centered(t.nq);
+        t.nqq = (double)(int64_t)t.nqw / unit;
+        u64 a = (r - t.hmod % r) % r;
+        if (small) a = (a + hm::mul(WRAP_CENTER % r, csum, r)) % r;
+        t.aq = (double)a / unit;
+        t.aw = a - WRAP_ROUND_BITS * t.nr;
     }
 
     // The YForm of every source (same index as srcs), from each prime's inverse-NTT constants.

@@ -291,7 +291,9 @@ class Context : public std::enable_shared_from_this<Context> {
     // Tuning (autotune.cpp): limbs per column-pass/row-pass launch pair (0 = all at once). A
     // chunk small enough keeps the pass intermediate in the on-die caches between the passes.
     u32 ntt_chunk_fwd = 0, ntt_chunk_inv = 0;
-    u32 conv_variant = 0, conv_tg = 8;  // base-conversion kernel variant and targets per workgroup
+    u32 conv_variant = 0, conv_tg = 32;  // base-conversion kernel variant and targets per workgroup
+    // (all of them: the sources are read once; 8 per workgroup took 17.54 against 16.83 ms per step of
+    // 256 switches at N = 2^16, 3.65 against 3.60 ms for the 32 x 32 product at 2^15)
     // The variant of mod_down's conversions (P -> Q) in batched programs (tuning key
     // "conv_variant_md"; 3 = conv_variant). Default 1: with 60-bit sources the exact f64 piece
     // sums beat two modular products per source (step 19.98 -> 19.54 ms on the 256-switch
