@@ -146,15 +146,13 @@ CKH_DEV u64 mul_mod(u64 a, u64 b, const PrimeConst& c) { return reduce128(mulhi(
 
 // ---- f64 arithmetic for primes below 2^50 (FP_PRIME_BOUND): residues as integer-valued f64.
 
-// u64 < 2^53 -> f64, exact.
-CKH_DEV double u2d(u64 v) { return __builtin_fma((double)(u32)(v >> 32), 4294967296.0, (double)(u32)v); }
+// u64 < 2^52 -> f64, exact: as the mantissa of 2^52 + v.
+CKH_DEV double u2d(u64 v) { return bits_f64(v | 0x4330000000000000ull) - 4503599627370496.0; }
 
-// Non-negative integer-valued f64 below 2^53 -> u64, exact.
-CKH_DEV u64 d2u(double d) {
-    const u32 hi = (u32)(d * (1.0 / 4294967296.0));
-    const double lo = __builtin_fma(-(double)hi, 4294967296.0, d);
-    return ((u64)hi << 32) | (u32)lo;
-}
+// Non-negative integer-valued f64 below 2^52 -> u64, exact, the same way back. (Against the
+// conversions of the two halves and an FMA these are two operations instead of three and five;
+// a conversion issues at the rate of an f64 operation.)
+CKH_DEV u64 d2u(double d) { return f64_bits(d + 4503599627370496.0) & 0x000fffffffffffffull; }
 
 // y w mod q as a signed integer-valued f64, for integer-valued y, w with |w| < q < 2^50 and
 // wq = w / q rounded once or twice: h = RN(y w) and l = fma(y, w, -h) split the product
