@@ -171,7 +171,8 @@ CKH_DEV u64 csub_sign(u64 x, u64 m) {
     return (int64_t)d < 0 ? x : d;
 }
 
-// The residue of one target g from the sources of a WRAP_SMALL conversion, y_j given minus 2^49.
+// One target g from the sources of a WRAP_SMALL conversion, y_j given minus 2^49: T - k r + 2 r,
+// below 4 r.
 template <u32 MAXS, class Tgt>
 CKH_DEV u64 conv_wrap_small(const Tgt& g, const u64 (&y)[MAXS], const double (&yd)[MAXS], u32 e, double ed) {
     u64 l = g->aw + (g->r << 1), m = 0;
@@ -185,11 +186,10 @@ CKH_DEV u64 conv_wrap_small(const Tgt& g, const u64 (&y)[MAXS], const double (&y
     }
     // rint(F) as the low bits of F + 1.5 2^52 (the constant's own bits are in aw)
     mad_wrap(l, m, f64_bits(F + WRAP_ROUND), g->nr);
-    // T - k r + 2 r, below 4 r
-    return csub_sign(csub_sign(wrap_word(l, m), g->r << 1), g->r);
+    return wrap_word(l, m);
 }
 
-// The residue of one target from the sources of a WRAP_LARGE conversion.
+// One target from the sources of a WRAP_LARGE conversion: congruent to T, below (1 + 2^-20) r.
 template <u32 MAXS, class Tgt>
 CKH_DEV u64 conv_wrap_large(const Tgt& g, const u64 (&y)[MAXS], const double (&yd)[MAXS], u32 e) {
     const u64 r = g->r;
@@ -209,7 +209,20 @@ CKH_DEV u64 conv_wrap_large(const Tgt& g, const u64 (&y)[MAXS], const double (&y
     const double ud = __builtin_fma((double)(u32)(U >> 32), 4294967296.0, (double)(u32)U);
     const double kd = __builtin_fma(ud, g->rinv, -0x1p-20);
     const u32 k = (u32)kd;  // a negative estimate (U < 2^-20 r) converts to 0
-    return csub_sign(U - (u64)k * r, r);
+    return U - (u64)k * r;
+}
+
+// One target of at least 2^50 from sources of any size: the exact 128-bit sum, reduced.
+template <u32 MAXS, class Tgt>
+CKH_DEV u64 conv_dot60(const Tgt& g, const PrimeConst& C, const u64 (&y)[MAXS], u64 e, bool exact) {
+    Dot60 acc;
+#pragma unroll
+    for (u32 j = 0; j < MAXS; ++j) acc.add(y[j], g->qhat[j]);
+    u64 hi, lo;
+    acc.get(hi, lo);
+    u64 o = reduce128(hi, lo, C);
+    if (exact) o = sub_mod(o, shoup(e, g->qmod, g->qmod_s, C.q), C.q);
+    return sub_mod(o, g->hmod, C.q);
 }
 
 // Coefficient c of one conversion (plan P, input polynomial in_p, output out_p, N = n): the
@@ -234,7 +247,8 @@ CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeCon
             }
             for (u32 t = t0; t < t1; ++t) {
                 const auto* g = cst(tgts + P.tgt_first + t);
-                st_nt(outp, (u64)g->limb * n + c, conv_wrap_small<MAXS>(g, Y.y, Y.yd, (u32)Y.e, ed));
+                const u64 o = conv_wrap_small<MAXS>(g, Y.y, Y.yd, (u32)Y.e, ed);
+                st_nt(outp, (u64)g->limb * n + c, csub_sign(csub_sign(o, g->r << 1), g->r));
             }
             return;
         }
@@ -243,7 +257,7 @@ CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeCon
         const auto* g = cst(tgts + P.tgt_first + t);
         u64 o;
         if (MAXS <= WRAP_SRC && g->wrap == WRAP_LARGE) {
-            o = conv_wrap_large<MAXS>(g, Y.y, Y.yd, (u32)Y.e);
+            o = csub_sign(conv_wrap_large<MAXS>(g, Y.y, Y.yd, (u32)Y.e), g->r);
         } else if (MAXS > WRAP_SRC && g->mode != TGT_INT) {
             // f64 modular products: the source's own (TGT_FP), or its 30-bit halves
             const double r = g->rf, rinv = g->rinv;
@@ -266,16 +280,7 @@ CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeCon
             if (P.exact) acc = acc - fmulmod(ed, g->qmod_f, g->qmod_q, r);
             o = d2u(fcanon(acc, r, rinv));
         } else {
-            // sources of any size to a target of at least 2^50: the exact 128-bit sum
-            const PrimeConst C = pc_int(pcs + g->prime);
-            Dot60 acc;
-#pragma unroll
-            for (u32 j = 0; j < MAXS; ++j) acc.add(Y.y[j], g->qhat[j]);
-            u64 hi, lo;
-            acc.get(hi, lo);
-            o = reduce128(hi, lo, C);
-            if (P.exact) o = sub_mod(o, shoup(Y.e, g->qmod, g->qmod_s, C.q), C.q);
-            o = sub_mod(o, g->hmod, C.q);
+            o = conv_dot60<MAXS>(g, pc_int(pcs + g->prime), Y.y, Y.e, P.exact);
         }
         st_nt(outp, (u64)g->limb * n + c, o);
     }

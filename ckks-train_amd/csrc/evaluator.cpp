@@ -328,7 +328,7 @@ static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
     Program prog;  // one program (one graph when captured) per batched switch
     if (pre) prog.step(S_AUTOMORPH, prog.add(*pre), (u32)pre->size());
     c.prog_decompose(prog, dec, small ? c.conv_variant_s : c.conv_variant);
-    c.prog_apply(prog, app);
+    c.prog_apply(prog, app, small ? c.conv_variant_s : c.md_variant());
     if (small) prog.set_conv_schedule(c.conv_variant_s, c.conv_tg_s);
     return prog;
 }
@@ -952,7 +952,7 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
     }
     Program prog;
     prog.step(S_AUTOMORPH, prog.add(aut), (u32)aut.size());
-    ctx.prog_apply(prog, tasks);
+    ctx.prog_apply(prog, tasks, ctx.md_variant());
     ctx.execute(prog, s);
     hip_check(hipGetLastError(), "hoisted rotate");
     count(&ckh_op_counter::rotations, nontrivial);
@@ -1040,7 +1040,7 @@ std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
     ctx.decompose(dec, s);
     Program prog;
     prog.step(S_AUTOMORPH, prog.add(aut), (u32)aut.size());
-    ctx.prog_apply(prog, tasks);
+    ctx.prog_apply(prog, tasks, ctx.md_variant());
     ctx.execute(prog, s);
     hip_check(hipGetLastError(), "hoisted rotate");
     count(&ckh_op_counter::rotations, nontrivial);

@@ -64,6 +64,18 @@ void ntt_fast_forward_finish(const NttTables& t, const LimbRef* refs, const Fini
 void ntt_fast_forward_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t stream);
 void ntt_fast_forward_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t stream);
 
+// The row pass alone with the finish of ntt_fast_forward_finish.
+void ntt_fast_forward_rows_finish(const NttTables& t, const LimbRef* refs, const FinishJob* fin, u32 nrefs,
+                                  hipStream_t stream);
+
+// Base conversions of at most WRAP_SRC sources (y form) fused with the column pass of every target:
+// each ref's limb holds the column pass's f64 / lazy intermediates afterwards, as after
+// ntt_fast_forward_cols.
+struct ConvTables;
+struct ConvColRef;
+void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
+                      hipStream_t stream);
+
 void rows_ip_launch(const NttTables& t, const RowIpJob* jobs, u32 njobs, hipStream_t stream);
 
 void rows_ip_fin_launch(const NttTables& t, const RowIpFinJob* jobs, u32 njobs, hipStream_t stream);

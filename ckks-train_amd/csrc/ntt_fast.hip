@@ -22,6 +22,7 @@ CKH_DEV u64 load_coherent(const u64* p) {
 }  // namespace ckh
 
 #include "ntt_passes.h"
+#include "conv_cols.h"
 
 namespace ckh {
 namespace fast {
@@ -70,6 +71,40 @@ __global__ __launch_bounds__(NT) void k_fwd_cols(const LimbRef* __restrict__ ref
                                                  u32 nrefs) {
     __shared__ u64 lds[LDS_WORDS];
     CKH_AR_DISPATCH((fwd_cols<M>(ar, ref.src, ref.dst, lds, log_n, tile)))
+}
+
+// The base conversion of a target fused with its column pass (conv_cols.h). Workgroups are dealt
+// round-robin to the 8 XCDs, so each XCD takes one contiguous run of work items: the targets of one
+// tile run on one XCD and share its sources in that L2 (1.9 GB fetched for the ModUp conversions of
+// 256 switches, each source once). Held to 4 waves per SIMD: 63 us for a switch's two conversions at
+// N = 2^16, 65-67 us at the 3 waves of 135-148 VGPRs.
+template <u32 M, u32 MAXS>
+__global__ __launch_bounds__(NT, MAXS <= 6 ? 4 : 3) void k_conv_cols(ConvTables T, const ConvColRef* __restrict__ refs,
+                                                  const Tw* __restrict__ tw, const FTw* __restrict__ twf, u32 items) {
+    __shared__ u64 lds[LDS_WORDS];
+    const u32 log_n = T.log_n;
+    const u32 item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (item >= items) return;
+    const ConvColRef R = refs[item >> (log_n - TL)];
+    u32 tile;
+    const u32 t = conv_col_item(R, item, 1u << (log_n - TL), tile);
+    const auto* g = cst(T.tgt + R.tgt_first + t);
+    const u32 prime = g->prime;
+    const PrimeConst* pc = T.pc + prime;
+    const u64 toff = (u64)prime << log_n;
+    u64* const out = R.out + ((u64)g->limb << log_n);
+    const u32 tid = threadIdx.x;
+    if (pc->q < FP_PRIME_BOUND) {
+        const FpAr ar{twf + toff, pc->qf, pc->qinv, {}, {}, nullptr};
+        double v[16];
+        conv_tile<M, MAXS>(ar, T.src, R, g, pc, log_n, tile, tid, v);
+        fwd_cols_tile<M>(ar, v, out, lds, log_n, tile, tid);
+    } else {
+        const IntAr ar{tw + toff, pc->q, 0, 0, 0, 0};
+        u64 v[16];
+        conv_tile<M, MAXS>(ar, T.src, R, g, pc, log_n, tile, tid, v);
+        fwd_cols_tile<M>(ar, v, out, lds, log_n, tile, tid);
+    }
 }
 
 // FIN: the finish variant (a separate instantiation: its prefetched operands cost registers).
@@ -468,6 +503,38 @@ void rows_ip_launch(const NttTables& t, const RowIpJob* jobs, u32 njobs, hipStre
         case 6: hipLaunchKernelGGL(fast::k_rows_ip<6>, grid, dim3(fast::NT), 0, s, jobs, t.pc, t.fwd_f, t.rf, t.log_n, njobs); break;
         case 7: hipLaunchKernelGGL(fast::k_rows_ip<7>, grid, dim3(fast::NT), 0, s, jobs, t.pc, t.fwd_f, t.rf, t.log_n, njobs); break;
         default: hipLaunchKernelGGL(fast::k_rows_ip<8>, grid, dim3(fast::NT), 0, s, jobs, t.pc, t.fwd_f, t.rf, t.log_n, njobs); break;
+    }
+}
+
+void ntt_fast_forward_rows_finish(const NttTables& t, const LimbRef* refs, const FinishJob* fin, u32 nrefs,
+                                  hipStream_t s) {
+    launch_m(t.log_n / 2, true, false, t, refs, nrefs, s, fin);
+}
+
+template <u32 M>
+static void conv_cols_m(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 items, u32 max_src,
+                        hipStream_t s) {
+    const dim3 grid((items + 7) / 8 * 8), block(fast::NT);
+    if (max_src <= 1)
+        hipLaunchKernelGGL((fast::k_conv_cols<M, 1>), grid, block, 0, s, c, refs, t.fwd, t.fwd_f, items);
+    else if (max_src <= 2)
+        hipLaunchKernelGGL((fast::k_conv_cols<M, 2>), grid, block, 0, s, c, refs, t.fwd, t.fwd_f, items);
+    else if (max_src <= 4)
+        hipLaunchKernelGGL((fast::k_conv_cols<M, 4>), grid, block, 0, s, c, refs, t.fwd, t.fwd_f, items);
+    else if (max_src <= 6)
+        hipLaunchKernelGGL((fast::k_conv_cols<M, 6>), grid, block, 0, s, c, refs, t.fwd, t.fwd_f, items);
+    else
+        hipLaunchKernelGGL((fast::k_conv_cols<M, 8>), grid, block, 0, s, c, refs, t.fwd, t.fwd_f, items);
+}
+
+void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
+                      hipStream_t s) {
+    if (nrefs == 0) return;
+    const u32 items = nrefs << (t.log_n - fast::TL);
+    switch (t.log_n - t.log_n / 2) {
+        case 6: conv_cols_m<6>(c, t, refs, items, max_src, s); break;
+        case 7: conv_cols_m<7>(c, t, refs, items, max_src, s); break;
+        default: conv_cols_m<8>(c, t, refs, items, max_src, s); break;
     }
 }
 

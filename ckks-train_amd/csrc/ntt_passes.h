@@ -69,6 +69,8 @@ struct FpAr {
     const FTw* rt;    // this prime's row factors, [row][ROW_FACTOR_SLOTS]
     double add = 0.0; // added to the outputs of gs_final<true> (an integer below q)
     CKH_DEV V from_canon(u64 x) const { return u2d(x); }
+    // a word x in (0, 4 q) standing for x - 2 q
+    CKH_DEV V from_wrapped(u64 x) const { return u2d(x) - (q + q); }
     CKH_DEV V from_mid(u64 x) const { return bits_f64(x); }
     CKH_DEV u64 to_mid(V v) const { return f64_bits(v); }
     CKH_DEV W tw(u32 idx) const { return tab[idx]; }
@@ -143,6 +145,7 @@ struct IntAr {
     u64 n_inv, n_inv_s, w_n_inv, w_n_inv_s;
     u64 add = 0;  // added to the outputs of gs_final<true> (below q)
     CKH_DEV V from_canon(u64 x) const { return x; }
+    CKH_DEV V from_wrapped(u64 x) const { return x; }  // below 4 q, congruent as it is
     CKH_DEV V from_mid(u64 x) const { return x; }
     CKH_DEV u64 to_mid(V v) const { return v; }
     CKH_DEV W tw(u32 idx) const { return tab[idx]; }
@@ -294,18 +297,15 @@ CKH_DEV void rows_round2_inv(const Ar& ar, typename Ar::V (&v)[16], u32 A, u32 r
 // four top bits vary). "e-layout": it holds ((hh << U | u) << R2) | j, e = (u << R2) | j (the
 // R2 low bits vary, plus U of the top bits).
 
+// The column pass of one tile from its loaded words (k-layout) on.
 template <u32 M, class Ar, class Lds>
-CKH_DEV void fwd_cols(const Ar& ar, const u64* __restrict__ in_p, u64* __restrict__ out_p, Lds lds, u32 log_n,
-                      u32 tile, u32 tid = threadIdx.x) {
-    const auto in = glb(in_p);
+CKH_DEV void fwd_cols_tile(const Ar& ar, typename Ar::V (&v)[16], u64* __restrict__ out_p, Lds lds, u32 log_n, u32 tile,
+                           u32 tid) {
     const auto out = glb(out_p);
     constexpr u32 R2 = M - 4, U = 4 - R2, TCL = TL - M, TC = 1u << TCL, JM = (1u << R2) - 1;
     const u32 B = log_n - M;
     const u32 cc = tid & (TC - 1), o = tid >> TCL;
     const u32 c0 = tile * TC;
-    typename Ar::V v[16];
-#pragma unroll
-    for (u32 k = 0; k < 16; ++k) v[k] = ar.from_canon(in[((u64)(o + (k << R2)) << B) + c0 + cc]);
 #pragma unroll
     for (u32 s = 0; s < 4; ++s) {
 #pragma unroll
@@ -338,6 +338,21 @@ CKH_DEV void fwd_cols(const Ar& ar, const u64* __restrict__ in_p, u64* __restric
         const u32 r = ((((o << U) | (e >> R2)) << R2) | (e & JM));
         out[((u64)r << B) + c0 + cc] = ar.to_mid(v[e]);
     }
+}
+
+
+template <u32 M, class Ar, class Lds>
+CKH_DEV void fwd_cols(const Ar& ar, const u64* __restrict__ in_p, u64* __restrict__ out_p, Lds lds, u32 log_n,
+                      u32 tile, u32 tid = threadIdx.x) {
+    const auto in = glb(in_p);
+    constexpr u32 R2 = M - 4, TCL = TL - M, TC = 1u << TCL;
+    const u32 B = log_n - M;
+    const u32 cc = tid & (TC - 1), o = tid >> TCL;
+    const u32 c0 = tile * TC;
+    typename Ar::V v[16];
+#pragma unroll
+    for (u32 k = 0; k < 16; ++k) v[k] = ar.from_canon(in[((u64)(o + (k << R2)) << B) + c0 + cc]);
+    fwd_cols_tile<M>(ar, v, out_p, lds, log_n, tile, tid);
 }
 
 // The row pass of one tile, its canonical outputs left in LDS in natural order (word i of the

@@ -530,6 +530,13 @@ void Context::build_tables() {
     conv.yf = dev_copy(ct.yform(t.pc));
     conv_src_first_.clear();
     for (const ConvPlan& pl : plans) conv_src_first_.push_back(pl.src_first);
+    conv_plans_ = plans;
+    conv_small_.clear();
+    for (const ConvPlan& pl : plans) {
+        u32 small = 1;
+        for (u32 j = 0; j < pl.nsrc; ++j) small = small && ct.srcs[pl.src_first + j].fp;
+        conv_small_.push_back(small);
+    }
     conv.tgt = dev_copy(ct.tgts);
     conv.plans = dev_copy(plans);
     conv.pc = d_pc;
@@ -640,6 +647,10 @@ void Context::run(const Program& p, const uint8_t* d, hipStream_t s) const {
             case S_FINISH: launch_finish((const FinishJob*)x, st.count, d_pc, log_n, s); break;
             case S_NTT_COLS: ntt_fast_forward_cols(ntt, (const LimbRef*)x, st.count, s); break;
             case S_NTT_ROWS: ntt_fast_forward_rows(ntt, (const LimbRef*)x, st.count, s); break;
+            case S_NTT_ROWS_FIN:
+                ntt_fast_forward_rows_finish(ntt, (const LimbRef*)x, (const FinishJob*)(d + st.off2), st.count, s);
+                break;
+            case S_CONV_COLS: conv_cols_launch(conv, ntt, (const ConvColRef*)x, st.count, st.a, s); break;
             case S_ROWS_IP: rows_ip_launch(ntt, (const RowIpJob*)x, st.count, s); break;
             case S_ROWS_IP_FIN: rows_ip_fin_launch(ntt, (const RowIpFinJob*)x, st.count, s); break;
             case S_ADD_SUM:
@@ -797,11 +808,26 @@ static void group_by_prime(std::vector<LimbRef>& r) {
 
 bool Context::yform_usable(u32 mask_bit) const { return (conv_yform & mask_bit) && ntt_fast_supported(log_n); }
 
+bool Context::conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const {
+    return conv_cols && nsrc <= WRAP_SRC && !(variant == 2 && conv.mf_ok) && ntt_fast_supported(log_n) && !fused_usable() &&
+           (nsrc <= CONV_COLS_ALWAYS || targets << (log_n - 12) <= CONV_COLS_ITEMS);
+}
+
+void Context::add_conv_cols(std::vector<ConvColRef>& refs, u32 plan, const u64* src, u64* out) const {
+    const ConvPlan& P = conv_plans_[plan];
+    const u32 first = (u32)refs.size();
+    refs.insert(refs.end(), P.ntgt, {src, out, first, P.ntgt, P.src_first, P.tgt_first, P.nsrc, conv_small_[plan]});
+}
+
 void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 variant) const {
     std::vector<LimbRef> intt, copies, nttr, cols;
     std::vector<ConvJob> jobs;
+    std::vector<ConvColRef> ccols;
     u32 max_tgt = 0;
     const bool yf = yform_usable(variant == 2 && conv.mf_ok ? 4 : 1);
+    u64 targets = 0;
+    for (const DecTask& t : tasks) targets += (u64)ndigits(t.level) * (t.level + 1 + np) - (t.level + 1);
+    const bool cc = yf && conv_cols_usable(alpha, targets, variant);
     for (const DecTask& t : tasks) {
         const u32 L = t.level + 1;
         const u64 ds = digit_words(t.level);
@@ -812,7 +838,10 @@ void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 
                                 yf ? conv_src_first_[modup_plan_[t.level][j]] + (i - dr[j].first) : 0});
         for (u32 j = 0; j < dr.size(); ++j) {
             u64* dj = t.dig + j * ds;
-            jobs.push_back({t.x, dj, modup_plan_[t.level][j], 0});
+            if (cc)
+                add_conv_cols(ccols, modup_plan_[t.level][j], t.x + dr[j].first * n, dj);
+            else
+                jobs.push_back({t.x, dj, modup_plan_[t.level][j], 0});
             if (t.copy_own)
                 for (u32 i = dr[j].first; i < dr[j].second; ++i) copies.push_back({t.d + i * n, dj + i * n, i, 0});
             for (u32 i = 0; i < L; ++i)
@@ -830,13 +859,18 @@ void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 
     p.step(S_CONV, p.add(jobs), (u32)jobs.size(), 0, max_tgt, alpha);
     if (!jobs.empty()) p.steps.back().yform = yf;
     p.step(S_COPY, p.add(copies), (u32)copies.size());
+    if (cc) {
+        p.step(S_CONV_COLS, p.add(ccols), (u32)ccols.size(), 0, alpha);
+        p.step(S_NTT_ROWS, p.add(nttr), (u32)nttr.size());
+        return;
+    }
     p.step_ntt(S_NTT_FWD, p.add(nttr), (u32)nttr.size(), 0, fused_usable());
     p.step(S_NTT_COLS, p.add(cols), (u32)cols.size());
 }
 
 // keyswitch::apply_key (keyswitch.rs:230-309) for a batch: the inner product over Q_l * P, then
 // mod_down of both sums.
-void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const {
+void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const {
     std::vector<IpJob> ip;
     u32 max_l = 0;
     for (const ApplyTask& t : tasks) max_l = std::max(max_l, t.level + 1);
@@ -858,7 +892,10 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const 
         p.step(S_IP, p.add(ip), (u32)ip.size());
         std::vector<LimbRef> intt, cols;
         std::vector<ConvJob> jobs;
-        const bool yf = yform_usable(2);
+        std::vector<ConvColRef> ccols;
+        u64 targets = 0;
+        for (const ApplyTask& t : tasks) targets += 2 * (t.level + 1);
+        const bool yf = yform_usable(2), cc = yf && conv_cols_usable(np, targets, md_variant);
         for (const ApplyTask& t : tasks) {
             const u32 L = t.level + 1;
             const u64 aw = (u64)(L + np) * n;
@@ -868,6 +905,10 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const 
                 u64* z = t.z + (u64)part * L * n;
                 const u32 sf = conv_src_first_[moddown_plan_[t.level]];
                 for (u32 k = 0; k < np; ++k) intt.push_back({acc + (L + k) * n, y + k * n, nq + k, yf ? sf + k : 0});
+                if (cc) {
+                    add_conv_cols(ccols, moddown_plan_[t.level], y, z);
+                    continue;
+                }
                 jobs.push_back({y, z, moddown_plan_[t.level], 0});
                 for (u32 i = 0; i < L; ++i) cols.push_back({z + i * n, z + i * n, i, 0});
             }
@@ -896,8 +937,9 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const 
             p.step_ntt(S_NTT_INV, p.add(intt), (u32)intt.size(), 0, fused_usable());
         p.step(S_CONV, p.add(jobs), (u32)jobs.size(), 0, max_l, np);
         if (!jobs.empty()) p.steps.back().yform = yf;
-        if (conv_variant_md < 3 && !jobs.empty()) p.steps.back().sched = 1u | (conv_variant_md << 1) | (conv_tg << 8);
+        if (!jobs.empty()) p.steps.back().sched = 1u | (md_variant << 1) | (conv_tg << 8);
         p.step(S_NTT_COLS, p.add(cols), (u32)cols.size());
+        p.step(S_CONV_COLS, p.add(ccols), (u32)ccols.size(), 0, np);
         p.step(S_ROWS_IP_FIN, p.add(rf), (u32)rf.size());
         return;
     }
@@ -926,23 +968,29 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const 
         md.push_back({t.acc, t.level, t.out_b, t.add_b, t.y, t.z});
         md.push_back({t.acc + aw, t.level, t.out_a, t.add_a, t.y + (u64)np * n, t.z + (u64)L * n});
     }
-    prog_mod_down(p, md);
+    prog_mod_down(p, md, md_variant);
 }
 
 // RnsPoly::mod_down (baseconv.rs:459-511) for a batch: INTT of the P limbs, the centered exact
 // conversion P -> Q_l, NTT, and (x - t) * P^-1 (+ the optional addend).
-void Context::prog_mod_down(Program& p, const std::vector<MdTask>& tasks) const {
+void Context::prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 variant) const {
     std::vector<LimbRef> intt, nttr;
     std::vector<ConvJob> jobs;
     std::vector<FinishJob> fin;
+    std::vector<ConvColRef> ccols;
     u32 max_l = 0;
-    const bool yf = yform_usable(2);
+    u64 targets = 0;
+    for (const MdTask& t : tasks) targets += t.level + 1;
+    const bool yf = yform_usable(2), cc = yf && conv_cols_usable(np, targets, variant);
     for (const MdTask& t : tasks) {
         const u32 L = t.level + 1;
         max_l = std::max(max_l, L);
         const u32 sf = conv_src_first_[moddown_plan_[t.level]];
         for (u32 k = 0; k < np; ++k) intt.push_back({t.acc + (L + k) * n, t.y + k * n, nq + k, yf ? sf + k : 0});
-        jobs.push_back({t.y, t.z, moddown_plan_[t.level], 0});
+        if (cc)
+            add_conv_cols(ccols, moddown_plan_[t.level], t.y, t.z);
+        else
+            jobs.push_back({t.y, t.z, moddown_plan_[t.level], 0});
         for (u32 i = 0; i < L; ++i) {
             u64* zi = t.z + i * n;
             nttr.push_back({zi, zi, i, 0});
@@ -957,9 +1005,13 @@ void Context::prog_mod_down(Program& p, const std::vector<MdTask>& tasks) const 
         p.step_ntt(S_NTT_INV, p.add(intt), (u32)intt.size(), 0, fused_usable());
     p.step(S_CONV, p.add(jobs), (u32)jobs.size(), 0, max_l, np);
     if (!jobs.empty()) p.steps.back().yform = yf;
-    if (conv_variant_md < 3 && !jobs.empty()) p.steps.back().sched = 1u | (conv_variant_md << 1) | (conv_tg << 8);
+    if (!jobs.empty()) p.steps.back().sched = 1u | (variant << 1) | (conv_tg << 8);
+    p.step(S_CONV_COLS, p.add(ccols), (u32)ccols.size(), 0, np);
     const size_t o_ntt = p.add(nttr), o_fin = p.add(fin);
-    p.step_ntt(S_NTT_FWD_FIN, o_ntt, (u32)nttr.size(), o_fin, fused_usable());
+    if (cc)
+        p.step(S_NTT_ROWS_FIN, o_ntt, (u32)nttr.size(), o_fin);
+    else
+        p.step_ntt(S_NTT_FWD_FIN, o_ntt, (u32)nttr.size(), o_fin, fused_usable());
 }
 
 // RnsPoly::rescale_by_last in NTT form (baseconv.rs:258-291) for a batch.
@@ -967,11 +1019,16 @@ void Context::prog_rescale(Program& p, const std::vector<RescaleTask>& tasks) co
     std::vector<LimbRef> intt, nttr;
     std::vector<ConvJob> jobs;
     std::vector<FinishJob> fin;
+    std::vector<ConvColRef> ccols;
     u32 max_t = 0;
+    const bool cc = conv_cols_usable(1, 0, conv_variant);
     for (const RescaleTask& t : tasks) {
         const u32 l = t.level;
-        intt.push_back({t.in + l * n, t.x, l, 0});
-        jobs.push_back({t.x, t.z, rescale_plan_[l], 0});
+        intt.push_back({t.in + l * n, t.x, l, cc ? conv_src_first_[rescale_plan_[l]] : 0});
+        if (cc)
+            add_conv_cols(ccols, rescale_plan_[l], t.x, t.z);
+        else
+            jobs.push_back({t.x, t.z, rescale_plan_[l], 0});
         for (u32 i = 0; i < l; ++i) {
             nttr.push_back({t.z + i * n, t.z + i * n, i, 0});
             fin.push_back({t.in + i * n, t.z + i * n, t.out + i * n, nullptr, qlinv_[l][i], qlinv_s_[l][i], i, 0,
@@ -979,10 +1036,17 @@ void Context::prog_rescale(Program& p, const std::vector<RescaleTask>& tasks) co
         }
         max_t = std::max(max_t, l);
     }
-    p.step_ntt(S_NTT_INV, p.add(intt), (u32)intt.size(), 0, fused_usable());
+    if (cc)
+        p.step(S_NTT_INV_Y, p.add(intt), (u32)intt.size());
+    else
+        p.step_ntt(S_NTT_INV, p.add(intt), (u32)intt.size(), 0, fused_usable());
     p.step(S_CONV, p.add(jobs), (u32)jobs.size(), 0, max_t, 1);
+    p.step(S_CONV_COLS, p.add(ccols), (u32)ccols.size(), 0, 1);
     const size_t o_ntt = p.add(nttr), o_fin = p.add(fin);
-    p.step_ntt(S_NTT_FWD_FIN, o_ntt, (u32)nttr.size(), o_fin, fused_usable());
+    if (cc)
+        p.step(S_NTT_ROWS_FIN, o_ntt, (u32)nttr.size(), o_fin);
+    else
+        p.step_ntt(S_NTT_FWD_FIN, o_ntt, (u32)nttr.size(), o_fin, fused_usable());
 }
 
 // RnsPoly::raise_from_level0 (crates/ckks-train-core/src/poly.rs:298-345; the device form of
@@ -1026,13 +1090,13 @@ void Context::decompose(const std::vector<DecTask>& tasks, hipStream_t s) {
 
 void Context::apply(const std::vector<ApplyTask>& tasks, hipStream_t s) {
     Program p;
-    prog_apply(p, tasks);
+    prog_apply(p, tasks, md_variant());
     execute(p, s);
 }
 
 void Context::mod_down(const std::vector<MdTask>& tasks, hipStream_t s) {
     Program p;
-    prog_mod_down(p, tasks);
+    prog_mod_down(p, tasks, md_variant());
     execute(p, s);
 }
 

@@ -15,6 +15,7 @@
 #include "../../include/ckh.h"
 #include "basis.h"
 #include "common.h"
+#include "conv_col_ref.h"
 #include "lifetime.h"
 #include "ntt.h"
 #include "ops.h"
@@ -151,7 +152,7 @@ struct RaiseTask {
 // Descriptor bytes plus the launch steps that read them (see runtime.cpp, "engine").
 enum StepKind : uint8_t {
     S_NTT_FWD, S_NTT_INV, S_CONV, S_COPY, S_IP, S_NTT_FWD_FIN, S_FINISH, S_NTT_COLS, S_NTT_ROWS, S_ROWS_IP,
-    S_MUL_SUM, S_AUTOMORPH, S_ADD_SUM, S_ROWS_IP_FIN, S_NTT_INV_Y
+    S_MUL_SUM, S_AUTOMORPH, S_ADD_SUM, S_ROWS_IP_FIN, S_NTT_INV_Y, S_CONV_COLS, S_NTT_ROWS_FIN
 };
 struct Program {
     struct Step {
@@ -273,8 +274,9 @@ class Context : public std::enable_shared_from_this<Context> {
     // variant: the conversion kernel variant the program's ModUp conversion will run with (it
     // decides whether the inverse NTT leaves the y form, tuning key "conv_yform").
     void prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 variant) const;
-    void prog_apply(Program& p, const std::vector<ApplyTask>& tasks) const;
-    void prog_mod_down(Program& p, const std::vector<MdTask>& tasks) const;
+    // md_variant: the conversion kernel variant of mod_down.
+    void prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const;
+    void prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 md_variant) const;
     void prog_rescale(Program& p, const std::vector<RescaleTask>& tasks) const;
     void run(const Program& p, const uint8_t* d, hipStream_t s) const;
     void execute(const Program& p, hipStream_t s);
@@ -299,10 +301,11 @@ class Context : public std::enable_shared_from_this<Context> {
     // sums beat two modular products per source (step 19.98 -> 19.54 ms on the 256-switch
     // workload), while the ModUp conversions (50-bit sources) keep conv_variant.
     u32 conv_variant_md = 1;
+    u32 md_variant() const { return conv_variant_md < 3 ? conv_variant_md : conv_variant; }
     // Batched key switches of at most small_limbs input limbs in all (a single switch, a few
     // small ones) have too few workgroups per launch to fill the device; they run their own
     // schedule (tuning keys "small_limbs", "conv_variant_small", "conv_tg_small", "fuse_ip_small").
-    u32 small_limbs = 48, conv_variant_s = 2, conv_tg_s = 8, fuse_ip_s = 0;
+    u32 small_limbs = 48, conv_variant_s = 0, conv_tg_s = 8, fuse_ip_s = 0;
     std::string autotune();
     // The key-switch candidates of autotune() timed on a caller's batch (autotune.cpp).
     std::string autotune_ks(const std::vector<const Poly*>& ds, const Ksk& key);
@@ -350,6 +353,16 @@ class Context : public std::enable_shared_from_this<Context> {
     // Default 7 (every kind).
     u32 conv_yform = 7;
     bool yform_usable(u32 mask_bit) const;
+    // Base conversions fused with the column pass of their targets (k_conv_cols; tuning key
+    // "conv_cols"), where their sources come in y form, at most WRAP_SRC of them, and neither the
+    // matrix-core kernel nor the one-launch transforms are selected. Above CONV_COLS_ALWAYS sources
+    // only up to CONV_COLS_ITEMS tiles of targets (conv_cols.h has the measurements: the same time at
+    // 10,000 tiles, a launch less; 11 % slower at 150,000).
+    static constexpr u32 CONV_COLS_ALWAYS = 4, CONV_COLS_ITEMS = 8192;
+    u32 conv_cols = 1;
+    bool conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const;
+    // Appends the targets of one conversion (plan, first source limb, output polynomial).
+    void add_conv_cols(std::vector<ConvColRef>& refs, u32 plan, const u64* src, u64* out) const;
     std::atomic<u64> graph_captures{0}, graph_launches{0};
 
    private:
@@ -408,6 +421,8 @@ class Context : public std::enable_shared_from_this<Context> {
     std::vector<u32> modup_maxtgt_;            // [level]
     std::vector<u32> moddown_plan_;            // [level]
     std::vector<u32> conv_src_first_;          // [plan]: its first source in the ConvSrc table
+    std::vector<ConvPlan> conv_plans_;         // the plans, and whether every source of each is below 2^50
+    std::vector<u32> conv_small_;
     std::vector<u32> rescale_plan_;            // [level], level >= 1
     std::vector<u32> raise_plan_;              // [top], top >= 1: q_0 -> q_1..q_top
     std::vector<u64> pinv_, pinv_s_;           // P^-1 mod q_i

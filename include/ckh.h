@@ -97,10 +97,10 @@ ckh_status ckh_autotune_ks(ckh_context *ctx, uint32_t n, const ckh_poly *const *
 /* Forces one tuning value: "ntt_chunk_fwd", "ntt_chunk_inv" (limbs per launch, 0 = all);
  * "graphs" (1 = replay repeated launch sequences from captured hipGraphs, the default; 0 = launch
  * directly); "graph_cache" (captured sequences kept per context); "conv_variant" (base conversion:
- * 0 = vector kernel, 1 = vector kernel with exact f64-piece sums for 60-bit sources, 2 = int8
- * matrix-core kernel); "conv_variant_md" (the variant of mod_down's conversions in batched
+ * 0 or 1 = vector kernel, 2 = int8 matrix-core kernel); "conv_variant_md" (the variant of mod_down's conversions in batched
  * switches, default 1; 3 = conv_variant); "conv_tg" (targets per base-conversion
- * workgroup); "fuse_ip" (1 = row pass fused into the inner product); "fuse_fin" (1, the default:
+ * workgroup); "conv_cols" (1, the default: base conversions of few sources or few targets fused with
+ * their targets' column pass); "fuse_ip" (1 = row pass fused into the inner product); "fuse_fin" (1, the default:
  * with fuse_ip, mod_down's finish of the Q limbs in the same kernel, so the inner-product sums
  * never reach memory); "conv_yform" (a mask of the conversions whose inverse NTT ends with the
  * conversion's first product, [x + h] (Q/q_j)^-1, folded into its last stage: 1 = ModUp on the
