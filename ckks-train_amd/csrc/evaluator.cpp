@@ -338,7 +338,7 @@ static void run_ks_on(Context& c, const std::vector<KsReq>& reqs, hipStream_t s,
                       const std::vector<AutJob>* pre = nullptr) {
     u64 total = 0;
     for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true);
-    BufPtr scratch = c.alloc(total, s);
+    BufPtr scratch = c.alloc(total, s, (u32)reqs.size());
     c.execute(ks_program(c, reqs, scratch->ptr, pre), s);
     hip_check(hipGetLastError(), "key switch");
 }
@@ -683,66 +683,73 @@ void Evaluator::check_mul_operands(const Ct& a, const Ct& b) const {
     if (a.level() == 0) fail(CKH_ERR_NO_LEVELS_LEFT, "no levels left");
 }
 
-// Evaluator::mul_no_relin (evaluator.rs:422-438).
+// Evaluator::mul_no_relin (evaluator.rs:422-438): the three components in one launch.
 CtPtr Evaluator::mul_no_relin(const Ct& a, const Ct& b) {
     check_mul_operands(a, b);
-    auto& x = a.comps;
-    auto& y = b.comps;
-    PolyPtr d0 = poly_pointwise(ctx, PW_MUL, *x[0], y[0].get());
-    PolyPtr t0 = poly_pointwise(ctx, PW_MUL, *x[0], y[1].get());
-    PolyPtr t1 = poly_pointwise(ctx, PW_MUL, *x[1], y[0].get());
-    PolyPtr d1 = poly_pointwise(ctx, PW_ADD, *t0, t1.get());
-    PolyPtr d2 = poly_pointwise(ctx, PW_MUL, *x[1], y[1].get());
-    CtPtr r = make_ct({d0, d1, d2}, a.scale * b.scale);
+    const u32 level = a.level();
+    const u64 Lw = (u64)(level + 1) * ctx.n;
+    BufPtr out = ctx.alloc_polys(3 * Lw, 3);
+    ctx.tick_launch();
+    tensor_launch({a.comps[0]->data(), a.comps[1]->data(), b.comps[0]->data(), b.comps[1]->data()}, out->ptr, level + 1,
+                  ctx.d_pc, ctx.log_n, ctx.stream());
+    hip_check(hipGetLastError(), "tensor product");
+    CtPtr r = make_ct({view(out, 0, level, 0, true), view(out, Lw, level, 0, true), view(out, 2 * Lw, level, 0, true)},
+                      a.scale * b.scale);
     count(&ckh_op_counter::ct_ct_tensor);
     return r;
 }
 
-// mul_no_relin of several pairs in one launch: per output limb the product (two products summed
-// for the middle component) as a multiply-sum job; the same residues as mul_no_relin.
-std::vector<CtPtr> Evaluator::mul_no_relin_batch(const std::vector<std::pair<const Ct*, const Ct*>>& pairs) {
-    u64 total = 0;
-    for (const auto& pr : pairs) {
-        check_mul_operands(*pr.first, *pr.second);
-        total += 3 * (u64)(pr.first->level() + 1) * ctx.n;
-    }
+// Sums of tensor products in one launch: sum i of pairs[i] (each a 2-component product of one
+// level), the same residues as mul_no_relin and add. Operands checked by the caller.
+std::vector<CtPtr> Evaluator::tensor_sums(const std::vector<std::vector<std::pair<const Ct*, const Ct*>>>& sums) {
     std::vector<CtPtr> res;
-    if (pairs.empty()) return res;
-    BufPtr out = ctx.alloc(total);
-    std::vector<MulSumJob> jobs;
-    std::vector<MulSumTerm> terms;
+    if (sums.empty()) return res;
+    u64 total = 0, products = 0;
+    for (const auto& s : sums) {
+        total += 3 * (u64)(s[0].first->level() + 1) * ctx.n;
+        products += s.size();
+    }
+    BufPtr out = ctx.alloc_polys(total, 3 * sums.size());
+    std::vector<TensorJob> jobs;
+    std::vector<TensorTerm> terms;
     u64 off = 0;
-    for (const auto& pr : pairs) {
-        const u32 level = pr.first->level();
-        const u64 L = level + 1, n = ctx.n;
-        const auto& x = pr.first->comps;
-        const auto& y = pr.second->comps;
-        for (const Poly* q : {x[0].get(), x[1].get(), y[0].get(), y[1].get()}) use(ctx, *q);
-        u64* d0 = out->ptr + off;
-        u64* d1 = d0 + L * n;
-        u64* d2 = d1 + L * n;
-        for (u32 i = 0; i < L; ++i) {
-            const u64 o = (u64)i * n;
-            jobs.push_back({d0 + o, (u32)terms.size(), 1, i, 0});
-            terms.push_back({x[0]->data() + o, y[0]->data() + o});
-            jobs.push_back({d1 + o, (u32)terms.size(), 2, i, 0});
-            terms.push_back({x[0]->data() + o, y[1]->data() + o});
-            terms.push_back({x[1]->data() + o, y[0]->data() + o});
-            jobs.push_back({d2 + o, (u32)terms.size(), 1, i, 0});
-            terms.push_back({x[1]->data() + o, y[1]->data() + o});
+    for (const auto& s : sums) {
+        const u32 level = s[0].first->level();
+        const u64 Lw = (u64)(level + 1) * ctx.n;
+        for (const auto& pr : s)
+            for (const Ct* ct : {pr.first, pr.second})
+                for (const auto& q : ct->comps) use(ctx, *q);
+        for (u32 i = 0; i <= level; ++i) {
+            const u64 o = (u64)i * ctx.n;
+            u64* d = out->ptr + off + o;
+            jobs.push_back({d, d + Lw, d + 2 * Lw, (u32)terms.size(), (u32)s.size(), i, 0});
+            for (const auto& pr : s) {
+                const auto &x = pr.first->comps, &y = pr.second->comps;
+                terms.push_back({x[0]->data() + o, x[1]->data() + o, y[0]->data() + o, y[1]->data() + o});
+            }
         }
-        res.push_back(make_ct({view(out, off, level, 0, true), view(out, off + L * n, level, 0, true),
-                               view(out, off + 2 * L * n, level, 0, true)},
-                              pr.first->scale * pr.second->scale));
-        off += 3 * L * n;
+        res.push_back(make_ct({view(out, off, level, 0, true), view(out, off + Lw, level, 0, true),
+                               view(out, off + 2 * Lw, level, 0, true)},
+                              s[0].first->scale * s[0].second->scale));
+        off += 3 * Lw;
     }
     Program prog;
     const size_t oj = prog.add(jobs), ot = prog.add(terms);
-    prog.step(S_MUL_SUM, oj, (u32)jobs.size(), ot);
+    prog.step(S_TENSOR_SUM, oj, (u32)jobs.size(), ot);
     ctx.execute(prog, ctx.stream());
     hip_check(hipGetLastError(), "tensor products");
-    count(&ckh_op_counter::ct_ct_tensor, pairs.size());
+    count(&ckh_op_counter::ct_ct_tensor, products);
     return res;
+}
+
+// mul_no_relin of several pairs in one launch.
+std::vector<CtPtr> Evaluator::mul_no_relin_batch(const std::vector<std::pair<const Ct*, const Ct*>>& pairs) {
+    std::vector<std::vector<std::pair<const Ct*, const Ct*>>> sums;
+    for (const auto& pr : pairs) {
+        check_mul_operands(*pr.first, *pr.second);
+        sums.push_back({pr});
+    }
+    return tensor_sums(sums);
 }
 
 // Evaluator::relinearize (evaluator.rs:441-458): (c0 + kb, c1 + ka), the additions fused into
@@ -770,7 +777,7 @@ std::vector<CtPtr> Evaluator::relinearize_batch(const std::vector<const Ct*>& ct
     }
     std::vector<CtPtr> res;
     if (cts.empty()) return res;
-    BufPtr out = ctx.alloc(total);
+    BufPtr out = ctx.alloc_polys(total, 2 * cts.size());
     std::vector<KsReq> reqs;
     u64 off = 0;
     for (const Ct* ct : cts) {
@@ -864,16 +871,7 @@ CtPtr Evaluator::relabel(const Ct& ct, double scale) {
 
 // Evaluator::apply_galois (evaluator.rs:640-647) + finish_galois (800-804).
 CtPtr Evaluator::apply_galois(const Ct& ct, u64 elt) {
-    const Ksk& key = galois_key(elt, ct.level());
-    const u32 level = ct.level();
-    const u64 L = level + 1;
-    PolyPtr d = poly_automorphism(ctx, *ct.comps[1], elt);
-    PolyPtr r0 = poly_automorphism(ctx, *ct.comps[0], elt);
-    BufPtr out = ctx.alloc(2 * L * ctx.n);
-    run_ks(ctx, {{d.get(), &key, r0->data(), nullptr, out->ptr, out->ptr + L * ctx.n}});
-    CtPtr r = make_ct({view(out, 0, level, 0, true), view(out, L * ctx.n, level, 0, true)}, ct.scale);
-    count(&ckh_op_counter::rotations);
-    return r;
+    return apply_galois_batch({{&ct, elt, &galois_key(elt, ct.level())}})[0];
 }
 
 static void check_galois_input(const Ct& ct) {
@@ -929,8 +927,8 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
     BufPtr digs = ctx.alloc(nd * dw + L * n);
     ctx.decompose({{ct.comps[1]->data(), level, digs->ptr, digs->ptr + nd * dw}}, s);
     const u64 per = (2 * (L + k) + 2 * k + 2 * L + L) * n;  // acc, y, z, sigma(c0)
-    BufPtr scratch = ctx.alloc(per * nontrivial);
-    BufPtr out = ctx.alloc(2 * L * n * nontrivial);
+    BufPtr scratch = ctx.alloc_polys(per * nontrivial, nontrivial);
+    BufPtr out = ctx.alloc_polys(2 * L * n * nontrivial, 2 * nontrivial);
     std::vector<ApplyTask> tasks;
     std::vector<AutJob> aut;  // sigma_g(c0) of every step, in the same program
     u32 t = 0;
@@ -1049,42 +1047,54 @@ std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
 
 std::vector<CtPtr> Evaluator::rotate_batch(const std::vector<std::pair<const Ct*, int32_t>>& items) {
     std::vector<CtPtr> res(items.size());
-    std::vector<std::tuple<size_t, u64, const Ksk*>> todo;
+    std::vector<GaloisItem> todo;
+    std::vector<size_t> at;
     for (size_t i = 0; i < items.size(); ++i) {
         const Ct& ct = *items[i].first;
         check_basis(ct);
         check_galois_input(ct);
         const u64 e = rotation_elt(items[i].second);
-        if (e == 0)
+        if (e == 0) {
             res[i] = make_ct(ct.comps, ct.scale);
-        else
-            todo.push_back({i, e, &galois_key(e, ct.level())});
+        } else {
+            todo.push_back({&ct, e, &galois_key(e, ct.level())});
+            at.push_back(i);
+        }
     }
     if (todo.empty()) return res;
+    std::vector<CtPtr> out = apply_galois_batch(todo);
+    for (size_t i = 0; i < at.size(); ++i) res[at[i]] = out[i];
+    return res;
+}
+
+// Rotations or conjugations of checked ciphertexts in one program: sigma_g of both components of
+// every item in one launch, then their key switches, sigma_g(c0) added in the finish.
+std::vector<CtPtr> Evaluator::apply_galois_batch(const std::vector<GaloisItem>& items) {
+    std::vector<CtPtr> res;
     u64 total = 0;
-    for (auto& [i, e, k] : todo) total += 4 * (u64)(items[i].first->level() + 1) * ctx.n;
-    BufPtr buf = ctx.alloc(total);  // per item: sigma(c1), sigma(c0), kb + sigma(c0), ka
+    for (const GaloisItem& it : items) total += 4 * (u64)(it.ct->level() + 1) * ctx.n;
+    BufPtr buf = ctx.alloc_polys(total, 4 * items.size());  // per item: sigma(c1), sigma(c0), kb + sigma(c0), ka
     std::vector<KsReq> reqs;
     std::vector<Poly> dpolys;
-    dpolys.reserve(todo.size());
+    dpolys.reserve(items.size());
     u64 off = 0;
     std::vector<AutJob> aut;  // sigma_g of both components, in the switch's program
-    for (auto& [i, e, k] : todo) {
-        const Ct& ct = *items[i].first;
+    for (const GaloisItem& it : items) {
+        const Ct& ct = *it.ct;
         const u32 level = ct.level();
         const u64 Lw = (u64)(level + 1) * ctx.n;
         u64* d = buf->ptr + off;
         for (u32 li = 0; li <= level; ++li) {
-            aut.push_back({ct.comps[1]->data() + li * ctx.n, d + li * ctx.n, e});
-            aut.push_back({ct.comps[0]->data() + li * ctx.n, d + Lw + li * ctx.n, e});
+            aut.push_back({ct.comps[1]->data() + li * ctx.n, d + li * ctx.n, it.elt});
+            aut.push_back({ct.comps[0]->data() + li * ctx.n, d + Lw + li * ctx.n, it.elt});
         }
         dpolys.push_back(Poly{buf, off, level, 0, true});
-        reqs.push_back({&dpolys.back(), k, d + Lw, nullptr, d + 2 * Lw, d + 3 * Lw});
-        res[i] = make_ct({view(buf, off + 2 * Lw, level, 0, true), view(buf, off + 3 * Lw, level, 0, true)}, ct.scale);
+        reqs.push_back({&dpolys.back(), it.key, d + Lw, nullptr, d + 2 * Lw, d + 3 * Lw});
+        res.push_back(make_ct({view(buf, off + 2 * Lw, level, 0, true), view(buf, off + 3 * Lw, level, 0, true)}, ct.scale));
         off += 4 * Lw;
     }
     run_ks_on(ctx, reqs, ctx.stream(), &aut);
-    count(&ckh_op_counter::rotations, todo.size());
+    count(&ckh_op_counter::rotations, items.size());
     return res;
 }
 
@@ -1131,8 +1141,8 @@ CtPtr Evaluator::sum_cts(const std::vector<CtPtr>& cts) {
     }
     const u32 level = c0.level();
     const u64 L = level + 1, n = ctx.n, nc = c0.comps.size();
-    BufPtr out = ctx.alloc(nc * L * n);
-    std::vector<MulSumJob> jobs;
+    BufPtr out = ctx.alloc_polys(nc * L * n, nc);
+    std::vector<AddSumJob> jobs;
     std::vector<const u64*> xs;
     for (u64 comp = 0; comp < nc; ++comp)
         for (u32 i = 0; i < L; ++i) {
@@ -1198,18 +1208,19 @@ CtPtr Evaluator::plain_bsgs(const std::vector<BsgsTerm>& terms, const std::vecto
     std::vector<MulSumTerm> mterms;
     for (size_t b = 0; b < blocks.size(); ++b) {
         const u32 k1 = blocks[b];
-        for (u32 c = 0; c < 2; ++c)
-            for (u32 i = 0; i < L; ++i) {
-                MulSumJob J{out->ptr + ((2 * b + c) * L + i) * n, (u32)mterms.size(), 0, i, 0};
-                for (size_t t = 0; t < terms.size(); ++t)
-                    for (u32 k2 = 0; k2 < baby; ++k2) {
-                        const size_t e = (size_t)k1 * baby + k2;
-                        if (!terms[t].present[e]) continue;
-                        mterms.push_back({xs[t][k2]->comps[c]->data() + i * n, entries[t][e]->data() + i * n});
-                        ++J.count;
-                    }
-                jobs.push_back(J);
-            }
+        for (u32 i = 0; i < L; ++i) {
+            u64* o = out->ptr + (2 * b * L + i) * n;
+            MulSumJob J{o, o + L * n, (u32)mterms.size(), 0, i, 0};
+            for (size_t t = 0; t < terms.size(); ++t)
+                for (u32 k2 = 0; k2 < baby; ++k2) {
+                    const size_t e = (size_t)k1 * baby + k2;
+                    if (!terms[t].present[e]) continue;
+                    const auto& x = xs[t][k2]->comps;
+                    mterms.push_back({x[0]->data() + i * n, x[1]->data() + i * n, entries[t][e]->data() + i * n});
+                    ++J.count;
+                }
+            jobs.push_back(J);
+        }
     }
     Program prog;
     const size_t oj = prog.add(jobs), ot = prog.add(mterms);
@@ -1363,6 +1374,28 @@ std::vector<bool> Evaluator::check_matvec_enc(const Ct& x, const std::vector<con
 
 CtPtr Evaluator::matvec_enc_run(const Ct& x, const std::vector<const Ct*>& entries, u32 baby, u32 giant, u32 stride,
                                 int32_t offset, const std::vector<bool>& present) {
+    if (config.lazy_relin && config.bsgs) {
+        // Every block's products summed at degree 2 in one launch, the blocks relinearized in one
+        // program and rotated in another: the same words and counts as one call each.
+        const std::vector<CtPtr> xs = baby_rotations({{&x, present}}, baby, giant, stride)[0];
+        std::vector<std::vector<std::pair<const Ct*, const Ct*>>> sums;
+        std::vector<int32_t> shifts;
+        for (u32 k1 = 0; k1 < giant; ++k1) {
+            std::vector<std::pair<const Ct*, const Ct*>> s;
+            for (u32 k2 = 0; k2 < baby; ++k2)
+                if (present[k1 * baby + k2]) s.push_back({entries[k1 * baby + k2], xs[k2].get()});
+            if (s.empty()) continue;
+            sums.push_back(std::move(s));
+            shifts.push_back((offset + (int32_t)(baby * k1)) * (int32_t)stride);
+        }
+        const std::vector<CtPtr> deg2 = tensor_sums(sums);
+        std::vector<const Ct*> to_relin;
+        for (auto& c : deg2) to_relin.push_back(c.get());
+        const std::vector<CtPtr> blocks = relinearize_batch(to_relin);
+        std::vector<std::pair<const Ct*, int32_t>> to_rotate;
+        for (size_t i = 0; i < blocks.size(); ++i) to_rotate.push_back({blocks[i].get(), shifts[i]});
+        return sum_cts(rotate_batch(to_rotate));
+    }
     if (config.lazy_relin)
         return bsgs(
             {{&x, present}}, baby, giant, stride, offset,

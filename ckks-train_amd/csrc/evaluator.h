@@ -146,6 +146,14 @@ class Evaluator {
     const Ksk& galois_key(u64 elt, u32 level) const;
     u64 rotation_elt(int32_t steps) const;  // 0 for a multiple of the slot count
     CtPtr apply_galois(const Ct& ct, u64 elt);
+    // One rotation or conjugation of a checked 2-component ciphertext under its looked-up key.
+    struct GaloisItem {
+        const Ct* ct;
+        u64 elt;
+        const Ksk* key;
+    };
+    std::vector<CtPtr> apply_galois_batch(const std::vector<GaloisItem>& items);
+    std::vector<CtPtr> tensor_sums(const std::vector<std::vector<std::pair<const Ct*, const Ct*>>>& sums);
     void check_mod_raise_input(const Ct& ct) const;
     CtPtr raise_ct(const Ct& ct);
     std::vector<bool> check_matvec_enc(const Ct& x, const std::vector<const Ct*>& entries, u32 baby, u32 giant,

@@ -5,28 +5,47 @@
 
 namespace ckh {
 
-// One limb of a key-switch inner product: acc_b = sum_j dig_j * key_b_j, acc_a = sum_j dig_j *
-// key_a_j over ndig digits (digit j's limb at dig + j * dig_stride). The key limb of part j is
-// at key + (2 j) * key_poly (b) and key + (2 j + 1) * key_poly (a). galois != 0 reads the digit
-// through the NTT-form automorphism permutation (hoisted rotations). When own is set, digit
-// own_j's limb (the digit's own, unconverted limb) is read from own instead.
-// out (one limb, prime `prime`) <- sum over the job's terms [first, first + count) of x * w mod q:
-// the BSGS block sums of plaintext products in one launch (MulSumTerm: two limb pointers).
+// out0 / out1 (one limb each, prime `prime`) <- sum over the job's terms [first, first + count) of
+// x0 * w and x1 * w mod q: the BSGS block sums of plaintext products, both components, in one launch.
 struct MulSumJob {
-    u64* out;
+    u64* out0;
+    u64* out1;
     u32 first, count, prime, pad;
 };
 struct MulSumTerm {
-    const u64* x;
+    const u64* x0;
+    const u64* x1;
     const u64* w;
 };
 void mul_sum_launch(const MulSumJob* jobs, const MulSumTerm* terms, u32 njobs, const PrimeConst* pc, u32 log_n,
                     hipStream_t stream);
 
-// out (one limb, prime `prime`) <- sum of the limbs xs[first, first + count) mod q.
-void add_sum_launch(const MulSumJob* jobs, const u64* const* xs, u32 njobs, const PrimeConst* pc, u32 log_n,
-                    hipStream_t stream);
+// out0, out1, out2 (one limb each) <- sum over the job's terms of the tensor products x0 y0,
+// x0 y1 + x1 y0 and x1 y1 mod q.
+struct TensorJob {
+    u64* out0;
+    u64* out1;
+    u64* out2;
+    u32 first, count, prime, pad;
+};
+struct TensorTerm {
+    const u64* x0;
+    const u64* x1;
+    const u64* y0;
+    const u64* y1;
+};
+void tensor_sum_launch(const TensorJob* jobs, const TensorTerm* terms, u32 njobs, const PrimeConst* pc, u32 log_n,
+                       hipStream_t stream);
+// The tensor product of polynomials of `limbs` Q limbs to out (three of them, back to back).
+void tensor_launch(const TensorTerm& t, u64* out, u32 limbs, const PrimeConst* pc, u32 log_n, hipStream_t stream);
 
+// out (one limb, prime `prime`) <- sum of the limbs xs[first, first + count) mod q.
+struct AddSumJob {
+    u64* out;
+    u32 first, count, prime, pad;
+};
+void add_sum_launch(const AddSumJob* jobs, const u64* const* xs, u32 njobs, const PrimeConst* pc, u32 log_n,
+                    hipStream_t stream);
 
 void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n,
                           hipStream_t stream);

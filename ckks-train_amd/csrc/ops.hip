@@ -22,18 +22,25 @@ void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u3
     hipLaunchKernelGGL(k_inner_product, dim3((n + 255) / 256, njobs), dim3(256), 0, stream, jobs, pc, log_n);
 }
 
+// Elementwise kernels take two words of a limb per thread, in one 16-byte load each (limbs are
+// 16-byte aligned: a multiple of N >= 2 words from a block's start). Bound by memory: the sixteen
+// rotations' gathers at N = 2^16 51 -> 45 us, the block sums of the 32 x 32 product at 2^15 270 ->
+// 237 us (with each diagonal read once for both components).
+typedef u64 u64x2 __attribute__((ext_vector_type(2)));
+static dim3 pairs_grid(u32 log_n, u32 rows) { return dim3((((1u << log_n) / 2) + 255) / 256, rows); }
+CKH_DEV auto glb2(const u64* p) { return glb((const u64x2*)p); }
+CKH_DEV auto glb2(u64* p) { return glb((u64x2*)p); }
+
 __global__ __launch_bounds__(256) void k_copy(const LimbRef* __restrict__ refs, u32 log_n) {
-    const u32 n = 1u << log_n;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
+    if (c >= (1u << log_n) / 2) return;
     const LimbRef r = refs[blockIdx.y];
-    glb(r.dst)[c] = glb(r.src)[c];
+    glb2(r.dst)[c] = glb2(r.src)[c];
 }
 
 void copy_launch(const LimbRef* refs, u32 nrefs, u32 log_n, hipStream_t stream) {
     if (nrefs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_copy, dim3((n + 255) / 256, nrefs), dim3(256), 0, stream, refs, log_n);
+    hipLaunchKernelGGL(k_copy, pairs_grid(log_n, nrefs), dim3(256), 0, stream, refs, log_n);
 }
 
 // Streaming copy of n16 16-byte words (a measurement of the HBM copy rate a kernel reaches).
@@ -48,73 +55,217 @@ void stream_copy_launch(const void* in, void* out, u64 bytes, hipStream_t stream
     if (blocks) hipLaunchKernelGGL(k_stream_copy, dim3(blocks), dim3(256), 0, stream, (const uint4*)in, (uint4*)out, n16);
 }
 
+// a * b mod q for reduced a, b: one f64 modular product below 2^50 (about 12 operations instead of
+// the 128-bit reduction's 55).
+CKH_DEV u64 mul_any(u64 a, u64 b, const PrimeConst& C) {
+    if (C.q >= FP_PRIME_BOUND) return mul_mod(a, b, C);
+    const double w = u2d(b);
+    return d2u(fcanon(fmulmod(u2d(a), w, w * C.qinv, C.qf), C.qf, C.qinv));
+}
+
 __global__ __launch_bounds__(256) void k_pointwise(u32 op, const u64* __restrict__ a, const u64* __restrict__ b,
                                                    u64* __restrict__ out, u32 prime0,
                                                    const PrimeConst* __restrict__ pc, u32 log_n) {
-    const u32 n = 1u << log_n;
+    const u32 half = (1u << log_n) / 2;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
-    const u64 i = (u64)blockIdx.y * n + c;
+    if (c >= half) return;
+    const u64 i = (u64)blockIdx.y * half + c;
     const PrimeConst C = pc[prime0 + blockIdx.y];
-    u64 v;
-    switch (op) {
-        case PW_ADD: v = add_mod(a[i], b[i], C.q); break;
-        case PW_SUB: v = sub_mod(a[i], b[i], C.q); break;
-        case PW_NEG: v = sub_mod(0, a[i], C.q); break;
-        case PW_MUL: v = mul_mod(a[i], b[i], C); break;
-        default: v = a[i]; break;
-    }
-    out[i] = v;
+    const u64x2 x = glb2(a)[i];
+    u64x2 y = {0, 0}, v;
+    if (op == PW_ADD || op == PW_SUB || op == PW_MUL) y = glb2(b)[i];
+#pragma unroll
+    for (u32 k = 0; k < 2; ++k) switch (op) {
+            case PW_ADD: v[k] = add_mod(x[k], y[k], C.q); break;
+            case PW_SUB: v[k] = sub_mod(x[k], y[k], C.q); break;
+            case PW_NEG: v[k] = sub_mod(0, x[k], C.q); break;
+            case PW_MUL: v[k] = mul_any(x[k], y[k], C); break;
+            default: v[k] = x[k]; break;
+        }
+    glb2(out)[i] = v;
 }
 
 void pointwise_launch(PwOp op, const u64* a, const u64* b, u64* out, u32 limbs, u32 prime0, const PrimeConst* pc,
                       u32 log_n, hipStream_t stream) {
     if (limbs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_pointwise, dim3((n + 255) / 256, limbs), dim3(256), 0, stream, (u32)op, a, b, out, prime0,
-                       pc, log_n);
+    hipLaunchKernelGGL(k_pointwise, pairs_grid(log_n, limbs), dim3(256), 0, stream, (u32)op, a, b, out, prime0, pc,
+                       log_n);
+}
+
+// Sums of products of reduced words mod one prime, two words side by side: f64 modular products
+// below 2^50 (each below 0.7 q in magnitude; reduced before more than 6 could add up), exact 128-bit
+// sums above (folded into a residue before 128 terms).
+struct FpSum {
+    double s[2] = {0.0, 0.0};
+    CKH_DEV void add(u64x2 x, u64x2 w, const PrimeConst& C) {
+#pragma unroll
+        for (u32 k = 0; k < 2; ++k) {
+            const double wd = u2d(w[k]);
+            s[k] += fmulmod(u2d(x[k]), wd, wd * C.qinv, C.qf);
+        }
+    }
+    CKH_DEV void fold(const PrimeConst& C) {
+#pragma unroll
+        for (u32 k = 0; k < 2; ++k) s[k] = freduce(s[k], C.qf, C.qinv);
+    }
+    CKH_DEV u64x2 get(const PrimeConst& C) const {
+        return u64x2{d2u(fcanon(s[0], C.qf, C.qinv)), d2u(fcanon(s[1], C.qf, C.qinv))};
+    }
+    static constexpr u32 FOLD = 2;  // terms between folds: a tensor's middle component has two products each
+};
+struct IntSum {
+    Dot60 d[2];
+    u64 r[2] = {0, 0};
+    CKH_DEV void add(u64x2 x, u64x2 w, const PrimeConst&) {
+#pragma unroll
+        for (u32 k = 0; k < 2; ++k) d[k].add(x[k], w[k]);
+    }
+    CKH_DEV void fold(const PrimeConst& C) {
+#pragma unroll
+        for (u32 k = 0; k < 2; ++k) {
+            u64 hi, lo;
+            d[k].get(hi, lo);
+            r[k] = add_mod(r[k], reduce128(hi, lo, C), C.q);
+            d[k] = Dot60{};
+        }
+    }
+    CKH_DEV u64x2 get(const PrimeConst& C) {
+        fold(C);
+        return u64x2{r[0], r[1]};
+    }
+    static constexpr u32 FOLD = 64;
+};
+
+// sum of x_t w_t for both components of x: the diagonal's word is read once for the two.
+template <class S>
+CKH_DEV void mul_sum_words(const MulSumJob& J, const MulSumTerm* terms, const PrimeConst& C, u32 c) {
+    S a, b;
+    for (u32 t = 0; t < J.count; ++t) {
+        const auto* T = cst(terms + J.first + t);
+        const u64x2 w = glb2(T->w)[c];
+        a.add(glb2(T->x0)[c], w, C);
+        b.add(glb2(T->x1)[c], w, C);
+        if (t % S::FOLD == S::FOLD - 1) {
+            a.fold(C);
+            b.fold(C);
+        }
+    }
+    glb2(J.out0)[c] = a.get(C);
+    glb2(J.out1)[c] = b.get(C);
 }
 
 __global__ __launch_bounds__(256) void k_mul_sum(const MulSumJob* __restrict__ jobs,
                                                  const MulSumTerm* __restrict__ terms,
                                                  const PrimeConst* __restrict__ pc, u32 log_n) {
-    const u32 n = 1u << log_n;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
+    if (c >= (1u << log_n) / 2) return;
     const MulSumJob J = jobs[blockIdx.y];
     const PrimeConst C = pc[J.prime];
-    u64 acc = 0;
-    for (u32 t = 0; t < J.count; ++t) {
-        const MulSumTerm T = terms[J.first + t];
-        acc = add_mod(acc, mul_mod(glb(T.x)[c], glb(T.w)[c], C), C.q);
-    }
-    glb(J.out)[c] = acc;
+    if (C.q < FP_PRIME_BOUND)
+        mul_sum_words<FpSum>(J, terms, C, c);
+    else
+        mul_sum_words<IntSum>(J, terms, C, c);
 }
 
 void mul_sum_launch(const MulSumJob* jobs, const MulSumTerm* terms, u32 njobs, const PrimeConst* pc, u32 log_n,
                     hipStream_t stream) {
     if (njobs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_mul_sum, dim3((n + 255) / 256, njobs), dim3(256), 0, stream, jobs, terms, pc, log_n);
+    hipLaunchKernelGGL(k_mul_sum, pairs_grid(log_n, njobs), dim3(256), 0, stream, jobs, terms, pc, log_n);
 }
 
-__global__ __launch_bounds__(256) void k_add_sum(const MulSumJob* __restrict__ jobs, const u64* const* __restrict__ xs,
-                                                 const PrimeConst* __restrict__ pc, u32 log_n) {
-    const u32 n = 1u << log_n;
+// The tensor product (x0 + x1 s)(y0 + y1 s) of two words' pairs added to the three sums.
+template <class S>
+CKH_DEV void tensor_add(S& d0, S& d1, S& d2, u64x2 x0, u64x2 x1, u64x2 y0, u64x2 y1,
+                        const PrimeConst& C) {
+    d0.add(x0, y0, C);
+    d1.add(x0, y1, C);
+    d1.add(x1, y0, C);
+    d2.add(x1, y1, C);
+}
+
+template <class S>
+CKH_DEV void tensor_sum_words(const TensorJob& J, const TensorTerm* terms, const PrimeConst& C, u32 c) {
+    S d0, d1, d2;
+    for (u32 t = 0; t < J.count; ++t) {
+        const auto* T = cst(terms + J.first + t);
+        tensor_add(d0, d1, d2, glb2(T->x0)[c], glb2(T->x1)[c], glb2(T->y0)[c], glb2(T->y1)[c], C);
+        if (t % S::FOLD == S::FOLD - 1) {
+            d0.fold(C);
+            d1.fold(C);
+            d2.fold(C);
+        }
+    }
+    glb2(J.out0)[c] = d0.get(C);
+    glb2(J.out1)[c] = d1.get(C);
+    glb2(J.out2)[c] = d2.get(C);
+}
+
+__global__ __launch_bounds__(256) void k_tensor_sum(const TensorJob* __restrict__ jobs,
+                                                    const TensorTerm* __restrict__ terms,
+                                                    const PrimeConst* __restrict__ pc, u32 log_n) {
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
-    const MulSumJob J = jobs[blockIdx.y];
-    const u64 q = pc[J.prime].q;
-    u64 acc = 0;
-    for (u32 t = 0; t < J.count; ++t) acc = add_mod(acc, glb(xs[J.first + t])[c], q);
-    glb(J.out)[c] = acc;
+    if (c >= (1u << log_n) / 2) return;
+    const TensorJob J = jobs[blockIdx.y];
+    const PrimeConst C = pc[J.prime];
+    if (C.q < FP_PRIME_BOUND)
+        tensor_sum_words<FpSum>(J, terms, C, c);
+    else
+        tensor_sum_words<IntSum>(J, terms, C, c);
 }
 
-void add_sum_launch(const MulSumJob* jobs, const u64* const* xs, u32 njobs, const PrimeConst* pc, u32 log_n,
+void tensor_sum_launch(const TensorJob* jobs, const TensorTerm* terms, u32 njobs, const PrimeConst* pc, u32 log_n,
+                       hipStream_t stream) {
+    if (njobs == 0) return;
+    hipLaunchKernelGGL(k_tensor_sum, pairs_grid(log_n, njobs), dim3(256), 0, stream, jobs, terms, pc, log_n);
+}
+
+// One tensor product of whole polynomials, the pointers in the launch itself (no descriptors).
+template <class S>
+CKH_DEV void tensor_words(const TensorTerm& T, u64* out, u32 limbs, const PrimeConst& C, u64 i, u64 half) {
+    S d0, d1, d2;
+    tensor_add(d0, d1, d2, glb2(T.x0)[i], glb2(T.x1)[i], glb2(T.y0)[i], glb2(T.y1)[i], C);
+    const auto o = glb2(out);
+    o[i] = d0.get(C);
+    o[limbs * half + i] = d1.get(C);
+    o[2 * limbs * half + i] = d2.get(C);
+}
+
+__global__ __launch_bounds__(256) void k_tensor(TensorTerm T, u64* out, u32 limbs, const PrimeConst* __restrict__ pc,
+                                                u32 log_n) {
+    const u32 half = (1u << log_n) / 2;
+    const u32 c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= half) return;
+    const PrimeConst C = pc[blockIdx.y];
+    const u64 i = (u64)blockIdx.y * half + c;
+    if (C.q < FP_PRIME_BOUND)
+        tensor_words<FpSum>(T, out, limbs, C, i, half);
+    else
+        tensor_words<IntSum>(T, out, limbs, C, i, half);
+}
+
+void tensor_launch(const TensorTerm& t, u64* out, u32 limbs, const PrimeConst* pc, u32 log_n, hipStream_t stream) {
+    if (limbs == 0) return;
+    hipLaunchKernelGGL(k_tensor, pairs_grid(log_n, limbs), dim3(256), 0, stream, t, out, limbs, pc, log_n);
+}
+
+__global__ __launch_bounds__(256) void k_add_sum(const AddSumJob* __restrict__ jobs, const u64* const* __restrict__ xs,
+                                                 const PrimeConst* __restrict__ pc, u32 log_n) {
+    const u32 c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= (1u << log_n) / 2) return;
+    const AddSumJob J = jobs[blockIdx.y];
+    const u64 q = pc[J.prime].q;
+    u64x2 acc = {0, 0};
+    for (u32 t = 0; t < J.count; ++t) {
+        const u64x2 x = glb2(xs[J.first + t])[c];
+        acc = u64x2{add_mod(acc[0], x[0], q), add_mod(acc[1], x[1], q)};
+    }
+    glb2(J.out)[c] = acc;
+}
+
+void add_sum_launch(const AddSumJob* jobs, const u64* const* xs, u32 njobs, const PrimeConst* pc, u32 log_n,
                     hipStream_t stream) {
     if (njobs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_add_sum, dim3((n + 255) / 256, njobs), dim3(256), 0, stream, jobs, xs, pc, log_n);
+    hipLaunchKernelGGL(k_add_sum, pairs_grid(log_n, njobs), dim3(256), 0, stream, jobs, xs, pc, log_n);
 }
 
 __global__ __launch_bounds__(256) void k_scalar_mul(const u64* __restrict__ a, u64* __restrict__ out,
@@ -138,19 +289,26 @@ void scalar_mul_launch(const u64* a, u64* out, u32 limbs, const u64* consts, boo
                        log_n);
 }
 
+// Words 2 c and 2 c + 1 of sigma_g(in): the lowest index bit is the highest of the bit-reversed one,
+// where adding N (times the odd g) flips the highest bit of the result only, so perm(2 c + 1) =
+// perm(2 c) ^ 1 and a pair comes from a pair, as it is or exchanged.
+CKH_DEV u64x2 galois_pair(const u64* in, u32 c, u64 g, u32 log_n) {
+    const u32 s = galois_index(2 * c, g, log_n);
+    const u64x2 v = glb2(in)[s >> 1];
+    return (s & 1) ? u64x2{v[1], v[0]} : v;
+}
+
 __global__ __launch_bounds__(256) void k_automorphism_ntt(const u64* __restrict__ in, u64* __restrict__ out, u64 g,
                                                           u32 log_n) {
-    const u32 n = 1u << log_n;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
-    const u64 base = (u64)blockIdx.y * n;
-    out[base + c] = in[base + galois_index(c, g, log_n)];
+    if (c >= (1u << log_n) / 2) return;
+    const u64 base = (u64)blockIdx.y << log_n;
+    glb2(out + base)[c] = galois_pair(in + base, c, g, log_n);
 }
 
 void automorphism_ntt_launch(const u64* in, u64* out, u32 limbs, u64 g, u32 log_n, hipStream_t stream) {
     if (limbs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_automorphism_ntt, dim3((n + 255) / 256, limbs), dim3(256), 0, stream, in, out, g, log_n);
+    hipLaunchKernelGGL(k_automorphism_ntt, pairs_grid(log_n, limbs), dim3(256), 0, stream, in, out, g, log_n);
 }
 
 // Coefficient form (crates/ckks-train-core/src/poly.rs:255-276): coefficient i moves to
@@ -190,17 +348,15 @@ void automorphism_coeff_launch(const u64* in, u64* out, u32 limbs, u32 level, u3
 }
 
 __global__ __launch_bounds__(256) void k_automorphism_batch(const AutJob* __restrict__ jobs, u32 log_n) {
-    const u32 n = 1u << log_n;
     const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
+    if (c >= (1u << log_n) / 2) return;
     const AutJob J = jobs[blockIdx.y];
-    glb(J.out)[c] = glb(J.in)[galois_index(c, J.galois, log_n)];
+    glb2(J.out)[c] = galois_pair(J.in, c, J.galois, log_n);
 }
 
 void automorphism_batch_launch(const AutJob* jobs, u32 njobs, u32 log_n, hipStream_t stream) {
     if (njobs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_automorphism_batch, dim3((n + 255) / 256, njobs), dim3(256), 0, stream, jobs, log_n);
+    hipLaunchKernelGGL(k_automorphism_batch, pairs_grid(log_n, njobs), dim3(256), 0, stream, jobs, log_n);
 }
 
 // Stateless seeded generator: word (seed, stream, index) is uniform below q by rejection on

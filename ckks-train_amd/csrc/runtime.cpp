@@ -284,11 +284,16 @@ void Context::trim_pool(u64 keep_bytes) {
     hip_check(hipMemPoolTrimTo(dp, keep_bytes), "hipMemPoolTrimTo");
 }
 
-BufPtr Context::alloc(size_t words, hipStream_t s) {
+BufPtr Context::alloc(size_t words, hipStream_t s, u32 polys) {
     void* p = nullptr;
     size_t bytes = std::max<size_t>(words, 1) * sizeof(u64), cls = 0;
-    if (fail_alloc_after.load() >= 0 && fail_alloc_after.fetch_sub(1) == 0)
-        fail(CKH_ERR_DEVICE, "out of device memory (injected allocation failure)");
+    if (fail_alloc_after.load() >= 0) {
+        const int64_t left = fail_alloc_after.fetch_sub(polys);
+        if (left >= 0 && left < (int64_t)polys) {
+            fail_alloc_after = -1;
+            fail(CKH_ERR_DEVICE, "out of device memory (injected allocation failure)");
+        }
+    }
     hipError_t e;
     if (pool_mode == 1) {
         cls = size_class(bytes);
@@ -655,12 +660,17 @@ void Context::run(const Program& p, const uint8_t* d, hipStream_t s) const {
             case S_ROWS_IP_FIN: rows_ip_fin_launch(ntt, (const RowIpFinJob*)x, st.count, s); break;
             case S_ADD_SUM:
                 for (u32 i = 0; i < st.count; i += MAX_ROWS)
-                    add_sum_launch((const MulSumJob*)x + i, (const u64* const*)(d + st.off2), std::min(MAX_ROWS, st.count - i),
+                    add_sum_launch((const AddSumJob*)x + i, (const u64* const*)(d + st.off2), std::min(MAX_ROWS, st.count - i),
                                    d_pc, log_n, s);
                 break;
             case S_AUTOMORPH:
                 for (u32 i = 0; i < st.count; i += MAX_ROWS)
                     automorphism_batch_launch((const AutJob*)x + i, std::min(MAX_ROWS, st.count - i), log_n, s);
+                break;
+            case S_TENSOR_SUM:
+                for (u32 i = 0; i < st.count; i += MAX_ROWS)
+                    tensor_sum_launch((const TensorJob*)x + i, (const TensorTerm*)(d + st.off2),
+                                      std::min(MAX_ROWS, st.count - i), d_pc, log_n, s);
                 break;
             case S_MUL_SUM:
                 for (u32 i = 0; i < st.count; i += MAX_ROWS)

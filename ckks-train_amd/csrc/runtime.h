@@ -152,7 +152,8 @@ struct RaiseTask {
 // Descriptor bytes plus the launch steps that read them (see runtime.cpp, "engine").
 enum StepKind : uint8_t {
     S_NTT_FWD, S_NTT_INV, S_CONV, S_COPY, S_IP, S_NTT_FWD_FIN, S_FINISH, S_NTT_COLS, S_NTT_ROWS, S_ROWS_IP,
-    S_MUL_SUM, S_AUTOMORPH, S_ADD_SUM, S_ROWS_IP_FIN, S_NTT_INV_Y, S_CONV_COLS, S_NTT_ROWS_FIN
+    S_MUL_SUM, S_AUTOMORPH, S_ADD_SUM, S_ROWS_IP_FIN, S_NTT_INV_Y, S_CONV_COLS, S_NTT_ROWS_FIN,
+    S_TENSOR_SUM
 };
 struct Program {
     struct Step {
@@ -232,8 +233,10 @@ class Context : public std::enable_shared_from_this<Context> {
     // other stream once an event recorded after its last use has completed; 0 = the device's
     // default stream-ordered pool with the runtime's reuse rules (which may hand a block to
     // another stream before its free has run, behind a dependency the runtime inserts).
-    BufPtr alloc(size_t words, hipStream_t s);
+    // polys: the polynomials the buffer holds, for the allocation-failure hook.
+    BufPtr alloc(size_t words, hipStream_t s, u32 polys = 1);
     BufPtr alloc(size_t words) { return alloc(words, stream()); }
+    BufPtr alloc_polys(size_t words, u64 polys) { return alloc(words, stream(), (u32)polys); }
     void free_buffer(Buffer* b);
     u32 pool_mode = 1;
     // The pool's bytes in use, its release threshold (bytes kept reserved after a
@@ -244,7 +247,9 @@ class Context : public std::enable_shared_from_this<Context> {
     void set_pool_release_threshold(u64 bytes);
     void trim_pool(u64 keep_bytes);
     // Test hook (tuning key "fail_alloc_after"): the n-th allocation from now fails with a device
-    // error, as an out-of-memory would; negative = off.
+    // error, as an out-of-memory would; negative = off. A buffer of several polynomials counts as
+    // one allocation for each, so that a failure can be placed inside a composite operation whatever
+    // buffers it shares.
     std::atomic<int64_t> fail_alloc_after{-1};
     // Test hooks as the reference's failing backend (crates/ckks-train-cuda/tests/cases/
     // failing.rs:34-67): "fail_launch_after" makes the n-th primitive launch from now (a
