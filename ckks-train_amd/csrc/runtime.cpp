@@ -120,13 +120,14 @@ Context::~Context() {
     }
     plans_.clear();
     for (auto& pl : retired_) {  // every stream was synchronized above
-        (void)hipEventDestroy(pl->done);
+        if (pl->done) (void)hipEventDestroy(pl->done);
         if (pl->exec) (void)hipGraphExecDestroy(pl->exec);
     }
     retired_.clear();
     for (auto s : streams_) (void)hipStreamSynchronize(s);
     cache_release(0);
-    for (hipEvent_t e : cache_events_) (void)hipEventDestroy(e);
+    for (auto& m : marks_)
+        if (m.second.ev) (void)hipEventDestroy(m.second.ev);
     for (void* a : perm_allocs_) (void)hipFree(a);
     for (auto s : streams_) (void)hipStreamDestroy(s);
     if (capture_stream_) (void)hipStreamDestroy(capture_stream_);
@@ -158,28 +159,62 @@ static size_t size_class(size_t b) {
     return (c + 4095) & ~(size_t)4095;
 }
 
+// A mark covering every free queued on s so far.
+void Context::mark_record(Mark& m, hipStream_t s) {
+    if (!m.ev && hipEventCreateWithFlags(&m.ev, hipEventDisableTiming) != hipSuccess) {
+        (void)hipGetLastError();
+        m.ev = nullptr;
+        return;
+    }
+    if (hipEventRecord(m.ev, s) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    m.seq = m.freed;
+    m.pending = true;
+}
+
+// Whether the stream's seq-th free and the work before it have completed.
+bool Context::mark_covers(Mark& m, u64 seq) {
+    if (m.done >= seq) return true;
+    if (!m.pending || hipEventQuery(m.ev) != hipSuccess) return false;
+    m.done = m.seq;
+    m.pending = false;
+    return m.done >= seq;
+}
+
 // A cached block of class cls for stream s: one last used on s (stream order makes it free for
-// the work queued after), else one whose event has completed; null if none.
+// the work queued after), else one whose last use has completed; null if none.
 void* Context::cache_take(size_t& cls, hipStream_t s) {
     std::lock_guard<std::mutex> lk(cache_mu_);
+    if (!cache_stream_) cache_stream_ = s;
+    if (s != cache_stream_) cache_multi_ = true;
     // The class itself first, then larger classes up to twice its size (a fitting free block is
     // reused instead of growing the cache with another class); within a class, a block last used
-    // on s, else one whose event has completed.
+    // on s, else one whose last use is known to have completed.
+    std::vector<hipStream_t> wanted;  // streams whose blocks could not be taken yet
     for (auto it = cache_.lower_bound(cls); it != cache_.end() && it->first <= 2 * cls; ++it) {
         std::vector<Cached>& v = it->second;
         size_t pick = v.size();
         for (size_t i = 0; i < v.size() && pick == v.size(); ++i)
             if (v[i].s == s) pick = i;
-        for (size_t i = 0; i < v.size() && pick == v.size(); ++i)
-            if (hipEventQuery(v[i].ready) == hipSuccess) pick = i;
+        for (size_t i = 0; i < v.size() && pick == v.size(); ++i) {
+            if (mark_covers(marks_[v[i].s], v[i].seq))
+                pick = i;
+            else if (std::find(wanted.begin(), wanted.end(), v[i].s) == wanted.end())
+                wanted.push_back(v[i].s);
+        }
         if (pick == v.size()) continue;
         void* p = v[pick].p;
-        cache_events_.push_back(v[pick].ready);
         v[pick] = v.back();
         v.pop_back();
         cls = it->first;
         cache_bytes_ -= cls;
         return p;
+    }
+    for (hipStream_t w : wanted) {  // for the next request
+        Mark& m = marks_[w];
+        if (!m.pending) mark_record(m, w);
     }
     return nullptr;
 }
@@ -188,34 +223,30 @@ void* Context::cache_take(size_t& cls, hipStream_t s) {
 // driver once that use has finished).
 void Context::cache_put(void* p, size_t cls, hipStream_t s) {
     std::lock_guard<std::mutex> lk(cache_mu_);
-    hipEvent_t ev = nullptr;
-    if (!cache_events_.empty()) {
-        ev = cache_events_.back();
-        cache_events_.pop_back();
-    } else if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
-        (void)hipGetLastError();
-        ev = nullptr;
-    }
-    if (cache_bytes_ + cls > cache_limit_ || !ev || hipEventRecord(ev, s) != hipSuccess) {
-        (void)hipGetLastError();
-        if (ev) cache_events_.push_back(ev);
+    if (cache_bytes_ + cls > cache_limit_) {
         (void)hipStreamSynchronize(s);
         (void)hipFree(p);
         return;
     }
-    cache_[cls].push_back({p, s, ev});
+    Mark& m = marks_[s];
+    cache_[cls].push_back({p, s, ++m.freed});
     cache_bytes_ += cls;
+    if (cache_multi_ && m.freed % MARK_EVERY == 0 && (!m.pending || mark_covers(m, m.seq))) mark_record(m, s);
 }
 
 // Returns cached blocks to the driver, largest first, until at most keep_bytes stay cached.
 void Context::cache_release(u64 keep_bytes) {
     std::lock_guard<std::mutex> lk(cache_mu_);
+    std::vector<hipStream_t> waited;
     for (auto it = cache_.rbegin(); it != cache_.rend() && cache_bytes_ > keep_bytes; ++it) {
         std::vector<Cached>& v = it->second;
         while (!v.empty() && cache_bytes_ > keep_bytes) {
-            (void)hipEventSynchronize(v.back().ready);
-            (void)hipFree(v.back().p);
-            cache_events_.push_back(v.back().ready);
+            const Cached& b = v.back();
+            if (!mark_covers(marks_[b.s], b.seq) && std::find(waited.begin(), waited.end(), b.s) == waited.end()) {
+                (void)hipStreamSynchronize(b.s);
+                waited.push_back(b.s);
+            }
+            (void)hipFree(b.p);
             v.pop_back();
             cache_bytes_ -= it->first;
         }
@@ -382,13 +413,36 @@ BufPtr Context::upload_blob(const void* host, size_t bytes, hipStream_t s) {
     return b;
 }
 
-// A ring slot of len bytes: slots are handed out in address order, wrapping at the end; a slot
-// still read by an unfinished copy (the oldest busy slots, from the previous lap) is waited for.
+// One completion event per stream that copied from the open run; the run's slots are busy until all
+// of them have completed.
+void Context::ring_close_run() {
+    for (hipStream_t s : run_streams_) {
+        hipEvent_t ev;
+        if (ring_events_.empty()) {
+            hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
+        } else {
+            ev = ring_events_.back();
+            ring_events_.pop_back();
+        }
+        hip_check(hipEventRecord(ev, s), "event");
+        ring_busy_.push_back({run_off_, run_len_, ev});
+    }
+    run_streams_.clear();
+    run_len_ = 0;
+}
+
+// A ring slot of len bytes: slots are handed out in address order, wrapping at the end; a run
+// still read by an unfinished copy (the oldest busy runs, from the previous lap) is waited for.
 size_t Context::ring_reserve(size_t len) {
     len = (len + 255) & ~(size_t)255;
-    if (ring_head_ + len > ring_cap_) ring_head_ = 0;
+    if (ring_head_ + len > ring_cap_) {
+        ring_close_run();
+        ring_head_ = 0;
+    }
     const size_t off = ring_head_;
     ring_head_ += len;
+    if (run_streams_.empty()) run_off_ = off;
+    run_len_ = ring_head_ - run_off_;
     while (!ring_busy_.empty()) {
         Staged& b = ring_busy_.front();
         const bool overlaps = b.off < off + len && off < b.off + b.len;
@@ -397,7 +451,7 @@ size_t Context::ring_reserve(size_t len) {
         ring_events_.push_back(b.ev);
         ring_busy_.pop_front();
     }
-    for (const Staged& b : ring_busy_)  // a later busy slot can overlap only after a wrap
+    for (const Staged& b : ring_busy_)  // a later busy run can overlap only after a wrap
         if (b.off < off + len && off < b.off + b.len) hip_check(hipEventSynchronize(b.ev), "staging ring");
     return off;
 }
@@ -411,15 +465,8 @@ void Context::h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
         const size_t off = ring_reserve(len);
         std::memcpy(ring_ + off, (const uint8_t*)src + done, len);
         hip_check(hipMemcpyAsync((uint8_t*)dst + done, ring_ + off, len, hipMemcpyHostToDevice, s), "upload");
-        hipEvent_t ev;
-        if (ring_events_.empty()) {
-            hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
-        } else {
-            ev = ring_events_.back();
-            ring_events_.pop_back();
-        }
-        hip_check(hipEventRecord(ev, s), "event");
-        ring_busy_.push_back({off, len, ev});
+        if (std::find(run_streams_.begin(), run_streams_.end(), s) == run_streams_.end()) run_streams_.push_back(s);
+        if (run_len_ >= RING_RUN) ring_close_run();
         done += len;
     }
 }
@@ -684,7 +731,10 @@ void Context::run(const Program& p, const uint8_t* d, hipStream_t s) const {
 void Context::execute(const Program& p, hipStream_t s) {
     if (p.steps.empty()) return;
     tick_launch();
-    if (use_graphs && execute_graph(p, s)) return;
+    u32 launches = 0;
+    for (const Program::Step& st : p.steps)
+        launches += st.kind == S_NTT_FWD || st.kind == S_NTT_INV || st.kind == S_NTT_INV_Y || st.kind == S_NTT_FWD_FIN ? 2 : 1;
+    if (use_graphs && launches > DIRECT_LAUNCHES && execute_graph(p, s)) return;
     BufPtr d = upload_blob(p.bytes.data(), p.bytes.size(), s);
     run(p, (const uint8_t*)d->ptr, s);
 }
@@ -697,21 +747,21 @@ void Context::drop_plan(size_t i) {
     plans_.erase(plans_.begin() + i);
     if (pl->desc) (void)hipFreeAsync(pl->desc, pl->s);
     pl->desc = nullptr;
-    if (pl->done && hipEventQuery(pl->done) == hipErrorNotReady) {
-        retired_.push_back(std::move(pl));
-        return;
+    if (!pl->exec) return;
+    if (hipEventCreateWithFlags(&pl->done, hipEventDisableTiming) != hipSuccess || hipEventRecord(pl->done, pl->s) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(pl->s);
     }
-    if (pl->done) (void)hipEventDestroy(pl->done);
-    if (pl->exec) (void)hipGraphExecDestroy(pl->exec);
+    retired_.push_back(std::move(pl));
 }
 
 // Destroys the retired plans whose last replay has finished (wait: all of them, after it).
 void Context::sweep_retired(bool wait) {
     for (size_t i = 0; i < retired_.size();) {
         Plan& pl = *retired_[i];
-        if (wait) (void)hipEventSynchronize(pl.done);
-        if (wait || hipEventQuery(pl.done) != hipErrorNotReady) {
-            (void)hipEventDestroy(pl.done);
+        if (wait && pl.done) (void)hipEventSynchronize(pl.done);
+        if (wait || !pl.done || hipEventQuery(pl.done) != hipErrorNotReady) {
+            if (pl.done) (void)hipEventDestroy(pl.done);
             if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
             retired_.erase(retired_.begin() + i);
         } else {
@@ -781,8 +831,6 @@ bool Context::execute_graph(const Program& p, hipStream_t s) {
         ++graph_captures;
     }
     hip_check(hipGraphLaunch(pl->exec, s), "hipGraphLaunch");
-    if (!pl->done) hip_check(hipEventCreateWithFlags(&pl->done, hipEventDisableTiming), "event");
-    hip_check(hipEventRecord(pl->done, s), "event");
     ++graph_launches;
     return true;
 }

@@ -331,6 +331,9 @@ class Context : public std::enable_shared_from_this<Context> {
     // descriptor bytes copied into the plan's own device buffer before each replay. Tuning key
     // "graphs" (1 = on) and "graph_cache" (plans kept per context, least recently used evicted).
     u32 use_graphs = 1, graph_cache_max = 64;
+    // Programs of at most this many launches are launched directly: a graph launch takes about 20 us
+    // of the host whatever it holds, a kernel launch 2.4 us.
+    static constexpr u32 DIRECT_LAUNCHES = 6;
     // The one-launch NTTs (tuning key "ntt_fused", 1 = on where the device's XCD layout was
     // verified at creation, off by default: measured no faster than the two launches on the key
     // switch, slower on small launches; "fused_lag": slots between a limb's first- and
@@ -371,16 +374,23 @@ class Context : public std::enable_shared_from_this<Context> {
     std::atomic<u64> graph_captures{0}, graph_launches{0};
 
    private:
+    // The pinned staging ring of h2d. A completion event costs the device as much as a small kernel
+    // (about 4.5 us of its stream), so copies share one: the ring's open run collects copies until
+    // RING_RUN bytes, then takes one event per stream that copied from it.
     struct Staged {
         size_t off, len;
         hipEvent_t ev;
     };
+    static constexpr size_t RING_RUN = (size_t)1 << 20;
     std::mutex ring_mu_;
     uint8_t* ring_ = nullptr;  // pinned host memory
     size_t ring_cap_ = 0, ring_head_ = 0;
+    size_t run_off_ = 0, run_len_ = 0;      // the open run
+    std::vector<hipStream_t> run_streams_;  // streams with copies from it
     std::deque<Staged> ring_busy_;
     std::vector<hipEvent_t> ring_events_;
     size_t ring_reserve(size_t len);
+    void ring_close_run();
     struct Plan {
         hipStream_t s = nullptr;
         std::vector<Program::Step> steps;
@@ -388,7 +398,7 @@ class Context : public std::enable_shared_from_this<Context> {
         void* desc = nullptr;  // stream-ordered allocation on s, outside Buffer (which would keep the
                                // context alive)
         hipGraphExec_t exec = nullptr;
-        hipEvent_t done = nullptr;  // recorded after each replay
+        hipEvent_t done = nullptr;  // recorded when the plan is evicted, after its last replay
         u64 last_use = 0;
     };
     std::mutex plan_mu_;
@@ -405,17 +415,32 @@ class Context : public std::enable_shared_from_this<Context> {
     void clear_plans();
 
     std::vector<hipStream_t> streams_;  // caller streams, then the service streams
-    // The block cache of pool mode 1: free blocks per size class, each with the stream of its
-    // last use and an event recorded there after it.
+    // The block cache of pool mode 1: free blocks per size class, each with the stream of its last use
+    // and its number among the blocks freed on that stream. Another stream may take a block once a
+    // mark (an event recorded after its free) has completed; a mark covers every earlier free of its
+    // stream. Marks are recorded only when another stream asks, and every MARK_EVERY frees once a
+    // second stream has allocated: an event per free took about 4.5 us of the stream each.
     struct Cached {
         void* p;
         hipStream_t s;
-        hipEvent_t ready;
+        u64 seq;
     };
+    struct Mark {
+        hipEvent_t ev = nullptr;
+        u64 freed = 0;    // blocks freed on the stream so far
+        u64 seq = 0;      // the pending mark covers frees up to here
+        u64 done = 0;     // frees known complete
+        bool pending = false;
+    };
+    static constexpr u64 MARK_EVERY = 8;
     std::mutex cache_mu_;
     std::map<size_t, std::vector<Cached>> cache_;
-    std::vector<hipEvent_t> cache_events_;
+    std::map<hipStream_t, Mark> marks_;
+    hipStream_t cache_stream_ = nullptr;  // the first stream that allocated
+    bool cache_multi_ = false;            // a second one has
     u64 cache_bytes_ = 0, cache_limit_ = ~0ull;
+    void mark_record(Mark& m, hipStream_t s);
+    bool mark_covers(Mark& m, u64 seq);
     // A free block of class cls or of a larger class up to 2 cls (cls is set to the block's).
     void* cache_take(size_t& cls, hipStream_t s);
     void cache_put(void* p, size_t cls, hipStream_t s);
