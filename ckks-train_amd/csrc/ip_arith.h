@@ -40,58 +40,97 @@ CKH_DEV u32 galois_index(u32 i, u64 g, u32 log_n) {
 // loads of a group are in flight together.
 constexpr u32 IP_GROUP = 4;
 
-CKH_DEV void ip_coeff(const IpJob& J, const PrimeConst& C, u32 log_n, u32 c) {
-    const u32 cs = J.galois ? galois_index(c, J.galois, log_n) : c;
-    const auto key = glb(J.key);
-    u64 dv[IP_GROUP], bv[IP_GROUP], av[IP_GROUP];
+// How ip_words reads and writes W consecutive words from word W c of a limb: one at a time here; the
+// kernel's own takes two in one 16-byte access.
+struct IpWord {
+    static constexpr u32 W = 1;
+    CKH_DEV static void load(const u64* p, u64 c, u64 (&w)[1]) { w[0] = glb(p)[c]; }
+    CKH_DEV static void load_key(const u64* p, u64 c, u64 (&w)[1]) { w[0] = glb(p)[c]; }
+    CKH_DEV static void store(u64* p, u64 c, const u64 (&w)[1]) { glb(p)[c] = w[0]; }
+    // the words of a digit read through the Galois permutation
+    CKH_DEV static void gather(const u64* p, u64 c, u64 g, u32 log_n, u64 (&w)[1]) {
+        w[0] = glb(p)[galois_index((u32)c, g, log_n)];
+    }
+};
+
+template <class Mem>
+CKH_DEV void ip_words(const IpJob& J, const PrimeConst& C, u32 log_n, u32 c) {
+    constexpr u32 W = Mem::W;
+    u64 dv[IP_GROUP][W], bv[IP_GROUP][W], av[IP_GROUP][W];
     auto load_group = [&](u32 j0) {
 #pragma unroll
         for (u32 u = 0; u < IP_GROUP; ++u) {
             const u32 j = j0 + u;
             if (j < J.ndig) {
-                dv[u] = glb((J.own && j == J.own_j) ? J.own : J.dig + j * J.dig_stride)[cs];
-                bv[u] = key[(2 * j) * J.key_poly + c];
-                av[u] = key[(2 * j + 1) * J.key_poly + c];
+                const u64* d = (J.own && j == J.own_j) ? J.own : J.dig + j * J.dig_stride;
+                if (J.galois)
+                    Mem::gather(d, c, J.galois, log_n, dv[u]);
+                else
+                    Mem::load(d, c, dv[u]);
+                Mem::load_key(J.key + (2 * j) * J.key_poly, c, bv[u]);
+                Mem::load_key(J.key + (2 * j + 1) * J.key_poly, c, av[u]);
             }
         }
     };
+    u64 ob[W], oa[W];
     if (C.q < FP_PRIME_BOUND) {
         const double q = C.qf, qinv = C.qinv;
-        double sb = 0.0, sa = 0.0;
+        double sb[W], sa[W];
+#pragma unroll
+        for (u32 w = 0; w < W; ++w) sb[w] = sa[w] = 0.0;
         for (u32 j0 = 0; j0 < J.ndig; j0 += IP_GROUP) {
             load_group(j0);
 #pragma unroll
             for (u32 u = 0; u < IP_GROUP; ++u) {
                 if (j0 + u < J.ndig) {
-                    const double d = u2d(dv[u]), b = u2d(bv[u]), a = u2d(av[u]);
-                    sb += fmulmod(d, b, b * qinv, q);
-                    sa += fmulmod(d, a, a * qinv, q);
+#pragma unroll
+                    for (u32 w = 0; w < W; ++w) {
+                        const double d = u2d(dv[u][w]), b = u2d(bv[u][w]), a = u2d(av[u][w]);
+                        sb[w] += fmulmod(d, b, b * qinv, q);
+                        sa[w] += fmulmod(d, a, a * qinv, q);
+                    }
                 }
             }
             // four products (|.| < 0.7 q each) since the last reduction
-            sb = freduce(sb, q, qinv);
-            sa = freduce(sa, q, qinv);
-        }
-        glb(J.acc_b)[c] = d2u(fcanon(sb, q, qinv));
-        glb(J.acc_a)[c] = d2u(fcanon(sa, q, qinv));
-        return;
-    }
-    Dot60 sb, sa;
-    for (u32 j0 = 0; j0 < J.ndig; j0 += IP_GROUP) {
-        load_group(j0);
 #pragma unroll
-        for (u32 u = 0; u < IP_GROUP; ++u) {
-            if (j0 + u < J.ndig) {
-                sb.add(dv[u], bv[u]);
-                sa.add(dv[u], av[u]);
+            for (u32 w = 0; w < W; ++w) {
+                sb[w] = freduce(sb[w], q, qinv);
+                sa[w] = freduce(sa[w], q, qinv);
             }
         }
+#pragma unroll
+        for (u32 w = 0; w < W; ++w) {
+            ob[w] = d2u(fcanon(sb[w], q, qinv));
+            oa[w] = d2u(fcanon(sa[w], q, qinv));
+        }
+    } else {
+        Dot60 sb[W], sa[W];
+        for (u32 j0 = 0; j0 < J.ndig; j0 += IP_GROUP) {
+            load_group(j0);
+#pragma unroll
+            for (u32 u = 0; u < IP_GROUP; ++u) {
+                if (j0 + u < J.ndig) {
+#pragma unroll
+                    for (u32 w = 0; w < W; ++w) {
+                        sb[w].add(dv[u][w], bv[u][w]);
+                        sa[w].add(dv[u][w], av[u][w]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (u32 w = 0; w < W; ++w) {
+            u64 hi, lo;
+            sb[w].get(hi, lo);
+            ob[w] = reduce128(hi, lo, C);
+            sa[w].get(hi, lo);
+            oa[w] = reduce128(hi, lo, C);
+        }
     }
-    u64 hi, lo;
-    sb.get(hi, lo);
-    glb(J.acc_b)[c] = reduce128(hi, lo, C);
-    sa.get(hi, lo);
-    glb(J.acc_a)[c] = reduce128(hi, lo, C);
+    Mem::store(J.acc_b, c, ob);
+    Mem::store(J.acc_a, c, oa);
 }
+
+CKH_DEV void ip_coeff(const IpJob& J, const PrimeConst& C, u32 log_n, u32 c) { ip_words<IpWord>(J, C, log_n, c); }
 
 }  // namespace ckh

@@ -47,7 +47,8 @@ struct AddSumJob {
 void add_sum_launch(const AddSumJob* jobs, const u64* const* xs, u32 njobs, const PrimeConst* pc, u32 log_n,
                     hipStream_t stream);
 
-void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n,
+// keys_once: no two jobs of the launch read the same key limb.
+void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n, bool keys_once,
                           hipStream_t stream);
 
 // ref.dst <- ref.src (one limb per descriptor).

@@ -6,22 +6,6 @@
 
 namespace ckh {
 
-// The key inner product of one coefficient (ip_arith.h: ip_coeff) per thread.
-__global__ __launch_bounds__(256) void k_inner_product(const IpJob* __restrict__ jobs,
-                                                       const PrimeConst* __restrict__ pc, u32 log_n) {
-    const u32 n = 1u << log_n;
-    const u32 c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
-    const IpJob J = jobs[blockIdx.y];
-    ip_coeff(J, pc[J.prime], log_n, c);
-}
-
-void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n, hipStream_t stream) {
-    if (njobs == 0) return;
-    const u32 n = 1u << log_n;
-    hipLaunchKernelGGL(k_inner_product, dim3((n + 255) / 256, njobs), dim3(256), 0, stream, jobs, pc, log_n);
-}
-
 // Elementwise kernels take two words of a limb per thread, in one 16-byte load each (limbs are
 // 16-byte aligned: a multiple of N >= 2 words from a block's start). Bound by memory: the sixteen
 // rotations' gathers at N = 2^16 51 -> 45 us, the block sums of the 32 x 32 product at 2^15 270 ->
@@ -30,6 +14,64 @@ typedef u64 u64x2 __attribute__((ext_vector_type(2)));
 static dim3 pairs_grid(u32 log_n, u32 rows) { return dim3((((1u << log_n) / 2) + 255) / 256, rows); }
 CKH_DEV auto glb2(const u64* p) { return glb((const u64x2*)p); }
 CKH_DEV auto glb2(u64* p) { return glb((u64x2*)p); }
+
+// Words 2 c and 2 c + 1 of sigma_g(in): the lowest index bit is the highest of the bit-reversed one,
+// where adding N (times the odd g) flips the highest bit of the result only, so perm(2 c + 1) =
+// perm(2 c) ^ 1 and a pair comes from a pair, as it is or exchanged.
+CKH_DEV u64x2 galois_pair(const u64* in, u32 c, u64 g, u32 log_n) {
+    const u32 s = galois_index(2 * c, g, log_n);
+    const u64x2 v = glb2(in)[s >> 1];
+    return (s & 1) ? u64x2{v[1], v[0]} : v;
+}
+
+// The key inner product (ip_arith.h: ip_words), two coefficients per thread. NT_KEY: non-temporal key
+// loads, for launches whose every key word is read once (rotations, each under its own key): the
+// digits, which all of them read, then stay in the caches. Bound by memory: sixteen hoisted rotations
+// at N = 2^16 (19 limbs) 432 -> 381 us, 5.6 TB/s; 410 us without the non-temporal loads, which a key
+// shared by 256 switches does not want (1,041 against 892 us).
+template <bool NT_KEY>
+struct IpPair {
+    static constexpr u32 W = 2;
+    CKH_DEV static void put(u64x2 v, u64 (&w)[2]) {
+        w[0] = v[0];
+        w[1] = v[1];
+    }
+    CKH_DEV static void load(const u64* p, u64 c, u64 (&w)[2]) { put(glb2(p)[c], w); }
+    CKH_DEV static void load_key(const u64* p, u64 c, u64 (&w)[2]) {
+        if constexpr (NT_KEY)
+            put(__builtin_nontemporal_load(glb2(p) + c), w);
+        else
+            put(glb2(p)[c], w);
+    }
+    CKH_DEV static void store(u64* p, u64 c, const u64 (&w)[2]) { glb2(p)[c] = u64x2{w[0], w[1]}; }
+    CKH_DEV static void gather(const u64* p, u64 c, u64 g, u32 log_n, u64 (&w)[2]) { put(galois_pair(p, (u32)c, g, log_n), w); }
+};
+
+template <class Mem>
+__global__ __launch_bounds__(256) void k_inner_product(const IpJob* __restrict__ jobs,
+                                                       const PrimeConst* __restrict__ pc, u32 log_n) {
+    const u32 c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= (1u << log_n) / Mem::W) return;
+    const IpJob J = jobs[blockIdx.y];
+    ip_words<Mem>(J, pc[J.prime], log_n, c);
+}
+
+// Below IP_PAIR_BLOCKS workgroups of pairs (4 per CU) a thread takes one coefficient: a launch that
+// does not fill the device is bound by latency (one switch at N = 2^12 61.6 against 63.1 us).
+constexpr u64 IP_PAIR_BLOCKS = 1024;
+
+void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n, bool keys_once,
+                          hipStream_t stream) {
+    if (njobs == 0) return;
+    const dim3 pairs = pairs_grid(log_n, njobs);
+    if ((u64)pairs.x * pairs.y < IP_PAIR_BLOCKS)
+        hipLaunchKernelGGL(k_inner_product<IpWord>, dim3(((1u << log_n) + 255) / 256, njobs), dim3(256), 0, stream, jobs,
+                           pc, log_n);
+    else if (keys_once)
+        hipLaunchKernelGGL(k_inner_product<IpPair<true>>, pairs, dim3(256), 0, stream, jobs, pc, log_n);
+    else
+        hipLaunchKernelGGL(k_inner_product<IpPair<false>>, pairs, dim3(256), 0, stream, jobs, pc, log_n);
+}
 
 __global__ __launch_bounds__(256) void k_copy(const LimbRef* __restrict__ refs, u32 log_n) {
     const u32 c = blockIdx.x * 256 + threadIdx.x;
@@ -287,15 +329,6 @@ void scalar_mul_launch(const u64* a, u64* out, u32 limbs, const u64* consts, boo
     const u32 n = 1u << log_n;
     hipLaunchKernelGGL(k_scalar_mul, dim3((n + 255) / 256, limbs), dim3(256), 0, stream, a, out, consts, (u32)neg, pc,
                        log_n);
-}
-
-// Words 2 c and 2 c + 1 of sigma_g(in): the lowest index bit is the highest of the bit-reversed one,
-// where adding N (times the odd g) flips the highest bit of the result only, so perm(2 c + 1) =
-// perm(2 c) ^ 1 and a pair comes from a pair, as it is or exchanged.
-CKH_DEV u64x2 galois_pair(const u64* in, u32 c, u64 g, u32 log_n) {
-    const u32 s = galois_index(2 * c, g, log_n);
-    const u64x2 v = glb2(in)[s >> 1];
-    return (s & 1) ? u64x2{v[1], v[0]} : v;
 }
 
 __global__ __launch_bounds__(256) void k_automorphism_ntt(const u64* __restrict__ in, u64* __restrict__ out, u64 g,

@@ -641,8 +641,9 @@ static void launch_conv(const ConvTables& t, const ConvJob* d, u32 njobs, u32 ma
         conv_launch(t, d + i, std::min(MAX_ROWS, njobs - i), max_tgt, max_src, variant, tg, yform, s);
 }
 
-static void launch_ip(const IpJob* d, u32 njobs, const PrimeConst* pc, u32 log_n, hipStream_t s) {
-    for (u32 i = 0; i < njobs; i += MAX_ROWS) inner_product_launch(d + i, std::min(MAX_ROWS, njobs - i), pc, log_n, s);
+static void launch_ip(const IpJob* d, u32 njobs, const PrimeConst* pc, u32 log_n, bool keys_once, hipStream_t s) {
+    for (u32 i = 0; i < njobs; i += MAX_ROWS)
+        inner_product_launch(d + i, std::min(MAX_ROWS, njobs - i), pc, log_n, keys_once, s);
 }
 
 static void launch_finish(const FinishJob* d, u32 njobs, const PrimeConst* pc, u32 log_n, hipStream_t s) {
@@ -688,7 +689,7 @@ void Context::run(const Program& p, const uint8_t* d, hipStream_t s) const {
                             st.sched ? st.sched >> 8 : conv_tg, st.yform, s);
                 break;
             case S_COPY: launch_copy((const LimbRef*)x, st.count, log_n, s); break;
-            case S_IP: launch_ip((const IpJob*)x, st.count, d_pc, log_n, s); break;
+            case S_IP: launch_ip((const IpJob*)x, st.count, d_pc, log_n, st.a != 0, s); break;
             case S_NTT_FWD_FIN:
                 if (st.ctl && fused_usable())
                     ntt_fast_forward_fused(ntt, (const LimbRef*)x, st.count, (const FinishJob*)(d + st.off2),
@@ -931,7 +932,15 @@ void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 
 void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const {
     std::vector<IpJob> ip;
     u32 max_l = 0;
-    for (const ApplyTask& t : tasks) max_l = std::max(max_l, t.level + 1);
+    std::vector<const Ksk*> keys;
+    for (const ApplyTask& t : tasks) {
+        max_l = std::max(max_l, t.level + 1);
+        keys.push_back(t.key);
+    }
+    // Several tasks, each under a key of its own: the key words are read once. (A single switch may
+    // be followed by another under the same key, which a cached copy serves.)
+    std::sort(keys.begin(), keys.end());
+    const u32 keys_once = tasks.size() > 1 && std::adjacent_find(keys.begin(), keys.end()) == keys.end();
     // Inner-product rows ordered by key limb across tasks, so rows reading the same key limb
     // run back to back (the shared key is re-read from L2, not HBM).
     for (u32 k = 0; k < np; ++k)
@@ -947,7 +956,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
     if (all_fused && fuse_fin) {
         // The P limbs' inner product, mod_down of the P parts up to the column pass of the
         // converted limbs, then per Q limb one kernel: row pass + inner product + finish.
-        p.step(S_IP, p.add(ip), (u32)ip.size());
+        p.step(S_IP, p.add(ip), (u32)ip.size(), 0, keys_once);
         std::vector<LimbRef> intt, cols;
         std::vector<ConvJob> jobs;
         std::vector<ConvColRef> ccols;
@@ -1017,7 +1026,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
                           t.acc + i * n, t.acc + aw + i * n, t.galois, t.own ? t.own + i * n : nullptr,
                           ndigits(t.level), i, i / alpha, 0});
         }
-    p.step(S_IP, p.add(ip), (u32)ip.size());
+    p.step(S_IP, p.add(ip), (u32)ip.size(), 0, keys_once);
     p.step(S_ROWS_IP, p.add(rip), (u32)rip.size());
     std::vector<MdTask> md;
     for (const ApplyTask& t : tasks) {
