@@ -76,4 +76,11 @@ CKH_DEV u32 xcd_tile(u32 bid, u32 nblocks) {
     return (bid % nx) * (nblocks / nx) + bid / nx;
 }
 
+// A word of a column-pass output written by another workgroup of the same launch: loaded at agent
+// scope (the sc1 bit), so the load misses this CU's vector L1 (which may hold an older copy of the
+// line) and reads the XCD's L2, where the writer's completed stores are.
+CKH_DEV u64 load_coherent(const u64* p) {
+    return __hip_atomic_load(glb(const_cast<u64*>(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 }  // namespace ckh

@@ -33,15 +33,12 @@ CKH_DEV u32 conv_col_item(const ConvColRef& R, u32 item, u32 tiles, u32& tile) {
 template <u32 MAXS>
 constexpr u32 CONV_AHEAD = MAXS <= 2 ? 8 : MAXS <= 4 ? 4 : 2;
 
-// The tile's words of target g in the column pass's k-layout, as that pass takes them: f64 primes
-// signed below 2 q, integer primes below 4 q.
-template <u32 M, u32 MAXS, class Ar, class Tgt>
-CKH_DEV void conv_tile(const Ar& ar, const ConvSrc* srcs, const ConvColRef& R, const Tgt& g, const PrimeConst* pc,
-                       u32 log_n, u32 tile, u32 tid, typename Ar::V (&v)[16]) {
-    constexpr u32 R2 = M - 4, TCL = TL - M, TC = 1u << TCL, G = CONV_AHEAD<MAXS>;
-    const u32 B = log_n - M;
-    const u32 cc = tid & (TC - 1), o = tid >> TCL;
-    const u32 base = (o << B) + tile * TC + cc;
+// W words of target g, word k that of coefficient base + (k << shift), as a column pass takes them: f64
+// primes signed below 2 q, integer primes below 4 q.
+template <u32 W, u32 MAXS, class Ar, class Tgt>
+CKH_DEV void conv_words(const Ar& ar, const ConvSrc* srcs, const ConvColRef& R, const Tgt& g, const PrimeConst* pc,
+                        u32 log_n, u32 base, u32 shift, typename Ar::V (&v)[W]) {
+    constexpr u32 G = CONV_AHEAD<MAXS> < W ? CONV_AHEAD<MAXS> : W;
     // An absent source reads the first one; its constants are 0.
     u64 off[MAXS];
     double inv[MAXS];
@@ -53,12 +50,12 @@ CKH_DEV void conv_tile(const Ar& ar, const ConvSrc* srcs, const ConvColRef& R, c
     const bool exact = R.nsrc > 1;
     auto words = [&](auto&& load_y, auto&& convert) {
 #pragma unroll
-        for (u32 k0 = 0; k0 < 16; k0 += G) {
+        for (u32 k0 = 0; k0 < W; k0 += G) {
             u64 x[G][MAXS];
 #pragma unroll
             for (u32 w = 0; w < G; ++w)
 #pragma unroll
-                for (u32 j = 0; j < MAXS; ++j) x[w][j] = glb(R.in + off[j])[base + ((k0 + w) << (R2 + B))];
+                for (u32 j = 0; j < MAXS; ++j) x[w][j] = glb(R.in + off[j])[base + ((k0 + w) << shift)];
 #pragma unroll
             for (u32 w = 0; w < G; ++w) {
                 double yd[MAXS], f = 0.0;
@@ -90,6 +87,15 @@ CKH_DEV void conv_tile(const Ar& ar, const ConvSrc* srcs, const ConvColRef& R, c
         words([](u64 x) { return u64_to_f64_rn(x); },
               [&](u64 (&y)[MAXS], double (&)[MAXS], u32 e) { return ar.from_canon(conv_dot60<MAXS>(g, C, y, e, exact)); });
     }
+}
+
+// The words of a tile in the column pass's k-layout.
+template <u32 M, u32 MAXS, class Ar, class Tgt>
+CKH_DEV void conv_tile(const Ar& ar, const ConvSrc* srcs, const ConvColRef& R, const Tgt& g, const PrimeConst* pc,
+                       u32 log_n, u32 tile, u32 tid, typename Ar::V (&v)[16]) {
+    constexpr u32 R2 = M - 4, TCL = TL - M, TC = 1u << TCL;
+    const u32 B = log_n - M;
+    conv_words<16, MAXS>(ar, srcs, R, g, pc, log_n, ((tid >> TCL) << B) + tile * TC + (tid & (TC - 1)), R2 + B, v);
 }
 
 }  // namespace fast

@@ -76,6 +76,34 @@ struct ConvColRef;
 void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
                       hipStream_t stream);
 
+// The narrow passes (ntt_narrow.hip), for launches of few tiles: each pass of the transforms, the fused
+// conversion, the inner product + inverse transform in y form (jobs: njobs limbs, both parts each; refs:
+// the 2 njobs limbs whose inverse column pass follows, in place) and the row pass + inner product + finish.
+//
+// Where the line lies, in 4096-word tiles of a launch: the row passes and, up to N = 2^14, the column
+// passes are faster narrow up to some thousand tiles (64 switches at 2^12: 134 against 146 us, 24 at 2^14:
+// 199 against 218, four at 2^16: 494 against 509; sixteen hoisted rotations at 2^16 1102 against 1147 us
+// with every row pass narrow, whose finish takes 279 us narrow and 227 wide at 9728 tiles). A narrow
+// column tile of 2^8 rows is 4 columns, half of each 64-byte sector, so above 2^14 the column passes
+// change over once the chip is full: at 640 tiles instead of 320 a 24-limb switch takes 196 against 187
+// us, at 256 an 8-limb one 96 against 91.
+constexpr u32 NARROW_TILES = 4096, NARROW_COL8_TILES = 320;
+inline bool narrow_rows(u32 log_n, u32 nrefs) { return ((u64)nrefs << (log_n - 12)) <= NARROW_TILES; }
+inline bool narrow_cols(u32 log_n, u32 nrefs) {
+    return ((u64)nrefs << (log_n - 12)) <= (log_n > 14 ? NARROW_COL8_TILES : NARROW_TILES);
+}
+struct IpInvJob;
+struct IpFinJob;
+void narrow_forward_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t stream);
+void narrow_forward_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, const FinishJob* fin, hipStream_t stream);
+void narrow_inverse_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t stream);
+void narrow_inverse_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, const YForm* yf, hipStream_t stream);
+void narrow_conv_cols(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
+                      hipStream_t stream);
+void narrow_ip_inverse(const NttTables& t, const IpInvJob* jobs, const LimbRef* refs, u32 njobs, const YForm* yf,
+                       hipStream_t stream);
+void narrow_ip_finish(const NttTables& t, const IpFinJob* jobs, u32 njobs, hipStream_t stream);
+
 void rows_ip_launch(const NttTables& t, const RowIpJob* jobs, u32 njobs, hipStream_t stream);
 
 void rows_ip_fin_launch(const NttTables& t, const RowIpFinJob* jobs, u32 njobs, hipStream_t stream);

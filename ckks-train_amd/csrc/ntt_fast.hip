@@ -8,19 +8,6 @@
 #include "common.h"
 #include "ntt.h"
 
-namespace ckh {
-namespace fast {
-
-// A word of a column-pass output written by another workgroup of the same launch: loaded at agent
-// scope (the sc1 bit), so the load misses this CU's vector L1 (which may hold an older copy of the
-// line) and reads the XCD's L2, where the writer's completed stores are.
-CKH_DEV u64 load_coherent(const u64* p) {
-    return __hip_atomic_load(glb(const_cast<u64*>(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-}  // namespace fast
-}  // namespace ckh
-
 #include "ntt_passes.h"
 #include "conv_cols.h"
 
@@ -466,23 +453,23 @@ static void launch_m(u32 m, bool fwd, bool cols, const NttTables& t, const LimbR
 
 // Split N = 2^(A+B): B = floor(log N / 2) row stages, A column stages (6..8 each).
 void ntt_fast_forward(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
-    const u32 B = t.log_n / 2, A = t.log_n - B;
-    launch_m(A, true, true, t, refs, nrefs, s);
-    launch_m(B, true, false, t, refs, nrefs, s);
+    ntt_fast_forward_cols(t, refs, nrefs, s);
+    ntt_fast_forward_rows(t, refs, nrefs, s);
 }
 
 void ntt_fast_forward_finish(const NttTables& t, const LimbRef* refs, const FinishJob* fin, u32 nrefs,
                              hipStream_t s) {
-    const u32 B = t.log_n / 2, A = t.log_n - B;
-    launch_m(A, true, true, t, refs, nrefs, s);
-    launch_m(B, true, false, t, refs, nrefs, s, fin);
+    ntt_fast_forward_cols(t, refs, nrefs, s);
+    ntt_fast_forward_rows_finish(t, refs, fin, nrefs, s);
 }
 
 void ntt_fast_forward_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
+    if (narrow_cols(t.log_n, nrefs)) return narrow_forward_cols(t, refs, nrefs, s);
     launch_m(t.log_n - t.log_n / 2, true, true, t, refs, nrefs, s);
 }
 
 void ntt_fast_forward_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
+    if (narrow_rows(t.log_n, nrefs)) return narrow_forward_rows(t, refs, nrefs, nullptr, s);
     launch_m(t.log_n / 2, true, false, t, refs, nrefs, s);
 }
 
@@ -508,6 +495,7 @@ void rows_ip_launch(const NttTables& t, const RowIpJob* jobs, u32 njobs, hipStre
 
 void ntt_fast_forward_rows_finish(const NttTables& t, const LimbRef* refs, const FinishJob* fin, u32 nrefs,
                                   hipStream_t s) {
+    if (narrow_rows(t.log_n, nrefs)) return narrow_forward_rows(t, refs, nrefs, fin, s);
     launch_m(t.log_n / 2, true, false, t, refs, nrefs, s, fin);
 }
 
@@ -530,6 +518,7 @@ static void conv_cols_m(const ConvTables& c, const NttTables& t, const ConvColRe
 void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
                       hipStream_t s) {
     if (nrefs == 0) return;
+    if (narrow_cols(t.log_n, nrefs)) return narrow_conv_cols(c, t, refs, nrefs, max_src, s);
     const u32 items = nrefs << (t.log_n - fast::TL);
     switch (t.log_n - t.log_n / 2) {
         case 6: conv_cols_m<6>(c, t, refs, items, max_src, s); break;
@@ -539,9 +528,14 @@ void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef*
 }
 
 void ntt_fast_inverse(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s, const YForm* yf) {
-    const u32 B = t.log_n / 2, A = t.log_n - B;
-    launch_m(B, false, false, t, refs, nrefs, s);
-    launch_m(A, false, true, t, refs, nrefs, s, nullptr, yf);
+    if (narrow_rows(t.log_n, nrefs))
+        narrow_inverse_rows(t, refs, nrefs, s);
+    else
+        launch_m(t.log_n / 2, false, false, t, refs, nrefs, s);
+    if (narrow_cols(t.log_n, nrefs))
+        narrow_inverse_cols(t, refs, nrefs, yf, s);
+    else
+        launch_m(t.log_n - t.log_n / 2, false, true, t, refs, nrefs, s, nullptr, yf);
 }
 
 }  // namespace ckh

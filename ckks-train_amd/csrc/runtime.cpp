@@ -703,6 +703,10 @@ void Context::run(const Program& p, const uint8_t* d, hipStream_t s) const {
             case S_NTT_ROWS_FIN:
                 ntt_fast_forward_rows_finish(ntt, (const LimbRef*)x, (const FinishJob*)(d + st.off2), st.count, s);
                 break;
+            case S_IP_INV:
+                narrow_ip_inverse(ntt, (const IpInvJob*)x, (const LimbRef*)(d + st.off2), st.count, conv.yf, s);
+                break;
+            case S_IP_FIN: narrow_ip_finish(ntt, (const IpFinJob*)x, st.count, s); break;
             case S_CONV_COLS: conv_cols_launch(conv, ntt, (const ConvColRef*)x, st.count, st.a, s); break;
             case S_ROWS_IP: rows_ip_launch(ntt, (const RowIpJob*)x, st.count, s); break;
             case S_ROWS_IP_FIN: rows_ip_fin_launch(ntt, (const RowIpFinJob*)x, st.count, s); break;
@@ -734,7 +738,10 @@ void Context::execute(const Program& p, hipStream_t s) {
     tick_launch();
     u32 launches = 0;
     for (const Program::Step& st : p.steps)
-        launches += st.kind == S_NTT_FWD || st.kind == S_NTT_INV || st.kind == S_NTT_INV_Y || st.kind == S_NTT_FWD_FIN ? 2 : 1;
+        launches += st.kind == S_NTT_FWD || st.kind == S_NTT_INV || st.kind == S_NTT_INV_Y || st.kind == S_NTT_FWD_FIN ||
+                            st.kind == S_IP_INV
+                        ? 2
+                        : 1;
     if (use_graphs && launches > DIRECT_LAUNCHES && execute_graph(p, s)) return;
     BufPtr d = upload_blob(p.bytes.data(), p.bytes.size(), s);
     run(p, (const uint8_t*)d->ptr, s);
@@ -933,10 +940,17 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
     std::vector<IpJob> ip;
     u32 max_l = 0;
     std::vector<const Ksk*> keys;
+    u64 targets = 0;
+    bool any_fused = false;
     for (const ApplyTask& t : tasks) {
         max_l = std::max(max_l, t.level + 1);
         keys.push_back(t.key);
+        targets += 2 * (t.level + 1);
+        any_fused |= t.fused;
     }
+    if (!any_fused && targets << (log_n - 12) <= NARROW_IP_TILES && yform_usable(2) &&
+        conv_cols_usable(np, targets, md_variant))
+        return prog_apply_narrow(p, tasks);
     // Several tasks, each under a key of its own: the key words are read once. (A single switch may
     // be followed by another under the same key, which a cached copy serves.)
     std::sort(keys.begin(), keys.end());
@@ -1036,6 +1050,40 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
         md.push_back({t.acc + aw, t.level, t.out_a, t.add_a, t.y + (u64)np * n, t.z + (u64)L * n});
     }
     prog_mod_down(p, md, md_variant);
+}
+
+// The apply stage of a small program: the P limbs' inner product in their inverse transform, mod_down's
+// conversion in the column pass of its targets, the Q limbs' inner product in the row pass that finishes
+// them. The sums never go to memory, and the launch of their own is saved.
+void Context::prog_apply_narrow(Program& p, const std::vector<ApplyTask>& tasks) const {
+    std::vector<IpInvJob> inv;
+    std::vector<LimbRef> cols;
+    std::vector<ConvColRef> ccols;
+    std::vector<IpFinJob> fin;
+    for (const ApplyTask& t : tasks) {
+        const u32 L = t.level + 1, plan = moddown_plan_[t.level], sf = conv_src_first_[plan];
+        const u64 yw = (u64)np * n, zw = (u64)L * n;
+        auto limb_ip = [&](u32 limb, u32 key_limb, const u64* own) {
+            return LimbIp{t.dig + limb * n, digit_words(t.level), own, t.key->buf->ptr + key_limb * n,
+                          t.key->poly_words(), t.galois, ndigits(t.level), limb / alpha};
+        };
+        for (u32 k = 0; k < np; ++k) {
+            inv.push_back({limb_ip(L + k, t.key->max_level + 1 + k, nullptr), t.y + k * n, yw, nq + k, 0});
+            for (u32 part = 0; part < 2; ++part) {
+                u64* y = t.y + part * yw + k * n;
+                cols.push_back({y, y, nq + k, sf + k});
+            }
+        }
+        for (u32 part = 0; part < 2; ++part) add_conv_cols(ccols, plan, t.y + part * yw, t.z + part * zw);
+        for (u32 i = 0; i < L; ++i)
+            fin.push_back({limb_ip(i, i, t.own ? t.own + i * n : nullptr), t.z + i * n, zw, t.out_b + i * n, t.out_a + i * n,
+                           t.add_b ? t.add_b + i * n : nullptr, t.add_a ? t.add_a + i * n : nullptr, pinv_[i], pinv_s_[i],
+                           {(double)pinv_[i], (double)pinv_[i] / (double)primes[i]}, i, 0});
+    }
+    const size_t o_inv = p.add(inv);
+    p.step(S_IP_INV, o_inv, (u32)inv.size(), p.add(cols));
+    p.step(S_CONV_COLS, p.add(ccols), (u32)ccols.size(), 0, np);
+    p.step(S_IP_FIN, p.add(fin), (u32)fin.size());
 }
 
 // RnsPoly::mod_down (baseconv.rs:459-511) for a batch: INTT of the P limbs, the centered exact

@@ -17,6 +17,7 @@
 #include "common.h"
 #include "conv_col_ref.h"
 #include "lifetime.h"
+#include "narrow_jobs.h"
 #include "ntt.h"
 #include "ops.h"
 
@@ -153,7 +154,7 @@ struct RaiseTask {
 enum StepKind : uint8_t {
     S_NTT_FWD, S_NTT_INV, S_CONV, S_COPY, S_IP, S_NTT_FWD_FIN, S_FINISH, S_NTT_COLS, S_NTT_ROWS, S_ROWS_IP,
     S_MUL_SUM, S_AUTOMORPH, S_ADD_SUM, S_ROWS_IP_FIN, S_NTT_INV_Y, S_CONV_COLS, S_NTT_ROWS_FIN,
-    S_TENSOR_SUM
+    S_TENSOR_SUM, S_IP_INV, S_IP_FIN
 };
 struct Program {
     struct Step {
@@ -281,6 +282,7 @@ class Context : public std::enable_shared_from_this<Context> {
     void prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 variant) const;
     // md_variant: the conversion kernel variant of mod_down.
     void prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const;
+    void prog_apply_narrow(Program& p, const std::vector<ApplyTask>& tasks) const;
     void prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 md_variant) const;
     void prog_rescale(Program& p, const std::vector<RescaleTask>& tasks) const;
     void run(const Program& p, const uint8_t* d, hipStream_t s) const;
@@ -368,6 +370,12 @@ class Context : public std::enable_shared_from_this<Context> {
     // 10,000 tiles, a launch less; 11 % slower at 150,000).
     static constexpr u32 CONV_COLS_ALWAYS = 4, CONV_COLS_ITEMS = 8192;
     u32 conv_cols = 1;
+    // A key switch's apply stage of at most this many 4096-word tiles of Q limbs (both parts) runs its
+    // inner product inside the row passes (narrow_ip_inverse, narrow_ip_finish): one launch and the sums'
+    // way through memory less against reading the digits once per part. One switch of 6 limbs at 2^12 37.2
+    // against 38.0 us, of 20 at 2^15 115.7 against 121.3, of 18 at 2^16 (576 tiles) 151 against 155, of 24
+    // (768) the same; two of 24 (1536) 340 against 328 us.
+    static constexpr u32 NARROW_IP_TILES = 1024;
     bool conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const;
     // Appends the targets of one conversion (plan, first source limb, output polynomial).
     void add_conv_cols(std::vector<ConvColRef>& refs, u32 plan, const u64* src, u64* out) const;
