@@ -25,6 +25,15 @@ namespace fast {
 constexpr u32 LW = 2, NW = 1u << LW;             // words per thread
 constexpr u32 NTL = 8 + LW, NTILE = 1u << NTL;   // words per tile
 constexpr u32 NLDS = NTILE + NTILE / 16;
+// A column tile of 2^8 rows takes twice the threads: 8 columns are a whole 64-byte sector. Against 4
+// columns a switch of 13 limbs at N = 2^15 takes 73 against 80 us, of 12 limbs at 2^16 97 against 107;
+// 16 columns on 1024 threads: 74 and 92, but 47 against 41 us for one limb at 2^15.
+template <u32 M>
+constexpr u32 NCL = M == 8 ? NTL + 1 : NTL;  // log2 of a column tile's words
+template <u32 M>
+constexpr u32 NCT = 1u << (NCL<M> - LW);  // its threads
+template <u32 M>
+constexpr u32 NCLDS = (1u << NCL<M>) + (1u << NCL<M>) / 16;
 
 // The sub-transform of 2^M words: 2^(M - LW) threads o hold NW words each; in the layout of shift p
 // thread o's word k has index sub(o, k, p) (bits p .. p + LW - 1 vary over k).
@@ -143,7 +152,7 @@ CKH_DEV void narrow_inv(const Ar& ar, const NarrowTw<M, Ar>& t, typename Ar::V (
 // The place of a thread in a column tile (2^M rows of TC columns) or a row tile (rows of 2^M words).
 template <u32 M>
 struct NarrowCol {
-    static constexpr u32 TCL = NTL - M;
+    static constexpr u32 TCL = NCL<M> - M;
     u32 B, c, o;  // words per row (log2), the thread's column, its part of it
     CKH_DEV NarrowCol(u32 log_n, u32 tile, u32 tid)
         : B(log_n - M), c((tile << TCL) + (tid & ((1u << TCL) - 1))), o(tid >> TCL) {}

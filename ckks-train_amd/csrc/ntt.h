@@ -83,10 +83,10 @@ void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef*
 // Where the line lies, in 4096-word tiles of a launch: the row passes and, up to N = 2^14, the column
 // passes are faster narrow up to some thousand tiles (64 switches at 2^12: 134 against 146 us, 24 at 2^14:
 // 199 against 218, four at 2^16: 494 against 509; sixteen hoisted rotations at 2^16 1102 against 1147 us
-// with every row pass narrow, whose finish takes 279 us narrow and 227 wide at 9728 tiles). A narrow
-// column tile of 2^8 rows is 4 columns, half of each 64-byte sector, so above 2^14 the column passes
-// change over once the chip is full: at 640 tiles instead of 320 a 24-limb switch takes 196 against 187
-// us, at 256 an 8-limb one 96 against 91.
+// with every row pass narrow, whose finish takes 279 us narrow and 227 wide at 9728 tiles). Above 2^14
+// the column passes change over once the chip is full: 320 tiles against 640 or more, 134 against 140
+// us for an 18-limb switch at 2^16 and 183 against 184 for 24 limbs, against none the same switch of 8
+// limbs 85 against 98; all column passes narrow, a batch of 256 switches takes 19.5 against 16.4 ms.
 constexpr u32 NARROW_TILES = 4096, NARROW_COL8_TILES = 320;
 inline bool narrow_rows(u32 log_n, u32 nrefs) { return ((u64)nrefs << (log_n - 12)) <= NARROW_TILES; }
 inline bool narrow_cols(u32 log_n, u32 nrefs) {

@@ -1,4 +1,6 @@
 // The narrow passes (narrow_passes.h) as kernels over batches of limbs, for launches of few tiles.
+#include <type_traits>
+
 #include "basis.h"
 #include "common.h"
 #include "ntt.h"
@@ -34,10 +36,10 @@ CKH_DEV void set_yform(IntAr& ar, const YForm* yf) {
 }
 
 template <u32 M>
-__global__ __launch_bounds__(NT) void k_narrow_fwd_cols(NttTables T, const LimbRef* __restrict__ refs) {
-    __shared__ u64 lds[NLDS];
-    const u32 log_n = T.log_n, tile = blockIdx.x & ((1u << (log_n - NTL)) - 1);
-    const LimbRef ref = refs[blockIdx.x >> (log_n - NTL)];
+__global__ __launch_bounds__(NCT<M>) void k_narrow_fwd_cols(NttTables T, const LimbRef* __restrict__ refs) {
+    __shared__ u64 lds[NCLDS<M>];
+    const u32 log_n = T.log_n, tile = blockIdx.x & ((1u << (log_n - NCL<M>)) - 1);
+    const LimbRef ref = refs[blockIdx.x >> (log_n - NCL<M>)];
     const NarrowCol<M> P(log_n, tile, threadIdx.x);
     with_prime(T.pc, T.fwd, T.fwd_f, ref.prime, log_n, [&](const auto& ar) {
         const auto in = glb(ref.src);
@@ -50,14 +52,14 @@ __global__ __launch_bounds__(NT) void k_narrow_fwd_cols(NttTables T, const LimbR
 
 // Items and their order as in k_conv_cols, over this tile's size.
 template <u32 M, u32 MAXS>
-__global__ __launch_bounds__(NT) void k_narrow_conv_cols(ConvTables C, NttTables T, const ConvColRef* __restrict__ refs,
+__global__ __launch_bounds__(NCT<M>) void k_narrow_conv_cols(ConvTables C, NttTables T, const ConvColRef* __restrict__ refs,
                                                          u32 items) {
-    __shared__ u64 lds[NLDS];
+    __shared__ u64 lds[NCLDS<M>];
     const u32 log_n = T.log_n, item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
     if (item >= items) return;
-    const ConvColRef R = refs[item >> (log_n - NTL)];
+    const ConvColRef R = refs[item >> (log_n - NCL<M>)];
     u32 tile;
-    const u32 t = conv_col_item(R, item, 1u << (log_n - NTL), tile);
+    const u32 t = conv_col_item(R, item, 1u << (log_n - NCL<M>), tile);
     const auto* g = cst(C.tgt + R.tgt_first + t);
     const u32 prime = g->prime;
     const NarrowCol<M> P(log_n, tile, threadIdx.x);
@@ -98,11 +100,11 @@ __global__ __launch_bounds__(NT) void k_narrow_inv_rows(NttTables T, const LimbR
 }
 
 template <u32 M, bool YF>
-__global__ __launch_bounds__(NT) void k_narrow_inv_cols(NttTables T, const LimbRef* __restrict__ refs,
+__global__ __launch_bounds__(NCT<M>) void k_narrow_inv_cols(NttTables T, const LimbRef* __restrict__ refs,
                                                         const YForm* __restrict__ yf) {
-    __shared__ u64 lds[NLDS];
-    const u32 log_n = T.log_n, tile = blockIdx.x & ((1u << (log_n - NTL)) - 1);
-    const LimbRef ref = refs[blockIdx.x >> (log_n - NTL)];
+    __shared__ u64 lds[NCLDS<M>];
+    const u32 log_n = T.log_n, tile = blockIdx.x & ((1u << (log_n - NCL<M>)) - 1);
+    const LimbRef ref = refs[blockIdx.x >> (log_n - NCL<M>)];
     with_prime(T.pc, T.inv, T.inv_f, ref.prime, log_n, [&](auto ar) {
         if constexpr (YF) set_yform(ar, yf + ref.aux);
         narrow_inv_cols<M, YF>(ar, ref.dst, (u64*)lds, log_n, tile, threadIdx.x);
@@ -133,50 +135,62 @@ __global__ __launch_bounds__(NT) void k_narrow_ip_fin(NttTables T, const IpFinJo
 
 }  // namespace fast
 
-#define CKH_NARROW(M_, KERNEL, ITEMS, ...)                                                                       \
-    do {                                                                                                         \
-        const dim3 grid((u32)(ITEMS)), block(fast::NT);                                                          \
-        switch (M_) {                                                                                            \
-            case 6: { constexpr u32 M = 6; hipLaunchKernelGGL((KERNEL), grid, block, 0, s, __VA_ARGS__); break; }  \
-            case 7: { constexpr u32 M = 7; hipLaunchKernelGGL((KERNEL), grid, block, 0, s, __VA_ARGS__); break; }  \
-            default: { constexpr u32 M = 8; hipLaunchKernelGGL((KERNEL), grid, block, 0, s, __VA_ARGS__); break; } \
-        }                                                                                                        \
-    } while (0)
-
-static u32 tiles_of(const NttTables& t, u32 limbs) { return limbs << (t.log_n - fast::NTL); }
-static u32 row_stages(const NttTables& t) { return t.log_n / 2; }
-static u32 col_stages(const NttTables& t) { return t.log_n - t.log_n / 2; }
+// f with the number of stages of a row or column pass as a compile-time constant.
+template <class F>
+static void with_stages(u32 m, F f) {
+    if (m == 6)
+        f(std::integral_constant<u32, 6>{});
+    else if (m == 7)
+        f(std::integral_constant<u32, 7>{});
+    else
+        f(std::integral_constant<u32, 8>{});
+}
+// Row passes: KERNEL over the tiles of `limbs` limbs.
+#define CKH_NARROW_ROWS(LIMBS, KERNEL, ...)                                                              \
+    with_stages(t.log_n / 2, [&](auto m) {                                                               \
+        constexpr u32 M = m.value;                                                                       \
+        hipLaunchKernelGGL((KERNEL), dim3((LIMBS) << (t.log_n - fast::NTL)), dim3(fast::NT), 0, s, __VA_ARGS__); \
+    })
+#define CKH_NARROW_COLS(LIMBS, KERNEL, ...)                                                              \
+    with_stages(t.log_n - t.log_n / 2, [&](auto m) {                                                     \
+        constexpr u32 M = m.value;                                                                       \
+        hipLaunchKernelGGL((KERNEL), dim3((LIMBS) << (t.log_n - fast::NCL<M>)), dim3(fast::NCT<M>), 0, s, __VA_ARGS__); \
+    })
 
 void narrow_forward_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
     if (nrefs == 0) return;
-    CKH_NARROW(col_stages(t), fast::k_narrow_fwd_cols<M>, tiles_of(t, nrefs), t, refs);
+    CKH_NARROW_COLS(nrefs, fast::k_narrow_fwd_cols<M>, t, refs);
 }
 
 void narrow_forward_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, const FinishJob* fin, hipStream_t s) {
     if (nrefs == 0) return;
     if (fin)
-        CKH_NARROW(row_stages(t), (fast::k_narrow_fwd_rows<M, true>), tiles_of(t, nrefs), t, refs, fin);
+        CKH_NARROW_ROWS(nrefs, (fast::k_narrow_fwd_rows<M, true>), t, refs, fin);
     else
-        CKH_NARROW(row_stages(t), (fast::k_narrow_fwd_rows<M, false>), tiles_of(t, nrefs), t, refs, fin);
+        CKH_NARROW_ROWS(nrefs, (fast::k_narrow_fwd_rows<M, false>), t, refs, fin);
 }
 
 void narrow_inverse_rows(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
     if (nrefs == 0) return;
-    CKH_NARROW(row_stages(t), fast::k_narrow_inv_rows<M>, tiles_of(t, nrefs), t, refs);
+    CKH_NARROW_ROWS(nrefs, fast::k_narrow_inv_rows<M>, t, refs);
 }
 
 void narrow_inverse_cols(const NttTables& t, const LimbRef* refs, u32 nrefs, const YForm* yf, hipStream_t s) {
     if (nrefs == 0) return;
     if (yf)
-        CKH_NARROW(col_stages(t), (fast::k_narrow_inv_cols<M, true>), tiles_of(t, nrefs), t, refs, yf);
+        CKH_NARROW_COLS(nrefs, (fast::k_narrow_inv_cols<M, true>), t, refs, yf);
     else
-        CKH_NARROW(col_stages(t), (fast::k_narrow_inv_cols<M, false>), tiles_of(t, nrefs), t, refs, yf);
+        CKH_NARROW_COLS(nrefs, (fast::k_narrow_inv_cols<M, false>), t, refs, yf);
 }
 
 template <u32 MAXS>
 static void conv_cols_s(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, hipStream_t s) {
-    const u32 items = tiles_of(t, nrefs);
-    CKH_NARROW(col_stages(t), (fast::k_narrow_conv_cols<M, MAXS>), (items + 7) / 8 * 8, c, t, refs, items);
+    with_stages(t.log_n - t.log_n / 2, [&](auto m) {
+        constexpr u32 M = m.value;
+        const u32 items = nrefs << (t.log_n - fast::NCL<M>);
+        hipLaunchKernelGGL((fast::k_narrow_conv_cols<M, MAXS>), dim3((items + 7) / 8 * 8), dim3(fast::NCT<M>), 0, s, c, t, refs,
+                           items);
+    });
 }
 
 void narrow_conv_cols(const ConvTables& c, const NttTables& t, const ConvColRef* refs, u32 nrefs, u32 max_src,
@@ -197,13 +211,13 @@ void narrow_conv_cols(const ConvTables& c, const NttTables& t, const ConvColRef*
 void narrow_ip_inverse(const NttTables& t, const IpInvJob* jobs, const LimbRef* refs, u32 njobs, const YForm* yf,
                        hipStream_t s) {
     if (njobs == 0) return;
-    CKH_NARROW(row_stages(t), fast::k_narrow_ip_inv_rows<M>, tiles_of(t, 2 * njobs), t, jobs);
+    CKH_NARROW_ROWS(2 * njobs, fast::k_narrow_ip_inv_rows<M>, t, jobs);
     narrow_inverse_cols(t, refs, 2 * njobs, yf, s);
 }
 
 void narrow_ip_finish(const NttTables& t, const IpFinJob* jobs, u32 njobs, hipStream_t s) {
     if (njobs == 0) return;
-    CKH_NARROW(row_stages(t), fast::k_narrow_ip_fin<M>, tiles_of(t, 2 * njobs), t, jobs);
+    CKH_NARROW_ROWS(2 * njobs, fast::k_narrow_ip_fin<M>, t, jobs);
 }
 
 }  // namespace ckh

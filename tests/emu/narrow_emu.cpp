@@ -73,13 +73,13 @@ struct OwnView {
 };
 
 template <class F>
-void run_group(OwnLds& lds, F f) {
+void run_group(OwnLds& lds, u32 threads, F f) {
     auto done = [&]() noexcept { lds.end_phase(); };
-    std::barrier bar(NT, done);
+    std::barrier bar(threads, done);
     emu::Group g{nullptr, [&bar] { bar.arrive_and_wait(); }};
     emu::current() = &g;
     std::vector<std::thread> th;
-    for (u32 t = 0; t < NT; ++t)
+    for (u32 t = 0; t < threads; ++t)
         th.emplace_back([&f, t] {
             threadIdx.x = t;
             f(t);
@@ -98,11 +98,11 @@ std::vector<u64> primes_of(unsigned bits, u64 count) {
 template <u32 LOGN>
 struct Replay {
     static constexpr u64 n = 1ull << LOGN;
-    static constexpr u32 B = LOGN / 2, A = LOGN - B, TILES = 1u << (LOGN - NTL);
+    static constexpr u32 B = LOGN / 2, A = LOGN - B, TILES = 1u << (LOGN - NTL), CTILES = 1u << (LOGN - NCL<A>);
     std::vector<u64> primes;
     HostNttTables nt;
     std::mt19937_64 rng{4711};
-    OwnLds lds{NLDS};
+    OwnLds lds{std::max(NLDS, NCLDS<A>)};
     std::vector<std::unique_ptr<emu::Tracked>> tr;
     explicit Replay(const std::vector<u64>& p) : primes(p), nt(build_ntt_tables(p, LOGN, true)) {}
 
@@ -143,28 +143,28 @@ struct Replay {
         track(b, "inv");
         OwnView lv{&lds};
         with(prime, true, [&](const auto& ar) {
-            for (u32 tile = 0; tile < TILES; ++tile)
-                run_group(lds, [&](u32 tid) {
+            for (u32 tile = 0; tile < CTILES; ++tile)
+                run_group(lds, NCT<A>, [&](u32 tid) {
                     const NarrowCol<A> P(LOGN, tile, tid);
                     narrow_fwd_cols<A>(ar, P, f.data(), lv, [&](auto& v) {
                         for (u32 k = 0; k < NW; ++k) v[k] = ar.from_canon(glb(in.data())[P.word(sub(P.o, k, A - LW))]);
                     });
                 });
             for (u32 tile = 0; tile < TILES; ++tile)
-                run_group(lds, [&](u32 tid) { narrow_fwd_rows_store<B>(ar, f.data(), lv, LOGN, tile, tid); });
+                run_group(lds, NT, [&](u32 tid) { narrow_fwd_rows_store<B>(ar, f.data(), lv, LOGN, tile, tid); });
         });
         or_ntt_forward_limbs(n, &primes[prime], 1, want.data());
         same(f, want.data(), "narrow forward transform differs");
         with(prime, false, [&](const auto& ar) {
             for (u32 tile = 0; tile < TILES; ++tile)
-                run_group(lds, [&](u32 tid) {
+                run_group(lds, NT, [&](u32 tid) {
                     const NarrowRow<B> P(tile, tid);
                     narrow_inv_rows<B>(ar, P, b.data(), lv, LOGN, [&](auto& v) {
                         for (u32 k = 0; k < NW; ++k) v[k] = ar.from_canon(glb(f.data())[P.word(NW * P.o + k)]);
                     });
                 });
-            for (u32 tile = 0; tile < TILES; ++tile)
-                run_group(lds, [&](u32 tid) { narrow_inv_cols<A, false>(ar, b.data(), lv, LOGN, tile, tid); });
+            for (u32 tile = 0; tile < CTILES; ++tile)
+                run_group(lds, NCT<A>, [&](u32 tid) { narrow_inv_cols<A, false>(ar, b.data(), lv, LOGN, tile, tid); });
         });
         same(b, in.data(), "narrow inverse transform differs");
         untrack();
@@ -218,9 +218,9 @@ struct Replay {
                 const IpInvJob J{limb_job(Q.size() + k, false), y.data() + k * n, yw, P[k], 0};
                 for (u32 part = 0; part < 2; ++part) {
                     for (u32 tile = 0; tile < TILES; ++tile)
-                        run_group(lds, [&](u32 tid) { narrow_ip_inv_rows<B>(ar, J, part, &nt.pc[P[k]], lv, LOGN, tile, tid); });
-                    for (u32 tile = 0; tile < TILES; ++tile)
-                        run_group(lds, [&](u32 tid) { narrow_inv_cols<A, true>(ar, y.data() + part * yw + k * n, lv, LOGN, tile, tid); });
+                        run_group(lds, NT, [&](u32 tid) { narrow_ip_inv_rows<B>(ar, J, part, &nt.pc[P[k]], lv, LOGN, tile, tid); });
+                    for (u32 tile = 0; tile < CTILES; ++tile)
+                        run_group(lds, NCT<A>, [&](u32 tid) { narrow_inv_cols<A, true>(ar, y.data() + part * yw + k * n, lv, LOGN, tile, tid); });
                 }
             });
         std::vector<uint32_t> perm(n);
@@ -275,15 +275,15 @@ struct Replay {
                            {(double)inv, (double)inv / (double)q}, Q[l], 0};
                 u64* zl = z.data() + part * zw + l * n;
                 with(Q[l], true, [&](const auto& ar) {
-                    for (u32 tile = 0; tile < TILES; ++tile)
-                        run_group(lds, [&](u32 tid) {
+                    for (u32 tile = 0; tile < CTILES; ++tile)
+                        run_group(lds, NCT<A>, [&](u32 tid) {
                             const NarrowCol<A> C(LOGN, tile, tid);
                             narrow_fwd_cols<A>(ar, C, zl, lv, [&](auto& v) {
                                 conv_words<NW, 4>(ar, T.srcs.data(), R, tgp, &nt.pc[Q[l]], LOGN, (u32)C.word(C.o), A - LW + C.B, v);
                             });
                         });
                     for (u32 tile = 0; tile < TILES; ++tile)
-                        run_group(lds, [&](u32 tid) { narrow_ip_fin<B>(ar, J, part, &nt.pc[Q[l]], q, lv, LOGN, tile, tid); });
+                        run_group(lds, NT, [&](u32 tid) { narrow_ip_fin<B>(ar, J, part, &nt.pc[Q[l]], q, lv, LOGN, tile, tid); });
                     const u64* got = out.data() + part * zw + l * n;
                     for (u64 i = 0; i < n; ++i)
                         if (got[i] != want[i]) emu::die("narrow row pass + inner product + finish differs", (double)i, l);
@@ -293,7 +293,7 @@ struct Replay {
                                       inv, hm::shoup(inv, q), Q[l], 0, {(double)inv, (double)inv / (double)q}};
                     std::fill(out.begin(), out.end(), ~0ull);
                     for (u32 tile = 0; tile < TILES; ++tile)
-                        run_group(lds, [&](u32 tid) { narrow_fin<B>(ar, zl, &F, q, lv, LOGN, tile, tid); });
+                        run_group(lds, NT, [&](u32 tid) { narrow_fin<B>(ar, zl, &F, q, lv, LOGN, tile, tid); });
                     for (u64 i = 0; i < n; ++i)
                         if (got[i] != want[i]) emu::die("narrow row pass + finish differs", (double)i, l);
                 });
