@@ -55,7 +55,7 @@ struct FinishJob {
     u64* out;
     const u64* add;
     u64 inv, inv_s;
-    u32 prime, pad;
+    u32 prime, add_galois;  // add_galois: the addend is read through this Galois permutation (0: as it is)
     FTw inv_f;  // inv and its quotient by q (f64 path, q < 2^50)
 };
 

@@ -3,6 +3,7 @@
 // matrix-core kernel. FMA contraction is disabled for this file (the f64 overflow estimate must
 // round like the CPU path).
 #include "basis.h"
+#include "ip_arith.h"
 
 #pragma clang fp contract(off)
 
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(256) void k_finish(const FinishJob* __restrict__ jo
     const FinishJob job = jobs[blockIdx.y];
     const u64 q = pc[job.prime].q;
     u64 v = shoup(sub_mod(glb(job.a)[c], glb(job.t)[c], q), job.inv, job.inv_s, q);
-    if (job.add) v = add_mod(v, glb(job.add)[c], q);
+    if (job.add) v = add_mod(v, glb(job.add)[job.add_galois ? galois_index(c, job.add_galois, log_n) : c], q);
     glb(job.out)[c] = v;
 }
 

@@ -895,7 +895,7 @@ CtPtr Evaluator::conjugate(const Ct& ct) {
 
 // Evaluator::hoisted_rotate (evaluator.rs:572-611): every key looked up first, one
 // decomposition of c1, then every step's inner product (digits read through sigma_g) and
-// mod_down in one batch; sigma_g(c0) is added in the mod_down finish.
+// mod_down in one batch; the mod_down finish adds c0, read through sigma_g.
 std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int32_t>& steps) {
     check_basis(ct);
     check_galois_input(ct);
@@ -926,11 +926,10 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
     hipStream_t s = ctx.stream();
     BufPtr digs = ctx.alloc(nd * dw + L * n);
     ctx.decompose({{ct.comps[1]->data(), level, digs->ptr, digs->ptr + nd * dw}}, s);
-    const u64 per = (2 * (L + k) + 2 * k + 2 * L + L) * n;  // acc, y, z, sigma(c0)
+    const u64 per = (2 * (L + k) + 2 * k + 2 * L) * n;  // acc, y, z
     BufPtr scratch = ctx.alloc_polys(per * nontrivial, nontrivial);
     BufPtr out = ctx.alloc_polys(2 * L * n * nontrivial, 2 * nontrivial);
     std::vector<ApplyTask> tasks;
-    std::vector<AutJob> aut;  // sigma_g(c0) of every step, in the same program
     u32 t = 0;
     for (size_t i = 0; i < steps.size(); ++i) {
         if (!keys[i].first) {
@@ -940,16 +939,14 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
         u64* acc = scratch->ptr + t * per;
         u64* y = acc + 2 * (L + k) * n;
         u64* z = y + 2 * k * n;
-        u64* r0 = z + 2 * L * n;
-        for (u32 li = 0; li < L; ++li) aut.push_back({ct.comps[0]->data() + li * n, r0 + li * n, keys[i].first});
         u64* ob = out->ptr + 2 * L * n * t;
-        tasks.push_back({digs->ptr, level, keys[i].first, keys[i].second, ob, ob + L * n, r0, nullptr, acc, y, z});
+        tasks.push_back({digs->ptr, level, keys[i].first, keys[i].second, ob, ob + L * n, ct.comps[0]->data(), nullptr, acc, y,
+                         z, nullptr, false, (u32)keys[i].first});
         res[i] = make_ct({view(out, 2 * L * n * t, level, 0, true), view(out, 2 * L * n * t + L * n, level, 0, true)},
                          ct.scale);
         ++t;
     }
     Program prog;
-    prog.step(S_AUTOMORPH, prog.add(aut), (u32)aut.size());
     ctx.prog_apply(prog, tasks, ctx.md_variant());
     ctx.execute(prog, s);
     hip_check(hipGetLastError(), "hoisted rotate");
@@ -959,7 +956,7 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
 
 // Hoisted rotations of several ciphertexts (each with its own steps) in batched launches: every
 // check first (nothing runs if one fails), one decomposition program for all inputs, then one
-// program of every step's automorphism, inner product and mod_down. The same words and counts
+// program of every step's inner product and mod_down. The same words and counts
 // as hoisted_rotate per item.
 std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
     const std::vector<std::pair<const Ct*, std::vector<int32_t>>>& items) {
@@ -981,7 +978,7 @@ std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
             nt += e != 0;
         }
         if (nt) dig_words += ctx.ndigits(level) * ctx.digit_words(level) + L * n;
-        scr_words += nt * (2 * (L + k) + 2 * k + 2 * L + L) * n;
+        scr_words += nt * (2 * (L + k) + 2 * k + 2 * L) * n;
         out_words += nt * 2 * L * n;
         nontrivial += nt;
     }
@@ -1001,13 +998,12 @@ std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
     BufPtr digs = ctx.alloc(dig_words), scratch = ctx.alloc(scr_words), out = ctx.alloc(out_words);
     std::vector<DecTask> dec;
     std::vector<ApplyTask> tasks;
-    std::vector<AutJob> aut;
     u64 dpos = 0, spos = 0, opos = 0;
     for (size_t i = 0; i < items.size(); ++i) {
         const Ct& ct = *items[i].first;
         const u32 level = ct.level();
         const u64 L = level + 1;
-        const u64 per = (2 * (L + k) + 2 * k + 2 * L + L) * n;
+        const u64 per = (2 * (L + k) + 2 * k + 2 * L) * n;
         bool any = false;
         for (auto& kk : keys[i]) any |= kk.first != 0;
         u64* dig = nullptr;
@@ -1026,18 +1022,16 @@ std::vector<std::vector<CtPtr>> Evaluator::hoisted_rotate_batch(
             u64* acc = scratch->ptr + spos;
             u64* y = acc + 2 * (L + k) * n;
             u64* z = y + 2 * k * n;
-            u64* r0 = z + 2 * L * n;
             spos += per;
-            for (u32 li = 0; li < L; ++li) aut.push_back({ct.comps[0]->data() + li * n, r0 + li * n, e});
             u64* ob = out->ptr + opos;
-            tasks.push_back({dig, level, e, keys[i][j].second, ob, ob + L * n, r0, nullptr, acc, y, z});
+            tasks.push_back({dig, level, e, keys[i][j].second, ob, ob + L * n, ct.comps[0]->data(), nullptr, acc, y, z, nullptr,
+                             false, (u32)e});
             res[i].push_back(make_ct({view(out, opos, level, 0, true), view(out, opos + L * n, level, 0, true)}, ct.scale));
             opos += 2 * L * n;
         }
     }
     ctx.decompose(dec, s);
     Program prog;
-    prog.step(S_AUTOMORPH, prog.add(aut), (u32)aut.size());
     ctx.prog_apply(prog, tasks, ctx.md_variant());
     ctx.execute(prog, s);
     hip_check(hipGetLastError(), "hoisted rotate");

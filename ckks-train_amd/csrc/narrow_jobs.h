@@ -36,7 +36,7 @@ struct IpFinJob {
     const u64 *add_b, *add_a;
     u64 inv, inv_s;
     FTw inv_f;
-    u32 prime, pad;
+    u32 prime, add_galois;  // add_galois: add_b is read through this Galois permutation (0: as it is)
 };
 
 }  // namespace ckh

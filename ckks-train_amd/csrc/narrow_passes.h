@@ -346,6 +346,13 @@ CKH_DEV void narrow_finish(const Ar& ar, const typename Ar::V (&a)[NW], const ty
     }
 }
 
+// NW consecutive words of an optional addend, read through a Galois permutation when g != 0.
+CKH_DEV void load_addend(const u64* p, u32 g, u32 i0, u32 log_n, u64 (&add)[NW]) {
+    if (!p) return;
+#pragma unroll
+    for (u32 k = 0; k < NW; ++k) add[k] = glb(p)[g ? galois_index(i0 + k, g, log_n) : i0 + k];
+}
+
 // The row pass, the inner product of one part and the finish.
 template <u32 M, class Ar, class Lds>
 CKH_DEV void narrow_ip_fin(const Ar& ar, const IpFinJob& J, u32 part, const PrimeConst* pc, u64 q, Lds lds, u32 log_n,
@@ -356,9 +363,7 @@ CKH_DEV void narrow_ip_fin(const Ar& ar, const IpFinJob& J, u32 part, const Prim
     const u64* add_p = part ? J.add_a : J.add_b;
     u64 add[NW] = {};
     narrow_fwd_rows<M>(ar, P, J.t + part * J.t_part, lds, log_n, v, [&] {
-        if (add_p)
-#pragma unroll
-            for (u32 k = 0; k < NW; ++k) add[k] = glb(add_p)[i0 + k];
+        load_addend(add_p, part ? 0 : J.add_galois, i0, log_n, add);
         limb_ip(ar, J.ip, part, pc, log_n, i0, a);
     });
     narrow_finish(ar, a, v, add_p != nullptr, add, part ? J.out_a : J.out_b, J.inv, J.inv_s, J.inv_f, q, i0);
@@ -372,9 +377,7 @@ CKH_DEV void narrow_fin(const Ar& ar, const u64* in_p, const FinishJob* fin, u64
     typename Ar::V v[NW], a[NW];
     u64 add[NW] = {};
     narrow_fwd_rows<M>(ar, P, in_p, lds, log_n, v, [&] {
-        if (fin->add)
-#pragma unroll
-            for (u32 k = 0; k < NW; ++k) add[k] = glb(fin->add)[i0 + k];
+        load_addend(fin->add, fin->add_galois, i0, log_n, add);
 #pragma unroll
         for (u32 k = 0; k < NW; ++k) a[k] = ar.from_canon(glb(fin->a)[i0 + k]);
     });

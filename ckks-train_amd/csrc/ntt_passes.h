@@ -30,6 +30,7 @@
 #pragma once
 
 #include "arith.h"
+#include "ip_arith.h"
 
 #ifndef CKH_WAVE_SYNC
 #define CKH_WAVE_SYNC() __syncthreads()
@@ -413,6 +414,7 @@ CKH_DEV void fwd_rows(const Ar& ar, const u64* __restrict__ in, u64* __restrict_
         const auto fa = glb(fin->a), fadd = glb(fin->add);
         const auto fout = glb(fin->out);
         const bool has_add = fin->add != nullptr;
+        const u32 g = fin->add_galois;
         const u64 inv = fin->inv, inv_s = fin->inv_s;
         u64 av[16], dv[16];
         // a (and the addend) loaded once the row pass's registers are free, before its last barrier
@@ -420,7 +422,8 @@ CKH_DEV void fwd_rows(const Ar& ar, const u64* __restrict__ in, u64* __restrict_
 #pragma unroll
             for (u32 k = 0; k < 16; ++k) {
                 av[k] = fa[tbase + tid + k * NT];
-                dv[k] = has_add ? (u64)fadd[tbase + tid + k * NT] : (u64)0;
+                const u32 i = (u32)tbase + tid + k * NT;
+                dv[k] = has_add ? (u64)fadd[g ? galois_index(i, g, log_n) : i] : (u64)0;
             }
         };
         if constexpr (Ar::F64) {

@@ -1046,7 +1046,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
     for (const ApplyTask& t : tasks) {
         const u32 L = t.level + 1;
         const u64 aw = (u64)(L + np) * n;
-        md.push_back({t.acc, t.level, t.out_b, t.add_b, t.y, t.z});
+        md.push_back({t.acc, t.level, t.out_b, t.add_b, t.y, t.z, t.add_galois});
         md.push_back({t.acc + aw, t.level, t.out_a, t.add_a, t.y + (u64)np * n, t.z + (u64)L * n});
     }
     prog_mod_down(p, md, md_variant);
@@ -1078,7 +1078,7 @@ void Context::prog_apply_narrow(Program& p, const std::vector<ApplyTask>& tasks)
         for (u32 i = 0; i < L; ++i)
             fin.push_back({limb_ip(i, i, t.own ? t.own + i * n : nullptr), t.z + i * n, zw, t.out_b + i * n, t.out_a + i * n,
                            t.add_b ? t.add_b + i * n : nullptr, t.add_a ? t.add_a + i * n : nullptr, pinv_[i], pinv_s_[i],
-                           {(double)pinv_[i], (double)pinv_[i] / (double)primes[i]}, i, 0});
+                           {(double)pinv_[i], (double)pinv_[i] / (double)primes[i]}, i, t.add_galois});
     }
     const size_t o_inv = p.add(inv);
     p.step(S_IP_INV, o_inv, (u32)inv.size(), p.add(cols));
@@ -1109,8 +1109,8 @@ void Context::prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 va
         for (u32 i = 0; i < L; ++i) {
             u64* zi = t.z + i * n;
             nttr.push_back({zi, zi, i, 0});
-            fin.push_back({t.acc + i * n, zi, t.out + i * n, t.add ? t.add + i * n : nullptr, pinv_[i], pinv_s_[i], i, 0,
-                           {(double)pinv_[i], (double)pinv_[i] / (double)primes[i]}});
+            fin.push_back({t.acc + i * n, zi, t.out + i * n, t.add ? t.add + i * n : nullptr, pinv_[i], pinv_s_[i], i,
+                           t.add_galois, {(double)pinv_[i], (double)pinv_[i] / (double)primes[i]}});
         }
     }
     group_by_prime(intt);

@@ -118,6 +118,7 @@ struct ApplyTask {
     u64* z;
     const u64* own = nullptr;  // set: the digits' own limbs are read from this d (not copied)
     bool fused = false;        // the digits come from a DecTask with fuse set (needs own)
+    u32 add_galois = 0;        // set (not with fused): add_b is read through sigma_add_galois
 };
 
 // One mod_down of a QpPoly sum (level l, l + 1 + k limbs, NTT form) -> out (l + 1 limbs) plus an
@@ -129,6 +130,7 @@ struct MdTask {
     const u64* add;
     u64* y;
     u64* z;
+    u32 add_galois = 0;  // set: add is read through this Galois permutation
 };
 
 // One rescale of a polynomial (level l -> l - 1): out (l limbs), scratch x (1 limb), z (l limbs).

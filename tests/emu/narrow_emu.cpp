@@ -1,7 +1,7 @@
 // CPU replay of the narrow passes (ckks-train_amd/csrc/narrow_passes.h): both transforms for N = 2^12 ..
 // 2^16, and at 2^12 and 2^13 a key switch's apply stage (inner product + inverse transform in y form;
 // conversion + column pass; row pass + inner product + finish, with and without the Galois permutation, an
-// own digit and addends; row pass + finish), for 50-, 40- and 60-bit primes, against the oracle's
+// own digit and addends, part b's read through the same permutation; row pass + finish), for 50-, 40- and 60-bit primes, against the oracle's
 // transforms and conversion and 128-bit sums. LDS: between two barriers no thread touches a slot that
 // another one writes. Test infrastructure only (built by tests/test_narrow.py).
 #include <algorithm>
@@ -266,13 +266,13 @@ struct Replay {
                 std::vector<u64> s = sum(l, own, part), want(n);
                 for (u64 i = 0; i < n; ++i) {
                     want[i] = mulm((s[i] + q - w[l * n + i]) % q, inv, q);
-                    if (add) want[i] = (want[i] + addv[part * zw + l * n + i]) % q;
+                    if (add) want[i] = (want[i] + addv[part * zw + l * n + (part ? i : perm[i])]) % q;
                 }
                 const ConvColRef R{y.data() + part * yw, nullptr, 0, 1, 0, l, (u32)P.size(), small};
                 const ConvTgt* tgp = &T.tgts[l];
                 IpFinJob J{limb_job(l, own), z.data() + l * n, zw, out.data() + l * n, out.data() + zw + l * n,
                            add ? addv.data() + l * n : nullptr, add ? addv.data() + zw + l * n : nullptr, inv, hm::shoup(inv, q),
-                           {(double)inv, (double)inv / (double)q}, Q[l], 0};
+                           {(double)inv, (double)inv / (double)q}, Q[l], (u32)galois};
                 u64* zl = z.data() + part * zw + l * n;
                 with(Q[l], true, [&](const auto& ar) {
                     for (u32 tile = 0; tile < CTILES; ++tile)
@@ -290,7 +290,7 @@ struct Replay {
                     // the finish alone, its first operand in memory
                     std::copy(s.begin(), s.end(), ownv.begin() + l * n);
                     const FinishJob F{ownv.data() + l * n, zl, out.data() + part * zw + l * n, add ? addv.data() + part * zw + l * n : nullptr,
-                                      inv, hm::shoup(inv, q), Q[l], 0, {(double)inv, (double)inv / (double)q}};
+                                      inv, hm::shoup(inv, q), Q[l], part ? 0 : (u32)galois, {(double)inv, (double)inv / (double)q}};
                     std::fill(out.begin(), out.end(), ~0ull);
                     for (u32 tile = 0; tile < TILES; ++tile)
                         run_group(lds, NT, [&](u32 tid) { narrow_fin<B>(ar, zl, &F, q, lv, LOGN, tile, tid); });
