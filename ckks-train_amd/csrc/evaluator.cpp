@@ -306,7 +306,7 @@ void check_switch(const Context& c, const Poly& d, const Ksk& key) {
 // The program of a batch of requests (decompose + apply, one launch per stage), its scratch laid
 // out from base (ks_scratch_words per request, in request order).
 static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
-                          const std::vector<AutJob>* pre = nullptr) {
+                          const std::vector<AutJob>* pre = nullptr, bool compact = false) {
     u64 limbs = 0;
     for (auto& r : reqs) limbs += r.d->level + 1;
     const bool small = limbs <= c.small_limbs;
@@ -326,6 +326,7 @@ static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
         app.push_back({dig, r.d->level, 0, r.key, r.out_b, r.out_a, r.add_b, r.add_a, acc, y, z, r.d->data(), fuse});
     }
     Program prog;  // one program (one graph when captured) per batched switch
+    prog.compact = compact;
     if (pre) prog.step(S_AUTOMORPH, prog.add(*pre), (u32)pre->size());
     c.prog_decompose(prog, dec, small ? c.conv_variant_s : c.conv_variant);
     c.prog_apply(prog, app, small ? c.conv_variant_s : c.md_variant());
@@ -463,6 +464,8 @@ void ks_switch_batch_static(Context& c, const std::vector<const Poly*>& ds, cons
     // Workspace: the switches' scratch from the start, the descriptor bytes after it.
     Program prog = ks_program(c, reqs, (u64*)c.static_scratch);
     const u64 desc_off = (scratch_bytes + 255) & ~(u64)255;
+    if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)  // the last bytes of the workspace
+        prog = ks_program(c, reqs, (u64*)c.static_scratch, nullptr, true);
     if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)
         fail(CKH_ERR_INVALID_PARAMS, "batch needs more than the static workspace");
     hipStream_t s = c.stream();

@@ -893,7 +893,7 @@ void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 
     const bool yf = yform_usable(variant == 2 && conv.mf_ok ? 4 : 1);
     u64 targets = 0;
     for (const DecTask& t : tasks) targets += (u64)ndigits(t.level) * (t.level + 1 + np) - (t.level + 1);
-    const bool cc = yf && conv_cols_usable(alpha, targets, variant);
+    const bool cc = yf && !p.compact && conv_cols_usable(alpha, targets, variant);
     for (const DecTask& t : tasks) {
         const u32 L = t.level + 1;
         const u64 ds = digit_words(t.level);
@@ -948,7 +948,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
         targets += 2 * (t.level + 1);
         any_fused |= t.fused;
     }
-    if (!any_fused && targets << (log_n - 12) <= NARROW_IP_TILES && yform_usable(2) &&
+    if (!any_fused && !p.compact && targets << (log_n - 12) <= NARROW_IP_TILES && yform_usable(2) &&
         conv_cols_usable(np, targets, md_variant))
         return prog_apply_narrow(p, tasks);
     // Several tasks, each under a key of its own: the key words are read once. (A single switch may
@@ -976,7 +976,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
         std::vector<ConvColRef> ccols;
         u64 targets = 0;
         for (const ApplyTask& t : tasks) targets += 2 * (t.level + 1);
-        const bool yf = yform_usable(2), cc = yf && conv_cols_usable(np, targets, md_variant);
+        const bool yf = yform_usable(2), cc = yf && !p.compact && conv_cols_usable(np, targets, md_variant);
         for (const ApplyTask& t : tasks) {
             const u32 L = t.level + 1;
             const u64 aw = (u64)(L + np) * n;
@@ -1096,7 +1096,7 @@ void Context::prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 va
     u32 max_l = 0;
     u64 targets = 0;
     for (const MdTask& t : tasks) targets += t.level + 1;
-    const bool yf = yform_usable(2), cc = yf && conv_cols_usable(np, targets, variant);
+    const bool yf = yform_usable(2), cc = yf && !p.compact && conv_cols_usable(np, targets, variant);
     for (const MdTask& t : tasks) {
         const u32 L = t.level + 1;
         max_l = std::max(max_l, L);

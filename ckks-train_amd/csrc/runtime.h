@@ -174,6 +174,8 @@ struct Program {
     };
     std::vector<uint8_t> bytes;
     std::vector<Step> steps;
+    bool compact = false;  // fewest descriptor bytes: no conversion fused with its column passes (a
+                           // descriptor per target), for a caller whose workspace is short of them
     // Appends v at a 16-byte aligned offset of the descriptor bytes and returns the offset.
     template <class T>
     size_t add(const std::vector<T>& v) {
