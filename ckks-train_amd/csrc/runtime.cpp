@@ -84,6 +84,9 @@ Context::Context(int ordinal, const ckh_params& p, u32 n_streams) {
         void* rp = nullptr;
         hip_check(hipHostMalloc(&rp, ring_cap_, hipHostMallocDefault), "hipHostMalloc(staging ring)");
         ring_ = (uint8_t*)rp;
+        void* rd = nullptr;
+        hip_check(hipHostGetDevicePointer(&rd, rp, 0), "hipHostGetDevicePointer(staging ring)");
+        ring_dev_ = (const uint8_t*)rd;
         for (int i = 0; i < 32; ++i) {
             hipEvent_t ev;
             hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
@@ -464,7 +467,11 @@ void Context::h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
         const size_t len = std::min(chunk_max, bytes - done);
         const size_t off = ring_reserve(len);
         std::memcpy(ring_ + off, (const uint8_t*)src + done, len);
-        hip_check(hipMemcpyAsync((uint8_t*)dst + done, ring_ + off, len, hipMemcpyHostToDevice, s), "upload");
+        uint8_t* to = (uint8_t*)dst + done;
+        if (len > UPLOAD_COMMAND && len <= UPLOAD_KERNEL && len % 16 == 0 && (uintptr_t)to % 16 == 0)
+            upload_launch(ring_dev_ + off, to, len, s);
+        else
+            hip_check(hipMemcpyAsync(to, ring_ + off, len, hipMemcpyHostToDevice, s), "upload");
         if (std::find(run_streams_.begin(), run_streams_.end(), s) == run_streams_.end()) run_streams_.push_back(s);
         if (run_len_ >= RING_RUN) ring_close_run();
         done += len;

@@ -396,6 +396,12 @@ class Context : public std::enable_shared_from_this<Context> {
     static constexpr size_t RING_RUN = (size_t)1 << 20;
     std::mutex ring_mu_;
     uint8_t* ring_ = nullptr;  // pinned host memory
+    const uint8_t* ring_dev_ = nullptr;  // the ring as kernels address it
+    // Uploads of more than UPLOAD_COMMAND and at most UPLOAD_KERNEL bytes are read by a kernel (upload_launch):
+    // up to 16 KB a copy command is a small kernel too and as fast (37.3 against 37.1 us for a switch at
+    // N = 2^12); beyond, it is a DMA transfer (eight switches at 2^12 181 -> 50 us, 64 relinearizations at
+    // 2^13 175 -> 157 us). Above 1 MB, ciphertexts rather than descriptors, the DMA engine keeps the rate.
+    static constexpr size_t UPLOAD_COMMAND = 16384, UPLOAD_KERNEL = 1 << 20;
     size_t ring_cap_ = 0, ring_head_ = 0;
     size_t run_off_ = 0, run_len_ = 0;      // the open run
     std::vector<hipStream_t> run_streams_;  // streams with copies from it
