@@ -259,9 +259,15 @@ CKH_DEV void narrow_inv_cols(const Ar& ar, u64* io_p, Lds lds, u32 log_n, u32 ti
 
 // ---------------------------------------------------------------- inner product
 
+// Digits of an inner product loaded before their products. Four keep 160-194 registers (2-3 waves per
+// SIMD); two take 114-132 and a switch of 24 limbs at N = 2^16 171 against 177 us, but where the rows have 2^6
+// words a launch is small and waits for one group more: 32.7 against 32.2 us at 2^12.
+template <u32 M>
+constexpr u32 NARROW_IP_GROUP = M == 6 ? 4 : 2;
+
 // Words i0 .. i0 + NW - 1 of one part of an inner product. f64 primes: signed sums, |.| <= q / 2; integer
 // primes: canonical words. A group's digits and keys are loaded before its products.
-template <class Ar>
+template <u32 G, class Ar>
 CKH_DEV void limb_ip(const Ar& ar, const LimbIp& J, u32 part, const PrimeConst* pc, u32 log_n, u32 i0, typename Ar::V (&out)[NW]) {
     u32 di[NW];
 #pragma unroll
@@ -270,10 +276,10 @@ CKH_DEV void limb_ip(const Ar& ar, const LimbIp& J, u32 part, const PrimeConst* 
     [[maybe_unused]] Dot60 d[NW];
 #pragma unroll
     for (u32 k = 0; k < NW; ++k) s[k] = 0.0;
-    for (u32 j0 = 0; j0 < J.ndig; j0 += IP_GROUP) {
-        u64 dv[IP_GROUP][NW], kv[IP_GROUP][NW];
+    for (u32 j0 = 0; j0 < J.ndig; j0 += G) {
+        u64 dv[G][NW], kv[G][NW];
 #pragma unroll
-        for (u32 u = 0; u < IP_GROUP; ++u) {
+        for (u32 u = 0; u < G; ++u) {
             const u32 j = j0 + u;
             if (j < J.ndig) {
                 const auto dig = glb((J.own && j == J.own_j) ? J.own : J.dig + j * J.dig_stride);
@@ -286,7 +292,7 @@ CKH_DEV void limb_ip(const Ar& ar, const LimbIp& J, u32 part, const PrimeConst* 
             }
         }
 #pragma unroll
-        for (u32 u = 0; u < IP_GROUP; ++u) {
+        for (u32 u = 0; u < G; ++u) {
             if (j0 + u < J.ndig) {
 #pragma unroll
                 for (u32 k = 0; k < NW; ++k) {
@@ -299,7 +305,7 @@ CKH_DEV void limb_ip(const Ar& ar, const LimbIp& J, u32 part, const PrimeConst* 
                 }
             }
         }
-        // four products (|.| < 0.7 q each) since the last reduction
+        // at most four products (|.| < 0.7 q each) since the last reduction
         if constexpr (Ar::F64) {
 #pragma unroll
             for (u32 k = 0; k < NW; ++k) s[k] = freduce(s[k], ar.q, ar.qinv);
@@ -323,7 +329,7 @@ CKH_DEV void narrow_ip_inv_rows(const Ar& ar, const IpInvJob& J, u32 part, const
                                 u32 tile, u32 tid) {
     const NarrowRow<M> P(tile, tid);
     narrow_inv_rows<M>(ar, P, J.out + part * J.out_part, lds, log_n,
-                       [&](typename Ar::V(&v)[NW]) { limb_ip(ar, J.ip, part, pc, log_n, P.word(NW * P.o), v); });
+                       [&](typename Ar::V(&v)[NW]) { limb_ip<NARROW_IP_GROUP<M>>(ar, J.ip, part, pc, log_n, P.word(NW * P.o), v); });
 }
 
 // (a - t) inv (+ add) of NW consecutive words: t the row pass's words (f64: |.| <= 2.6 q), a the first
@@ -364,7 +370,7 @@ CKH_DEV void narrow_ip_fin(const Ar& ar, const IpFinJob& J, u32 part, const Prim
     u64 add[NW] = {};
     narrow_fwd_rows<M>(ar, P, J.t + part * J.t_part, lds, log_n, v, [&] {
         load_addend(add_p, part ? 0 : J.add_galois, i0, log_n, add);
-        limb_ip(ar, J.ip, part, pc, log_n, i0, a);
+        limb_ip<NARROW_IP_GROUP<M>>(ar, J.ip, part, pc, log_n, i0, a);
     });
     narrow_finish(ar, a, v, add_p != nullptr, add, part ? J.out_a : J.out_b, J.inv, J.inv_s, J.inv_f, q, i0);
 }

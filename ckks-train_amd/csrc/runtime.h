@@ -376,9 +376,9 @@ class Context : public std::enable_shared_from_this<Context> {
     u32 conv_cols = 1;
     // A key switch's apply stage of at most this many 4096-word tiles of Q limbs (both parts) runs its
     // inner product inside the row passes (narrow_ip_inverse, narrow_ip_finish): one launch and the sums'
-    // way through memory less against reading the digits once per part. One switch of 6 limbs at 2^12 37.2
-    // against 38.0 us, of 20 at 2^15 115.7 against 121.3, of 18 at 2^16 (576 tiles) 151 against 155, of 24
-    // (768) the same; two of 24 (1536) 340 against 328 us.
+    // way through memory less against reading the digits once per part. One switch of 6 limbs at 2^12 32.1
+    // against 34.7 us (launched directly), of 20 at 2^15 97 against 102, of 18 at 2^16 130 against 139, of
+    // 24 (768 tiles) 174 against 184; two of 24 (1536 tiles) 307 against 306.
     static constexpr u32 NARROW_IP_TILES = 1024;
     bool conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const;
     // Appends the targets of one conversion (plan, first source limb, output polynomial).
