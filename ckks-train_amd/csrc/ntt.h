@@ -87,6 +87,13 @@ void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef*
 // the column passes change over once the chip is full: 320 tiles against 640 or more, 134 against 140
 // us for an 18-limb switch at 2^16 and 183 against 184 for 24 limbs, against none the same switch of 8
 // limbs 85 against 98; all column passes narrow, a batch of 256 switches takes 19.5 against 16.4 ms.
+//
+// Transforms of their own (narrow_alone) change over at 128 tiles: the narrow passes load 12 twiddles for 4
+// words, which bounds 50-bit limbs from about 256 tiles on (forward at 2^14, wide / narrow: 64 tiles 10.2 /
+// 8.2 us, 256 12.0 / 19.0, 3,840 88 / 123), where a key switch's launches hold 60-bit limbs, whose wide
+// passes read the whole table too.
+constexpr u32 NARROW_ALONE_TILES = 128;
+inline bool narrow_alone(u32 log_n, u32 nrefs) { return ((u64)nrefs << (log_n - 12)) <= NARROW_ALONE_TILES; }
 constexpr u32 NARROW_TILES = 4096, NARROW_COL8_TILES = 320;
 inline bool narrow_rows(u32 log_n, u32 nrefs) { return ((u64)nrefs << (log_n - 12)) <= NARROW_TILES; }
 inline bool narrow_cols(u32 log_n, u32 nrefs) {

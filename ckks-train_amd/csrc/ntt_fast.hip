@@ -453,8 +453,13 @@ static void launch_m(u32 m, bool fwd, bool cols, const NttTables& t, const LimbR
 
 // Split N = 2^(A+B): B = floor(log N / 2) row stages, A column stages (6..8 each).
 void ntt_fast_forward(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s) {
-    ntt_fast_forward_cols(t, refs, nrefs, s);
-    ntt_fast_forward_rows(t, refs, nrefs, s);
+    if (narrow_alone(t.log_n, nrefs)) {
+        narrow_forward_cols(t, refs, nrefs, s);
+        narrow_forward_rows(t, refs, nrefs, nullptr, s);
+    } else {
+        launch_m(t.log_n - t.log_n / 2, true, true, t, refs, nrefs, s);
+        launch_m(t.log_n / 2, true, false, t, refs, nrefs, s);
+    }
 }
 
 void ntt_fast_forward_finish(const NttTables& t, const LimbRef* refs, const FinishJob* fin, u32 nrefs,
@@ -528,11 +533,11 @@ void conv_cols_launch(const ConvTables& c, const NttTables& t, const ConvColRef*
 }
 
 void ntt_fast_inverse(const NttTables& t, const LimbRef* refs, u32 nrefs, hipStream_t s, const YForm* yf) {
-    if (narrow_rows(t.log_n, nrefs))
+    if (yf ? narrow_rows(t.log_n, nrefs) : narrow_alone(t.log_n, nrefs))
         narrow_inverse_rows(t, refs, nrefs, s);
     else
         launch_m(t.log_n / 2, false, false, t, refs, nrefs, s);
-    if (narrow_cols(t.log_n, nrefs))
+    if (yf ? narrow_cols(t.log_n, nrefs) : narrow_alone(t.log_n, nrefs))
         narrow_inverse_cols(t, refs, nrefs, yf, s);
     else
         launch_m(t.log_n - t.log_n / 2, false, true, t, refs, nrefs, s, nullptr, yf);
