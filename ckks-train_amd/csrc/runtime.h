@@ -308,9 +308,8 @@ class Context : public std::enable_shared_from_this<Context> {
     // (all of them: the sources are read once; 8 per workgroup took 17.54 against 16.83 ms per step of
     // 256 switches at N = 2^16, 3.65 against 3.60 ms for the 32 x 32 product at 2^15)
     // The variant of mod_down's conversions (P -> Q) in batched programs (tuning key
-    // "conv_variant_md"; 3 = conv_variant). Default 1: with 60-bit sources the exact f64 piece
-    // sums beat two modular products per source (step 19.98 -> 19.54 ms on the 256-switch
-    // workload), while the ModUp conversions (50-bit sources) keep conv_variant.
+    // "conv_variant_md"; 3 = conv_variant). 0 and 1 are the same vector kernel, 2 the matrix-core
+    // kernel (15.90 against 16.85 ms for 256 switches at N = 2^16).
     u32 conv_variant_md = 1;
     u32 md_variant() const { return conv_variant_md < 3 ? conv_variant_md : conv_variant; }
     // Batched key switches of at most small_limbs input limbs in all (a single switch, a few
