@@ -51,8 +51,9 @@ void add_sum_launch(const AddSumJob* jobs, const u64* const* xs, u32 njobs, cons
 void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n, bool keys_once,
                           hipStream_t stream);
 
-// out <- bytes (a multiple of 16) of pinned host memory, both 16-byte aligned.
-void upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream);
+// out <- bytes (a multiple of 16) of pinned host memory, both 16-byte aligned. Returns the launch's own status:
+// the callers' synchronizations do not report a launch that was refused.
+hipError_t upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream);
 
 // ref.dst <- ref.src (one limb per descriptor).
 // Grid-stride copy of bytes (a multiple of 16) with 16-byte loads and stores.

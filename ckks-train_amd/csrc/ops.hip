@@ -93,9 +93,13 @@ __global__ __launch_bounds__(256) void k_upload(const uint4* __restrict__ in, ui
     if (i < n16) out[i] = in[i];
 }
 
-void upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream) {
-    const u32 n16 = (u32)(bytes / 16);
-    if (n16) hipLaunchKernelGGL(k_upload, dim3((n16 + 255) / 256), dim3(256), 0, stream, (const uint4*)pinned, (uint4*)out, n16);
+hipError_t upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream) {
+    const uint4* in = (const uint4*)pinned;
+    uint4* to = (uint4*)out;
+    u32 n16 = (u32)(bytes / 16);
+    if (n16 == 0) return hipSuccess;
+    void* args[] = {&in, &to, &n16};
+    return hipLaunchKernel((const void*)k_upload, dim3((n16 + 255) / 256), dim3(256), args, 0, stream);
 }
 
 // Streaming copy of n16 16-byte words (a measurement of the HBM copy rate a kernel reaches).

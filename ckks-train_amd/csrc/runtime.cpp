@@ -469,7 +469,7 @@ void Context::h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
         std::memcpy(ring_ + off, (const uint8_t*)src + done, len);
         uint8_t* to = (uint8_t*)dst + done;
         if (len > UPLOAD_COMMAND && len <= UPLOAD_KERNEL && len % 16 == 0 && (uintptr_t)to % 16 == 0)
-            upload_launch(ring_dev_ + off, to, len, s);
+            hip_check(upload_launch(ring_dev_ + off, to, len, s), "upload");
         else
             hip_check(hipMemcpyAsync(to, ring_ + off, len, hipMemcpyHostToDevice, s), "upload");
         if (std::find(run_streams_.begin(), run_streams_.end(), s) == run_streams_.end()) run_streams_.push_back(s);

@@ -1,0 +1,81 @@
+// Checks of the runtime's own code on the host model of HIP (hip_model.h): one function per check,
+// named on the command line. A failed check ends the program with a message.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+#include "../../ckks-train_amd/csrc/evaluator.h"
+#include "../../ckks-train_amd/csrc/hostmath.h"
+#include "hip_model.h"
+
+using namespace ckh;
+
+#define CHECK(x, ...)                                                      \
+    do {                                                                   \
+        if (!(x)) {                                                        \
+            std::fprintf(stderr, "CHECK FAILED (%s:%d): %s ", __FILE__, __LINE__, #x); \
+            std::fprintf(stderr, "" __VA_ARGS__);                          \
+            std::fprintf(stderr, "\n");                                    \
+            std::exit(1);                                                  \
+        }                                                                  \
+    } while (0)
+
+// The largest primes = 1 mod 2N below 2^bits, each once.
+static std::vector<u64> primes_of(u32 log_n, const std::vector<u32>& bits) {
+    std::map<u32, u64> next;
+    std::vector<u64> out;
+    const u64 m = 2ull << log_n;
+    for (u32 b : bits) {
+        u64 q = next.count(b) ? next[b] - m : ((1ull << b) - 1) / m * m + 1;
+        while (q >= (1ull << b) || !hm::is_prime(q)) q -= m;
+        next[b] = q;
+        out.push_back(q);
+    }
+    return out;
+}
+
+static std::shared_ptr<Context> make(u32 log_n, u32 nq, u32 np, u32 dnum, u32 streams = 2) {
+    std::vector<u32> bits(nq, 50);
+    bits.insert(bits.end(), np, 59);
+    const std::vector<u64> p = primes_of(log_n, bits);
+    ckh_params prm{};
+    prm.log_n = log_n;
+    prm.nq = nq;
+    prm.np = np;
+    prm.dnum = dnum;
+    prm.q = p.data();
+    prm.p = p.data() + nq;
+    return std::make_shared<Context>(0, prm, streams);
+}
+
+// An upload whose kernel was not launched is an error, not a buffer of stale words.
+static void upload_launch_checked() {
+    auto c = make(12, 6, 2, 3);
+    std::vector<u64> words(8192);
+    BufPtr b = c->alloc(words.size());
+    model::refuse_launch = true;
+    bool failed = false;
+    try {
+        c->h2d(b->ptr, words.data(), words.size() * 8, c->stream());
+    } catch (const Error& e) {
+        failed = e.status == CKH_ERR_DEVICE;
+    }
+    CHECK(failed);
+    c->h2d(b->ptr, words.data(), words.size() * 8, c->stream());  // and the next one works
+}
+
+int main(int argc, char** argv) {
+    const std::map<std::string, void (*)()> checks = {
+        {"upload_launch_checked", upload_launch_checked},
+    };
+    auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
+    if (it == checks.end()) {
+        std::fprintf(stderr, "no such check\n");
+        return 2;
+    }
+    it->second();
+    std::printf("ok\n");
+    return 0;
+}

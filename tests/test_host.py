@@ -1,0 +1,43 @@
+"""The runtime's host code (ckks-train_amd/csrc/runtime.cpp, evaluator.cpp, server.cpp, autotune.cpp) on a host
+model of the HIP runtime (tests/host/hip_model.cpp): streams whose work runs only when something waits for it,
+copies that move their bytes when they run, kernels that do nothing. The checks are in tests/host/checks.cpp."""
+import concurrent.futures
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(os.path.dirname(HERE), "ckks-train_amd", "csrc")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+SOURCES = [os.path.join(CSRC, f) for f in ("runtime.cpp", "evaluator.cpp", "server.cpp", "autotune.cpp")] + [
+    os.path.join(HERE, "host", f) for f in ("hip_model.cpp", "checks.cpp")]
+# undefined shifts and overflowing signed arithmetic of the host code end a check
+FLAGS = ["--offload-host-only", "-O1", "-std=c++17", "-fPIC", "-ffp-contract=off", "-Xarch_host",
+         "-fsanitize=shift,signed-integer-overflow,bounds", "-Xarch_host",
+         "-fsanitize-trap=shift,signed-integer-overflow,bounds"]
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    out = tmp_path_factory.mktemp("host")
+
+    def compile_one(src):
+        obj = str(out / (os.path.basename(src) + ".o"))
+        subprocess.run([HIPCC, *FLAGS, "-c", src, "-o", obj], check=True)
+        return obj
+
+    with concurrent.futures.ThreadPoolExecutor(6) as ex:
+        objs = list(ex.map(compile_one, SOURCES))
+    prog = str(out / "checks")
+    subprocess.run(["g++", *objs, "-o", prog, "-pthread"], check=True)
+    return prog
+
+
+@pytest.mark.parametrize("check", [
+    "upload_launch_checked",
+])
+def test_host(exe, check):
+    r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.returncode, r.stdout + r.stderr)
