@@ -51,7 +51,7 @@ void add_sum_launch(const AddSumJob* jobs, const u64* const* xs, u32 njobs, cons
 void inner_product_launch(const IpJob* jobs, u32 njobs, const PrimeConst* pc, u32 log_n, bool keys_once,
                           hipStream_t stream);
 
-// out <- bytes (a multiple of 16) of pinned host memory, both 16-byte aligned. Returns the launch's own status:
+// out <- bytes (a multiple of 4) of pinned host memory, both 16-byte aligned. Returns the launch's own status:
 // the callers' synchronizations do not report a launch that was refused.
 hipError_t upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream);
 

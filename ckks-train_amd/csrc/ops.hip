@@ -85,21 +85,25 @@ void copy_launch(const LimbRef* refs, u32 nrefs, u32 log_n, hipStream_t stream) 
     hipLaunchKernelGGL(k_copy, pairs_grid(log_n, nrefs), dim3(256), 0, stream, refs, log_n);
 }
 
-// Staged descriptor bytes to the device, 16 per thread, read from pinned host memory. A copy command of
+// Staged descriptor bytes to the device, 16 per thread and the rest a word per thread (descriptors are of 8
+// bytes modulo 16: a program of an odd number of them ends so), read from pinned host memory. A copy command of
 // more than 16 KB goes to a DMA engine instead: 19 us of the host, 6 us of copying and a switch of queues on
 // either side; the workgroups here read over the bus together.
-__global__ __launch_bounds__(256) void k_upload(const uint4* __restrict__ in, uint4* __restrict__ out, u32 n16) {
+__global__ __launch_bounds__(256) void k_upload(const uint4* __restrict__ in, uint4* __restrict__ out, u32 n16, u32 words) {
     const u32 i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n16) out[i] = in[i];
+    if (i < n16)
+        out[i] = in[i];
+    else if (i - n16 < words)
+        ((u32*)(out + n16))[i - n16] = ((const u32*)(in + n16))[i - n16];
 }
 
 hipError_t upload_launch(const void* pinned, void* out, u64 bytes, hipStream_t stream) {
     const uint4* in = (const uint4*)pinned;
     uint4* to = (uint4*)out;
-    u32 n16 = (u32)(bytes / 16);
-    if (n16 == 0) return hipSuccess;
-    void* args[] = {&in, &to, &n16};
-    return hipLaunchKernel((const void*)k_upload, dim3((n16 + 255) / 256), dim3(256), args, 0, stream);
+    u32 n16 = (u32)(bytes / 16), words = (u32)(bytes % 16 / 4);
+    if (n16 + words == 0) return hipSuccess;
+    void* args[] = {&in, &to, &n16, &words};
+    return hipLaunchKernel((const void*)k_upload, dim3((n16 + words + 255) / 256), dim3(256), args, 0, stream);
 }
 
 // Streaming copy of n16 16-byte words (a measurement of the HBM copy rate a kernel reaches).

@@ -468,7 +468,7 @@ void Context::h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {
         const size_t off = ring_reserve(len);
         std::memcpy(ring_ + off, (const uint8_t*)src + done, len);
         uint8_t* to = (uint8_t*)dst + done;
-        if (len > UPLOAD_COMMAND && len <= UPLOAD_KERNEL && len % 16 == 0 && (uintptr_t)to % 16 == 0)
+        if (len > UPLOAD_COMMAND && len <= UPLOAD_KERNEL && len % 4 == 0 && (uintptr_t)to % 16 == 0)
             hip_check(upload_launch(ring_dev_ + off, to, len, s), "upload");
         else
             hip_check(hipMemcpyAsync(to, ring_ + off, len, hipMemcpyHostToDevice, s), "upload");
@@ -827,7 +827,7 @@ bool Context::execute_graph(const Program& p, hipStream_t s) {
         }
     }
     // The previous replay (on this same stream: plans are per stream) reads the descriptor buffer
-    // being rewritten. The rewrite is a DMA from pinned staging memory queued on s, so it runs
+    // being rewritten. The rewrite is a copy from pinned staging memory queued on s (h2d), so it runs
     // after that replay in stream order; the host does not wait.
     h2d(pl->desc, p.bytes.data(), p.bytes.size(), s);
     if (!pl->exec) {

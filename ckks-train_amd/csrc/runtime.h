@@ -327,7 +327,7 @@ class Context : public std::enable_shared_from_this<Context> {
     // Copies a host blob to a fresh device buffer on stream s.
     BufPtr upload_blob(const void* host, size_t bytes, hipStream_t s);
     // Host-to-device copy ordered on stream s: the bytes are staged in a pinned ring (so the copy
-    // is an ordinary stream-ordered DMA and `src` may be reused on return). Ring slots are reused
+    // is stream-ordered, a command or a kernel by its size, and `src` may be reused on return). Ring slots are reused
     // only after the copies that read them have completed.
     void h2d(void* dst, const void* src, size_t bytes, hipStream_t s);
 
@@ -399,7 +399,7 @@ class Context : public std::enable_shared_from_this<Context> {
     // Uploads of more than UPLOAD_COMMAND and at most UPLOAD_KERNEL bytes are read by a kernel (upload_launch):
     // up to 16 KB a copy command is a small kernel too and as fast (37.3 against 37.1 us for a switch at
     // N = 2^12); beyond, it is a DMA transfer (eight switches at 2^12 181 -> 50 us, 64 relinearizations at
-    // 2^13 175 -> 157 us). Above 1 MB, ciphertexts rather than descriptors, the DMA engine keeps the rate.
+    // 2^13 175 -> 157 us; with one limb more, whose descriptors end 8 bytes into a 16-byte word, 391 -> 146). Above 1 MB, ciphertexts rather than descriptors, the DMA engine keeps the rate.
     static constexpr size_t UPLOAD_COMMAND = 16384, UPLOAD_KERNEL = 1 << 20;
     size_t ring_cap_ = 0, ring_head_ = 0;
     size_t run_off_ = 0, run_len_ = 0;      // the open run

@@ -66,9 +66,43 @@ static void upload_launch_checked() {
     c->h2d(b->ptr, words.data(), words.size() * 8, c->stream());  // and the next one works
 }
 
+// Uploads on the kernel's range of sizes go by the kernel whatever their last bytes, and arrive whole; so do the
+// descriptors of batches of odd and even numbers of limbs.
+static void uploads_of_every_length() {
+    auto c = make(12, 6, 2, 3);
+    hipStream_t s = c->stream();
+    std::vector<u32> words(8192);
+    for (size_t i = 0; i < words.size(); ++i) words[i] = (u32)i * 2654435761u;
+    for (size_t bytes : {16388, 16392, 16396, 16400, 16404, 32760, 32764}) {
+        BufPtr b = c->alloc(bytes / 8 + 1);
+        model::uploads.clear();
+        c->h2d(b->ptr, words.data(), bytes, s);
+        CHECK(model::uploads.size() == 1 && model::uploads[0].kernel, "%zu bytes", bytes);
+        CHECK(hipStreamSynchronize(s) == hipSuccess);
+        CHECK(std::memcmp(b->ptr, words.data(), bytes) == 0, "%zu bytes", bytes);
+    }
+    KskPtr key = ksk_uniform(*c, 5, 0, 1);
+    for (u32 count = 60; count < 64; ++count) {
+        std::vector<PolyPtr> ps;
+        std::vector<const Poly*> in;
+        for (u32 i = 0; i < count; ++i) {
+            ps.push_back(poly_uniform(*c, i % 3 ? 4 : 5, 0, true, i, 0));
+            in.push_back(ps.back().get());
+        }
+        for (u32 pass = 0; pass < 3; ++pass) {
+            model::uploads.clear();
+            ks_switch_batch(*c, in, *key);
+            CHECK(model::uploads.size() == 1);
+            CHECK(model::uploads[0].bytes > 16384 && model::uploads[0].kernel, "%u switches: %zu bytes", count,
+                  model::uploads[0].bytes);
+        }
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
+        {"uploads_of_every_length", uploads_of_every_length},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {
