@@ -955,8 +955,9 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
         targets += 2 * (t.level + 1);
         any_fused |= t.fused;
     }
-    if (!any_fused && !p.compact && targets << (log_n - 12) <= NARROW_IP_TILES && yform_usable(2) &&
-        conv_cols_usable(np, targets, md_variant))
+    // (Tiles are counted only where the register-radix passes, and with them the tiles, exist.)
+    if (!any_fused && !p.compact && yform_usable(2) && conv_cols_usable(np, targets, md_variant) &&
+        targets << (log_n - 12) <= NARROW_IP_TILES)
         return prog_apply_narrow(p, tasks);
     // Several tasks, each under a key of its own: the key words are read once. (A single switch may
     // be followed by another under the same key, which a cached copy serves.)

@@ -99,10 +99,27 @@ static void uploads_of_every_length() {
     }
 }
 
+// Key switches, hoisted rotations, products and rescales are put together at every ring size (undefined shifts of
+// the rules end the program).
+static void programs_at_every_ring_size() {
+    for (u32 log_n = 2; log_n <= 17; ++log_n) {
+        auto c = make(log_n, 4, 2, 2);
+        const u64 g = galois_elt(c->n, 1);
+        Evaluator ev(*c, ksk_uniform(*c, 3, 0, 1), {ksk_uniform(*c, 3, g, 2)});
+        Ct a{{poly_uniform(*c, 3, 0, true, 3, 0), poly_uniform(*c, 3, 0, true, 4, 0)}, 1024.0};
+        ks_switch(*c, *a.comps[0], *ev.relin);
+        ev.rescale(*ev.mul(a, a));
+        if (log_n > 2) ev.rotate(a, 1);
+        ev.hoisted_rotate(a, {0, 1});
+        c->synchronize_all();
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
         {"uploads_of_every_length", uploads_of_every_length},
+        {"programs_at_every_ring_size", programs_at_every_ring_size},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -38,6 +38,7 @@ def exe(tmp_path_factory):
 @pytest.mark.parametrize("check", [
     "upload_launch_checked",
     "uploads_of_every_length",
+    "programs_at_every_ring_size",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
