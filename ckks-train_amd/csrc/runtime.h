@@ -320,6 +320,7 @@ class Context : public std::enable_shared_from_this<Context> {
     // The key-switch candidates of autotune() timed on a caller's batch (autotune.cpp).
     std::string autotune_ks(const std::vector<const Poly*>& ds, const Ksk& key);
     std::string autotune_small(const Poly& d, const Ksk& key);
+    std::vector<u32> tg_candidates(const std::vector<const Poly*>& ds, const Ksk& key, u32 present, bool small) const;
     void set_tuning(const std::string& key, int64_t value);
     int64_t get_tuning(const std::string& key) const;
     // This GPU's fixed workspace (ckh_key_switch_batch_static), looked up at context creation.

@@ -115,11 +115,41 @@ static void programs_at_every_ring_size() {
     }
 }
 
+// Where no candidate is faster the autotuner keeps the present settings, and it times each kernel and grouping of a
+// batch that converts apart once, and no grouping where none is used.
+static void autotuner_keeps_what_is_not_beaten() {
+    const char* keys[] = {"conv_variant", "conv_variant_md", "conv_tg", "fuse_ip", "conv_variant_small", "conv_tg_small",
+                          "fuse_ip_small", "ntt_chunk_fwd", "ntt_chunk_inv"};
+    auto c = make(12, 12, 6, 2);
+    std::map<std::string, int64_t> before;
+    for (const char* k : keys) before[k] = c->get_tuning(k);
+    const std::string all = c->autotune();
+    for (const char* k : keys) CHECK(c->get_tuning(k) == before[k], "%s", k);
+    CHECK(all.find("conv1_") == std::string::npos);
+    CHECK(all.find("_tg16") == std::string::npos, "%s", all.c_str());
+
+    KskPtr key = ksk_uniform(*c, 11, 0, 1);
+    std::vector<PolyPtr> ps;
+    std::vector<const Poly*> batch;
+    for (u32 i = 0; i < 900; ++i) {  // enough tiles for conversions of their own
+        ps.push_back(poly_uniform(*c, 11, 0, true, i, 0));
+        batch.push_back(ps.back().get());
+    }
+    c->set_tuning("conv_tg", 8);
+    const std::string ks = c->autotune_ks(batch, *key);
+    CHECK(c->get_tuning("conv_tg") == 8);
+    CHECK(ks.find("conv0_tg16") != std::string::npos && ks.find("tg24") == std::string::npos, "%s", ks.c_str());
+    c->set_tuning("conv_tg", 32);  // as many as 24 or 16 take here: all
+    CHECK(c->autotune_ks(batch, *key).find("conv0_tg16") == std::string::npos);
+    CHECK(c->get_tuning("conv_tg") == 32);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
         {"uploads_of_every_length", uploads_of_every_length},
         {"programs_at_every_ring_size", programs_at_every_ring_size},
+        {"autotuner_keeps_what_is_not_beaten", autotuner_keeps_what_is_not_beaten},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

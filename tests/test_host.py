@@ -39,6 +39,7 @@ def exe(tmp_path_factory):
     "upload_launch_checked",
     "uploads_of_every_length",
     "programs_at_every_ring_size",
+    "autotuner_keeps_what_is_not_beaten",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
