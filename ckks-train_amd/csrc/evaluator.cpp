@@ -281,9 +281,16 @@ KskPtr ksk_uniform(Context& c, u32 max_level, u64 galois, u64 seed) {
 
 namespace {
 // Scratch words of one key switch at level l: x (L), digits, acc (2 (L + k)), y (2k), z (2L).
-u64 ks_scratch_words(const Context& c, u32 level, bool with_digits) {
+u64 ks_scratch_words(const Context& c, u32 level, bool with_digits, bool with_acc = true) {
     const u64 L = level + 1, k = c.np;
-    return c.n * (L + (with_digits ? c.ndigits(level) * (L + k) : 0) + 2 * (L + k) + 2 * k + 2 * L);
+    return c.n * (L + (with_digits ? c.ndigits(level) * (L + k) : 0) + (with_acc ? 2 * (L + k) : 0) + 2 * k + 2 * L);
+}
+
+// Whether a batch of switches of `limbs` limbs in all takes the apply stage that leaves acc unused.
+bool ks_without_acc(const Context& c, u64 limbs) {
+    const bool small = limbs <= c.small_limbs;
+    if ((small ? c.fuse_ip_s : c.fuse_ip) && c.fuse_ip_possible()) return false;
+    return c.narrow_apply(2 * limbs, small ? c.conv_variant_s : c.md_variant());
 }
 
 struct KsReq {
@@ -304,9 +311,9 @@ void check_switch(const Context& c, const Poly& d, const Ksk& key) {
 }
 
 // The program of a batch of requests (decompose + apply, one launch per stage), its scratch laid
-// out from base (ks_scratch_words per request, in request order).
+// out from base (ks_scratch_words per request, in request order; acc only with with_acc).
 static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
-                          const std::vector<AutJob>* pre = nullptr, bool compact = false) {
+                          const std::vector<AutJob>* pre = nullptr, bool with_acc = true, bool compact = false) {
     u64 limbs = 0;
     for (auto& r : reqs) limbs += r.d->level + 1;
     const bool small = limbs <= c.small_limbs;
@@ -319,7 +326,7 @@ static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
         u64* x = p;
         u64* dig = x + L * c.n;
         u64* acc = dig + (u64)c.ndigits(r.d->level) * (L + k) * c.n;
-        u64* y = acc + 2 * (L + k) * c.n;
+        u64* y = acc + (with_acc ? 2 * (L + k) * c.n : 0);
         u64* z = y + 2 * k * c.n;
         p = z + 2 * L * c.n;
         dec.push_back({r.d->data(), r.d->level, dig, x, false, fuse});
@@ -337,10 +344,12 @@ static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
 // decompose + apply for a batch of requests, in one launch per stage.
 static void run_ks_on(Context& c, const std::vector<KsReq>& reqs, hipStream_t s,
                       const std::vector<AutJob>* pre = nullptr) {
-    u64 total = 0;
-    for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true);
+    u64 total = 0, limbs = 0;
+    for (auto& r : reqs) limbs += r.d->level + 1;
+    const bool with_acc = !ks_without_acc(c, limbs);
+    for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true, with_acc);
     BufPtr scratch = c.alloc(total, s, (u32)reqs.size());
-    c.execute(ks_program(c, reqs, scratch->ptr, pre), s);
+    c.execute(ks_program(c, reqs, scratch->ptr, pre, with_acc), s);
     hip_check(hipGetLastError(), "key switch");
 }
 
@@ -465,7 +474,7 @@ void ks_switch_batch_static(Context& c, const std::vector<const Poly*>& ds, cons
     Program prog = ks_program(c, reqs, (u64*)c.static_scratch);
     const u64 desc_off = (scratch_bytes + 255) & ~(u64)255;
     if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)  // the last bytes of the workspace
-        prog = ks_program(c, reqs, (u64*)c.static_scratch, nullptr, true);
+        prog = ks_program(c, reqs, (u64*)c.static_scratch, nullptr, true, true);
     if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)
         fail(CKH_ERR_INVALID_PARAMS, "batch needs more than the static workspace");
     hipStream_t s = c.stream();
@@ -794,6 +803,19 @@ std::vector<CtPtr> Evaluator::relinearize_batch(const std::vector<const Ct*>& ct
     run_ks(ctx, reqs);
     count(&ckh_op_counter::relins, cts.size());
     return res;
+}
+
+// relinearize_batch of 3-component ciphertexts of the caller's own, their first two components overwritten (the
+// finish reads an addend's word before it writes that word). Key checked by the caller.
+void Evaluator::relinearize_in_place(std::vector<CtPtr>& cts) {
+    std::vector<KsReq> reqs;
+    for (auto& ct : cts) {
+        u64 *c0 = ct->comps[0]->data(), *c1 = ct->comps[1]->data();
+        reqs.push_back({ct->comps[2].get(), relin.get(), c0, c1, c0, c1});
+    }
+    run_ks(ctx, reqs);
+    for (auto& ct : cts) ct->comps.pop_back();
+    count(&ckh_op_counter::relins, cts.size());
 }
 
 CtPtr Evaluator::mul(const Ct& a, const Ct& b) {
@@ -1372,9 +1394,10 @@ std::vector<bool> Evaluator::check_matvec_enc(const Ct& x, const std::vector<con
 CtPtr Evaluator::matvec_enc_run(const Ct& x, const std::vector<const Ct*>& entries, u32 baby, u32 giant, u32 stride,
                                 int32_t offset, const std::vector<bool>& present) {
     if (config.lazy_relin && config.bsgs) {
-        // Every block's products summed at degree 2 in one launch, the blocks relinearized in one
-        // program and rotated in another: the same words and counts as one call each.
-        const std::vector<CtPtr> xs = baby_rotations({{&x, present}}, baby, giant, stride)[0];
+        // The blocks' products summed at degree 2 in one launch, the blocks relinearized in one program
+        // and rotated in another, as many blocks at a time as matvec_enc_workspace_bytes has room for:
+        // the same words and counts as one call each.
+        std::vector<CtPtr> xs = baby_rotations({{&x, present}}, baby, giant, stride)[0];
         std::vector<std::vector<std::pair<const Ct*, const Ct*>>> sums;
         std::vector<int32_t> shifts;
         for (u32 k1 = 0; k1 < giant; ++k1) {
@@ -1385,13 +1408,24 @@ CtPtr Evaluator::matvec_enc_run(const Ct& x, const std::vector<const Ct*>& entri
             sums.push_back(std::move(s));
             shifts.push_back((offset + (int32_t)(baby * k1)) * (int32_t)stride);
         }
-        const std::vector<CtPtr> deg2 = tensor_sums(sums);
-        std::vector<const Ct*> to_relin;
-        for (auto& c : deg2) to_relin.push_back(c.get());
-        const std::vector<CtPtr> blocks = relinearize_batch(to_relin);
-        std::vector<std::pair<const Ct*, int32_t>> to_rotate;
-        for (size_t i = 0; i < blocks.size(); ++i) to_rotate.push_back({blocks[i].get(), shifts[i]});
-        return sum_cts(rotate_batch(to_rotate));
+        u64 copies = 0, rotated = 0;
+        for (u32 k2 = 0; k2 < baby; ++k2) copies += xs[k2] && rotation_elt((int32_t)(k2 * stride)) != 0;
+        for (int32_t sh : shifts) rotated += rotation_elt(sh) != 0;
+        const size_t at_once = enc_blocks_at_once(x.level(), baby, giant, copies, sums.size(), rotated);
+        CtPtr acc;
+        for (size_t b0 = 0; b0 < sums.size(); b0 += at_once) {
+            const size_t b1 = std::min(sums.size(), b0 + at_once);
+            std::vector<CtPtr> blocks = tensor_sums({sums.begin() + b0, sums.begin() + b1});
+            if (b1 == sums.size()) xs.clear();
+            if (sums.size() + rotated == 1) return relinearize(*blocks[0]);  // the result as it is: no third component kept
+            relinearize_in_place(blocks);
+            std::vector<std::pair<const Ct*, int32_t>> to_rotate;
+            for (size_t i = 0; i < blocks.size(); ++i) to_rotate.push_back({blocks[i].get(), shifts[b0 + i]});
+            std::vector<CtPtr> parts = rotate_batch(to_rotate);
+            if (acc) parts.push_back(acc);
+            acc = sum_cts(parts);
+        }
+        return acc;
     }
     if (config.lazy_relin)
         return bsgs(
@@ -1411,14 +1445,34 @@ CtPtr Evaluator::matvec_enc(const Ct& x, const std::vector<const Ct*>& entries, 
     return counted([&] { return matvec_enc_run(x, entries, baby, giant, stride, offset, present); });
 }
 
-// Device bytes one matvec_enc of this engine holds at its peak, an upper estimate: the shared
-// decomposition, the hoisted steps' scratch and rotated copies, a degree-2 product and its sum,
-// one key switch's scratch with its output, and the blocks awaiting their giant rotation.
+// Device bytes one matvec_enc of this engine (in the optimised form) holds at its peak, an upper estimate in
+// whole limbs: the shared decomposition, the hoisted steps' scratch and rotated copies, a degree-2 product and
+// its sum, one key switch's scratch with its output, and the blocks awaiting their giant rotation.
 u64 Evaluator::matvec_enc_workspace_bytes(u32 level, u32 baby, u32 giant) const {
     const u64 q = level + 1, k = ctx.np, nd = ctx.ndigits(level), qp = q + k;
     const u64 limbs = nd * qp + q + (baby - 1) * (2 * qp + 2 * k + 5 * q) + 6 * q +
                       (q + nd * qp + 2 * qp + 2 * k + 2 * q) + 2 * q + 4 * q * giant;
     return limbs * ctx.n * 8;
+}
+
+// How many of `blocks` giant blocks matvec_enc takes at once within matvec_enc_workspace_bytes (equal groups, each
+// a batch). `copies` baby rotations hold a ciphertext of their own, `rotated` blocks have a giant rotation. A
+// block's product takes 3 limbs per limb of the level, its relinearization a switch's scratch beside it, its
+// rotation another and 4 limbs; the copies are freed once the last group's products are queued, and the
+// groups before it leave their sum. 4 x 4 blocks at N = 2^14 (6 limbs) take 208 us at once and 463 us one by
+// one; 2 x 4 at 2^15 (12 limbs) 411 at once and 508 in twos.
+size_t Evaluator::enc_blocks_at_once(u32 level, u32 baby, u32 giant, u64 copies, u64 blocks, u64 rotated) const {
+    const u64 q = level + 1, xs = 2 * q * copies;
+    const u64 room = matvec_enc_workspace_bytes(level, baby, giant) / (ctx.n * 8);
+    auto scratch = [&](u64 m) { return m * ks_scratch_words(ctx, level, true, !ks_without_acc(ctx, m * q)) / ctx.n; };
+    if (std::max({xs + 3 * q * blocks, 3 * q * blocks + scratch(blocks), 3 * q * blocks + 4 * q * rotated + scratch(rotated)}) <=
+        room)
+        return blocks;
+    for (u64 groups = 2; groups < blocks; ++groups) {
+        const u64 m = (blocks + groups - 1) / groups;
+        if (xs + 2 * q + 7 * q * m + scratch(m) <= room) return m;
+    }
+    return 1;
 }
 
 // CudaEvaluator::matvec_enc_batch (crates/ckks-train-cuda/src/evaluator.rs:437-519): every job

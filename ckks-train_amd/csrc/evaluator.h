@@ -154,6 +154,8 @@ class Evaluator {
     };
     std::vector<CtPtr> apply_galois_batch(const std::vector<GaloisItem>& items);
     std::vector<CtPtr> tensor_sums(const std::vector<std::vector<std::pair<const Ct*, const Ct*>>>& sums);
+    void relinearize_in_place(std::vector<CtPtr>& cts);
+    size_t enc_blocks_at_once(u32 level, u32 baby, u32 giant, u64 copies, u64 blocks, u64 rotated) const;
     void check_mod_raise_input(const Ct& ct) const;
     CtPtr raise_ct(const Ct& ct);
     std::vector<bool> check_matvec_enc(const Ct& x, const std::vector<const Ct*>& entries, u32 baby, u32 giant,

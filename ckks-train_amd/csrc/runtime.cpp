@@ -886,6 +886,11 @@ bool Context::conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const {
            (nsrc <= CONV_COLS_ALWAYS || targets << (log_n - 12) <= CONV_COLS_ITEMS);
 }
 
+// (Tiles are counted only where the register-radix passes, and with them the tiles, exist.)
+bool Context::narrow_apply(u64 targets, u32 md_variant) const {
+    return yform_usable(2) && conv_cols_usable(np, targets, md_variant) && targets << (log_n - 12) <= NARROW_IP_TILES;
+}
+
 void Context::add_conv_cols(std::vector<ConvColRef>& refs, u32 plan, const u64* src, u64* out) const {
     const ConvPlan& P = conv_plans_[plan];
     const u32 first = (u32)refs.size();
@@ -955,10 +960,7 @@ void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md
         targets += 2 * (t.level + 1);
         any_fused |= t.fused;
     }
-    // (Tiles are counted only where the register-radix passes, and with them the tiles, exist.)
-    if (!any_fused && !p.compact && yform_usable(2) && conv_cols_usable(np, targets, md_variant) &&
-        targets << (log_n - 12) <= NARROW_IP_TILES)
-        return prog_apply_narrow(p, tasks);
+    if (!any_fused && !p.compact && narrow_apply(targets, md_variant)) return prog_apply_narrow(p, tasks);
     // Several tasks, each under a key of its own: the key words are read once. (A single switch may
     // be followed by another under the same key, which a cached copy serves.)
     std::sort(keys.begin(), keys.end());

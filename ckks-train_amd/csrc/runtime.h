@@ -381,6 +381,8 @@ class Context : public std::enable_shared_from_this<Context> {
     // 24 (768 tiles) 174 against 184; two of 24 (1536 tiles) 307 against 306.
     static constexpr u32 NARROW_IP_TILES = 1024;
     bool conv_cols_usable(u32 nsrc, u64 targets, u32 variant) const;
+    // Whether an apply stage of `targets` Q limbs (both parts; no digit fused) does so: its acc is unused.
+    bool narrow_apply(u64 targets, u32 md_variant) const;
     // Appends the targets of one conversion (plan, first source limb, output polynomial).
     void add_conv_cols(std::vector<ConvColRef>& refs, u32 plan, const u64* src, u64* out) const;
     std::atomic<u64> graph_captures{0}, graph_launches{0};

@@ -144,12 +144,64 @@ static void autotuner_keeps_what_is_not_beaten() {
     CHECK(c->get_tuning("conv_tg") == 32);
 }
 
+// Largest device memory that f holds beyond what was live before, its result included.
+template <class F>
+static u64 peak_of(Context& c, F&& f) {
+    const u64 before = c.live_bytes;
+    u64 peak = 0;
+    model::on_launch = [&] { peak = std::max<u64>(peak, c.live_bytes - before); };
+    f();
+    model::on_launch = nullptr;
+    c.synchronize_all();
+    return peak;
+}
+
+// A product with encrypted diagonals stays within the memory it is admitted by (in the pool that does not round
+// sizes, launched directly; 64 KB for the launches' descriptors).
+static void encrypted_products_stay_within_their_estimate() {
+    const u32 sets[][3] = {{6, 2, 3}, {12, 4, 3}, {24, 6, 4}, {20, 4, 5}};
+    for (auto& s : sets) {
+        auto c = make(12, s[0], s[1], s[2]);
+        c->set_tuning("pool", 0);
+        c->set_tuning("graphs", 0);
+        std::map<u64, KskPtr> keys;
+        for (u32 baby : {1u, 2u, 4u, 8u, 32u})
+            for (u32 giant : {1u, 2u, 4u, 16u, 32u})
+                for (u32 level : {s[0] - 1, s[0] / 2})
+                    for (u32 every : {1u, 3u})
+                        for (int32_t offset : {0, -1}) {
+                            if (offset <= -(int32_t)(baby * giant)) continue;
+                            std::vector<KskPtr> galois;
+                            auto need = [&](int32_t step) {
+                                const u64 g = galois_elt(c->n, step);
+                                if (!keys.count(g)) keys[g] = ksk_uniform(*c, s[0] - 1, g, 7);
+                                galois.push_back(keys[g]);
+                            };
+                            for (u32 k = 1; k < baby; ++k) need((int32_t)k);
+                            for (u32 k = 0; k < giant; ++k) need(offset + (int32_t)(baby * k));
+                            Evaluator ev(*c, ksk_uniform(*c, s[0] - 1, 0, 1), galois);
+                            auto ct = [&] {
+                                return Ct{{poly_uniform(*c, level, 0, true, 3, 0), poly_uniform(*c, level, 0, true, 4, 0)}, 1024.0};
+                            };
+                            const Ct x = ct(), w = ct();
+                            std::vector<const Ct*> entries(baby * giant, nullptr);
+                            for (u32 i = 0; i < baby * giant; i += every) entries[i] = &w;
+                            CtPtr out;
+                            const u64 peak = peak_of(*c, [&] { out = ev.matvec_enc(x, entries, baby, giant, 1, offset); });
+                            const u64 room = ev.matvec_enc_workspace_bytes(level, baby, giant) + 65536;
+                            CHECK(peak <= room, "%u primes, level %u, %u x %u, offset %d: %llu above %llu", s[0], level, baby,
+                                  giant, offset, (unsigned long long)peak, (unsigned long long)room);
+                        }
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
         {"uploads_of_every_length", uploads_of_every_length},
         {"programs_at_every_ring_size", programs_at_every_ring_size},
         {"autotuner_keeps_what_is_not_beaten", autotuner_keeps_what_is_not_beaten},
+        {"encrypted_products_stay_within_their_estimate", encrypted_products_stay_within_their_estimate},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -85,8 +85,11 @@ float elapsed_ms = 1.0f;
 uint64_t records_while_capturing = 0;
 size_t free_bytes = (size_t)1 << 40;
 
+std::function<void()> on_launch;
+
 void kernel() {
     LOCKED;
+    if (on_launch) on_launch();
     if (refuse_launch) {
         refuse_launch = false;
         last_error = hipErrorLaunchFailure;

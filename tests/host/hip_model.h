@@ -11,7 +11,7 @@
 
 #include <cstddef>
 #include <cstdint>
-#include <random>
+#include <functional>
 #include <vector>
 
 namespace model {
@@ -26,6 +26,8 @@ extern bool refuse_launch;              // the next kernel launch is refused (an
 extern float elapsed_ms;                // what hipEventElapsedTime reports
 extern uint64_t records_while_capturing;  // event records on a stream that a caller captures
 extern size_t free_bytes;               // what hipMemGetInfo reports
+
+extern std::function<void()> on_launch;  // called at every kernel launch
 
 void kernel();                          // one launch: counted, or refused
 void queue_copy(void* dst, const void* src, size_t bytes, hipStream_t s);

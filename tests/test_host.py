@@ -40,6 +40,7 @@ def exe(tmp_path_factory):
     "uploads_of_every_length",
     "programs_at_every_ring_size",
     "autotuner_keeps_what_is_not_beaten",
+    "encrypted_products_stay_within_their_estimate",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
