@@ -34,7 +34,7 @@ u64 Server::footprint(const ServedOp& op) const {
     switch (op.kind) {
         case CKH_OP_RELINEARIZE: limbs = ks + 2 * L; break;
         case CKH_OP_HOISTED_ROTATE:
-            limbs = d * (L + k) + L + op.steps.size() * (2 * (L + k) + 2 * k + 2 * L + L + 2 * L);
+            limbs = d * (L + k) + L + op.steps.size() * (2 * (L + k) + 2 * k + 2 * L + 2 * L);
             break;
         default: limbs = 3 * L + ks + 2 * L + 2 * L + 2 * (1 + L); break;
     }

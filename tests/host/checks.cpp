@@ -8,6 +8,7 @@
 
 #include "../../ckks-train_amd/csrc/evaluator.h"
 #include "../../ckks-train_amd/csrc/hostmath.h"
+#include "../../ckks-train_amd/csrc/server.h"
 #include "hip_model.h"
 
 using namespace ckh;
@@ -195,6 +196,54 @@ static void encrypted_products_stay_within_their_estimate() {
     }
 }
 
+// A served request is admitted by the memory it holds: never less (but for descriptors), and hoisted rotations,
+// whose scratch has one form, by just that.
+static void served_requests_are_admitted_by_what_they_hold() {
+    auto c = make(12, 12, 4, 3);
+    c->set_tuning("pool", 0);
+    c->set_tuning("graphs", 0);
+    std::vector<KskPtr> galois;
+    std::vector<int32_t> steps;
+    for (int32_t k = 1; k <= 5; ++k) {
+        galois.push_back(ksk_uniform(*c, 11, galois_elt(c->n, k), 7));
+        steps.push_back(k);
+    }
+    auto ev = std::make_shared<Evaluator>(*c, ksk_uniform(*c, 11, 0, 1), galois);
+    for (u32 level : {11u, 6u, 1u})
+        for (u32 kind : {CKH_OP_RELINEARIZE, CKH_OP_HOISTED_ROTATE, CKH_OP_MUL_RELIN_RESCALE}) {
+            auto ct = [&](u32 comps) {
+                auto r = std::make_shared<Ct>();
+                for (u32 i = 0; i < comps; ++i) r->comps.push_back(poly_uniform(*c, level, 0, true, i, 0));
+                r->scale = 1024.0;
+                return r;
+            };
+            auto op = std::make_shared<ServedOp>();
+            op->kind = kind;
+            op->ev = ev;
+            op->a = ct(kind == CKH_OP_RELINEARIZE ? 3 : 2);
+            op->b = kind == CKH_OP_MUL_RELIN_RESCALE ? ct(2) : nullptr;
+            if (kind == CKH_OP_HOISTED_ROTATE) op->steps = steps;
+            c->synchronize_all();
+            u64 held = 0;
+            ckh_server_stats st{};
+            {
+                ckh_server_config cfg{};
+                cfg.hbm_budget_bytes = 1ull << 40;
+                Server srv(cfg);
+                held = peak_of(*c, [&] {
+                    const u64 ticket = srv.submit(op);
+                    OpPtr done;
+                    while (!srv.poll(ticket, false, done)) c->synchronize_all();
+                    CHECK(done->status == CKH_OK, "%s", done->err.c_str());
+                });
+                st = srv.stats();
+            }
+            CHECK(st.peak_bytes + 65536 >= held, "kind %u: %llu held", kind, (unsigned long long)held);
+            if (kind == CKH_OP_HOISTED_ROTATE)
+                CHECK(st.peak_bytes <= held, "%llu counted, %llu held", (unsigned long long)st.peak_bytes, (unsigned long long)held);
+        }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
@@ -202,6 +251,7 @@ int main(int argc, char** argv) {
         {"programs_at_every_ring_size", programs_at_every_ring_size},
         {"autotuner_keeps_what_is_not_beaten", autotuner_keeps_what_is_not_beaten},
         {"encrypted_products_stay_within_their_estimate", encrypted_products_stay_within_their_estimate},
+        {"served_requests_are_admitted_by_what_they_hold", served_requests_are_admitted_by_what_they_hold},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

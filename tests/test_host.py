@@ -41,6 +41,7 @@ def exe(tmp_path_factory):
     "programs_at_every_ring_size",
     "autotuner_keeps_what_is_not_beaten",
     "encrypted_products_stay_within_their_estimate",
+    "served_requests_are_admitted_by_what_they_hold",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
