@@ -348,7 +348,7 @@ static void run_ks_on(Context& c, const std::vector<KsReq>& reqs, hipStream_t s,
     for (auto& r : reqs) limbs += r.d->level + 1;
     const bool with_acc = !ks_without_acc(c, limbs);
     for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true, with_acc);
-    BufPtr scratch = c.alloc(total, s, (u32)reqs.size());
+    BufPtr scratch = c.alloc(total, s);
     c.execute(ks_program(c, reqs, scratch->ptr, pre, with_acc), s);
     hip_check(hipGetLastError(), "key switch");
 }
@@ -700,7 +700,7 @@ CtPtr Evaluator::mul_no_relin(const Ct& a, const Ct& b) {
     check_mul_operands(a, b);
     const u32 level = a.level();
     const u64 Lw = (u64)(level + 1) * ctx.n;
-    BufPtr out = ctx.alloc_polys(3 * Lw, 3);
+    BufPtr out = ctx.alloc(3 * Lw);
     ctx.tick_launch();
     tensor_launch({a.comps[0]->data(), a.comps[1]->data(), b.comps[0]->data(), b.comps[1]->data()}, out->ptr, level + 1,
                   ctx.d_pc, ctx.log_n, ctx.stream());
@@ -721,7 +721,7 @@ std::vector<CtPtr> Evaluator::tensor_sums(const std::vector<std::vector<std::pai
         total += 3 * (u64)(s[0].first->level() + 1) * ctx.n;
         products += s.size();
     }
-    BufPtr out = ctx.alloc_polys(total, 3 * sums.size());
+    BufPtr out = ctx.alloc(total);
     std::vector<TensorJob> jobs;
     std::vector<TensorTerm> terms;
     u64 off = 0;
@@ -789,7 +789,7 @@ std::vector<CtPtr> Evaluator::relinearize_batch(const std::vector<const Ct*>& ct
     }
     std::vector<CtPtr> res;
     if (cts.empty()) return res;
-    BufPtr out = ctx.alloc_polys(total, 2 * cts.size());
+    BufPtr out = ctx.alloc(total);
     std::vector<KsReq> reqs;
     u64 off = 0;
     for (const Ct* ct : cts) {
@@ -952,8 +952,8 @@ std::vector<CtPtr> Evaluator::hoisted_rotate(const Ct& ct, const std::vector<int
     BufPtr digs = ctx.alloc(nd * dw + L * n);
     ctx.decompose({{ct.comps[1]->data(), level, digs->ptr, digs->ptr + nd * dw}}, s);
     const u64 per = (2 * (L + k) + 2 * k + 2 * L) * n;  // acc, y, z
-    BufPtr scratch = ctx.alloc_polys(per * nontrivial, nontrivial);
-    BufPtr out = ctx.alloc_polys(2 * L * n * nontrivial, 2 * nontrivial);
+    BufPtr scratch = ctx.alloc(per * nontrivial);
+    BufPtr out = ctx.alloc(2 * L * n * nontrivial);
     std::vector<ApplyTask> tasks;
     u32 t = 0;
     for (size_t i = 0; i < steps.size(); ++i) {
@@ -1092,7 +1092,7 @@ std::vector<CtPtr> Evaluator::apply_galois_batch(const std::vector<GaloisItem>& 
     std::vector<CtPtr> res;
     u64 total = 0;
     for (const GaloisItem& it : items) total += 4 * (u64)(it.ct->level() + 1) * ctx.n;
-    BufPtr buf = ctx.alloc_polys(total, 4 * items.size());  // per item: sigma(c1), sigma(c0), kb + sigma(c0), ka
+    BufPtr buf = ctx.alloc(total);  // per item: sigma(c1), sigma(c0), kb + sigma(c0), ka
     std::vector<KsReq> reqs;
     std::vector<Poly> dpolys;
     dpolys.reserve(items.size());
@@ -1160,7 +1160,7 @@ CtPtr Evaluator::sum_cts(const std::vector<CtPtr>& cts) {
     }
     const u32 level = c0.level();
     const u64 L = level + 1, n = ctx.n, nc = c0.comps.size();
-    BufPtr out = ctx.alloc_polys(nc * L * n, nc);
+    BufPtr out = ctx.alloc(nc * L * n);
     std::vector<AddSumJob> jobs;
     std::vector<const u64*> xs;
     for (u64 comp = 0; comp < nc; ++comp)

@@ -318,12 +318,13 @@ void Context::trim_pool(u64 keep_bytes) {
     hip_check(hipMemPoolTrimTo(dp, keep_bytes), "hipMemPoolTrimTo");
 }
 
-BufPtr Context::alloc(size_t words, hipStream_t s, u32 polys) {
+BufPtr Context::alloc(size_t words, hipStream_t s) {
     void* p = nullptr;
     size_t bytes = std::max<size_t>(words, 1) * sizeof(u64), cls = 0;
     if (fail_alloc_after.load() >= 0) {
+        const int64_t polys = std::max<int64_t>(1, (words + nq * n - 1) / (nq * n));
         const int64_t left = fail_alloc_after.fetch_sub(polys);
-        if (left >= 0 && left < (int64_t)polys) {
+        if (left >= 0 && left < polys) {
             fail_alloc_after = -1;
             fail(CKH_ERR_DEVICE, "out of device memory (injected allocation failure)");
         }

@@ -238,10 +238,8 @@ class Context : public std::enable_shared_from_this<Context> {
     // other stream once an event recorded after its last use has completed; 0 = the device's
     // default stream-ordered pool with the runtime's reuse rules (which may hand a block to
     // another stream before its free has run, behind a dependency the runtime inserts).
-    // polys: the polynomials the buffer holds, for the allocation-failure hook.
-    BufPtr alloc(size_t words, hipStream_t s, u32 polys = 1);
+    BufPtr alloc(size_t words, hipStream_t s);
     BufPtr alloc(size_t words) { return alloc(words, stream()); }
-    BufPtr alloc_polys(size_t words, u64 polys) { return alloc(words, stream(), (u32)polys); }
     void free_buffer(Buffer* b);
     u32 pool_mode = 1;
     // The pool's bytes in use, its release threshold (bytes kept reserved after a
@@ -251,10 +249,10 @@ class Context : public std::enable_shared_from_this<Context> {
     u64 pool_unused_reserve();  // reserved by the pool but not in use
     void set_pool_release_threshold(u64 bytes);
     void trim_pool(u64 keep_bytes);
-    // Test hook (tuning key "fail_alloc_after"): the n-th allocation from now fails with a device
-    // error, as an out-of-memory would; negative = off. A buffer of several polynomials counts as
-    // one allocation for each, so that a failure can be placed inside a composite operation whatever
-    // buffers it shares.
+    // Test hook (tuning key "fail_alloc_after"): the n-th polynomial's worth of device memory from now
+    // (nq limbs; every buffer counts at least once) fails its buffer's allocation with a device error, as
+    // an out-of-memory would; negative = off. Counted by size, a failure can be placed inside a composite
+    // operation whatever buffers it shares.
     std::atomic<int64_t> fail_alloc_after{-1};
     // Test hooks as the reference's failing backend (crates/ckks-train-cuda/tests/cases/
     // failing.rs:34-67): "fail_launch_after" makes the n-th primitive launch from now (a

@@ -117,10 +117,11 @@ ckh_status ckh_autotune_ks(ckh_context *ctx, uint32_t n, const ckh_poly *const *
  * wait depth and workgroups per CU). Read only (ckh_get_tuning): "xcds", "stat_mallocs",
  * "stat_malloc_us", "stat_oom", "stat_cached_bytes". Test hooks, as the reference's failing
  * backend (crates/ckks-train-cuda/tests/cases/failing.rs:34-67), negative = off:
- * "fail_alloc_after" (the n-th device allocation from now fails with CKH_ERR_DEVICE, as an
- * out-of-memory would; a buffer of several polynomials counts once for each); "fail_launch_after" (the n-th launch from now, counted per program,
- * elementwise kernel or automorphism, fails with CKH_ERR_DEVICE before anything of it is queued;
- * the hook disarms itself when it fires); "fail_upload" (1 = every upload of polynomial,
+ * "fail_alloc_after" (the allocation that reaches the n-th polynomial's worth of device memory from
+ * now, nq limbs each and a smaller buffer one, fails with CKH_ERR_DEVICE, as an out-of-memory
+ * would); "fail_launch_after" (the n-th launch from now, counted per program, elementwise kernel or
+ * automorphism, fails with CKH_ERR_DEVICE before anything of it is queued); both hooks disarm
+ * themselves when they fire; "fail_upload" (1 = every upload of polynomial,
  * ciphertext or key limbs fails with CKH_ERR_DEVICE). Setting a hook keeps captured plans. */
 ckh_status ckh_set_tuning(ckh_context *ctx, const char *key, int64_t value);
 /* CudaDevice::pool_used_memory / set_pool_release_threshold / trim_pool

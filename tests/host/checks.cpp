@@ -244,6 +244,51 @@ static void served_requests_are_admitted_by_what_they_hold() {
         }
 }
 
+// The allocation-failure hook counts what a call allocates in polynomials' worths (nq limbs, a smaller buffer one):
+// armed within that count every call fails, and is disarmed; armed after it the call succeeds.
+static void allocation_hook_counts_by_size() {
+    auto c = make(12, 6, 2, 3);
+    c->set_tuning("pool", 0);
+    c->set_tuning("graphs", 0);
+    std::vector<KskPtr> galois;
+    for (int32_t k : {1, 2, 3, 4}) galois.push_back(ksk_uniform(*c, 5, galois_elt(c->n, k), 7));
+    Evaluator ev(*c, ksk_uniform(*c, 5, 0, 1), galois);
+    Ct a, d;
+    for (u32 i = 0; i < 3; ++i) d.comps.push_back(poly_uniform(*c, 5, 0, true, i, 0));
+    a.comps = {d.comps[0], d.comps[1]};
+    a.scale = d.scale = 1024.0;
+    const std::vector<const Ct*> three(3, &d), entries(8, &a);
+    const std::function<void()> calls[] = {
+        [&] { ks_switch(*c, *a.comps[0], *ev.relin); },
+        [&] { ev.relinearize_batch(three); },
+        [&] { ev.hoisted_rotate(a, {1, 2, 3}); },
+        [&] { ev.hoisted_rotate_batch({{&a, {1, 2}}, {&a, {3}}}); },
+        [&] { ev.rotate_batch({{&a, 1}, {&a, 4}}); },
+        [&] { ev.rescale(*ev.mul(a, a)); },
+        [&] { ev.matvec_enc(a, entries, 4, 2, 1, 0); },
+    };
+    const u64 unit = 6 * c->n * 8;
+    for (auto& call : calls) {
+        u64 total = 0;
+        model::on_malloc = [&](size_t bytes) { total += std::max<u64>(1, (bytes + unit - 1) / unit); };
+        call();
+        model::on_malloc = nullptr;
+        for (u64 at = 0; at <= total; ++at) {
+            c->fail_alloc_after = (int64_t)at;
+            bool failed = false;
+            try {
+                call();
+            } catch (const Error& e) {
+                failed = e.status == CKH_ERR_DEVICE;
+                CHECK(c->fail_alloc_after == -1);
+            }
+            CHECK(failed == (at < total), "call %zu at %llu of %llu", (size_t)(&call - calls), (unsigned long long)at,
+                  (unsigned long long)total);
+            c->fail_alloc_after = -1;
+        }
+    }
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
@@ -252,6 +297,7 @@ int main(int argc, char** argv) {
         {"autotuner_keeps_what_is_not_beaten", autotuner_keeps_what_is_not_beaten},
         {"encrypted_products_stay_within_their_estimate", encrypted_products_stay_within_their_estimate},
         {"served_requests_are_admitted_by_what_they_hold", served_requests_are_admitted_by_what_they_hold},
+        {"allocation_hook_counts_by_size", allocation_hook_counts_by_size},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -86,6 +86,7 @@ uint64_t records_while_capturing = 0;
 size_t free_bytes = (size_t)1 << 40;
 
 std::function<void()> on_launch;
+std::function<void(size_t)> on_malloc;
 
 void kernel() {
     LOCKED;
@@ -222,6 +223,7 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
 
 hipError_t hipMalloc(void** p, size_t bytes) {
     LOCKED;
+    if (model::on_malloc) model::on_malloc(bytes);
     *p = reserve(bytes);
     return *p ? hipSuccess : fail_with(hipErrorOutOfMemory);
 }

@@ -28,6 +28,7 @@ extern uint64_t records_while_capturing;  // event records on a stream that a ca
 extern size_t free_bytes;               // what hipMemGetInfo reports
 
 extern std::function<void()> on_launch;  // called at every kernel launch
+extern std::function<void(size_t)> on_malloc;  // called with the bytes of every device allocation
 
 void kernel();                          // one launch: counted, or refused
 void queue_copy(void* dst, const void* src, size_t bytes, hipStream_t s);

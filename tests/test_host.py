@@ -42,6 +42,7 @@ def exe(tmp_path_factory):
     "autotuner_keeps_what_is_not_beaten",
     "encrypted_products_stay_within_their_estimate",
     "served_requests_are_admitted_by_what_they_hold",
+    "allocation_hook_counts_by_size",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
