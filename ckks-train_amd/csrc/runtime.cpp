@@ -162,8 +162,18 @@ static size_t size_class(size_t b) {
     return (c + 4095) & ~(size_t)4095;
 }
 
-// A mark covering every free queued on s so far.
+// Whether a caller is capturing s (ckh_stream_handle): an event recorded there now would join the caller's graph and
+// say nothing of the work queued before the capture.
+static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return true;
+}
+
+// A mark covering every free queued on s so far (none while s is being captured).
 void Context::mark_record(Mark& m, hipStream_t s) {
+    if (capturing(s)) return;
     if (!m.ev && hipEventCreateWithFlags(&m.ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
         m.ev = nullptr;

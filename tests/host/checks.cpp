@@ -4,6 +4,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <random>
 #include <string>
 
 #include "../../ckks-train_amd/csrc/evaluator.h"
@@ -289,6 +290,63 @@ static void allocation_hook_counts_by_size() {
     }
 }
 
+// Memory written by copies still queued on one stream goes to no other stream's buffer, at random steps of both
+// streams; with `capture`, while a caller captures the first stream from time to time.
+static void cached_blocks(bool capture) {
+    auto c = make(12, 6, 2, 3, 2);
+    std::mt19937 g(5);
+    hipStream_t s[2];
+    for (u32 i = 0; i < 2; ++i) {
+        c->set_stream(i);
+        s[i] = c->stream();
+    }
+    const size_t words = 4096;
+    std::vector<u64> src[2] = {std::vector<u64>(words, 1), std::vector<u64>(words, 2)};
+    u64 reused = 0;
+    bool capturing = false;
+    std::map<u64*, u32> last;  // the stream that used a block last
+    struct Held {
+        BufPtr b;
+        u32 stream;
+    };
+    std::vector<Held> held;
+    for (u32 round = 0; round < 20000; ++round) {
+        if (capture && g() % 16 == 0) model::set_capturing(s[0], capturing = !capturing);
+        const u32 i = capturing ? 1 : g() % 2;
+        c->set_stream(i);
+        if (held.size() == 12 || g() % 2) {  // a release, on the stream that used the buffer
+            for (size_t k = 0; k < held.size(); ++k)
+                if (held[k].stream == i) {
+                    held.erase(held.begin() + k);
+                    break;
+                }
+        } else {
+            BufPtr b = c->alloc(words);
+            auto it = last.find(b->ptr);
+            if (it != last.end() && it->second != i) {
+                // the copies that the other stream queued on this block have all run
+                ++reused;
+                CHECK(b->ptr[0] == it->second + 1 && b->ptr[words - 1] == it->second + 1, "round %u", round);
+            }
+            if (it == last.end() || it->second != i) std::memset(b->ptr, 0xff, words * 8);
+            last[b->ptr] = i;
+            model::queue_copy(b->ptr, src[i].data(), words * 8, s[i]);
+            held.push_back({b, i});
+        }
+        for (u32 k = g() % 3; k > 0; --k) model::step(s[g() % 2]);
+        if (g() % 64 == 0) {
+            while (model::step(s[0])) {}
+            while (model::step(s[1])) {}
+        }
+    }
+    if (capturing) model::set_capturing(s[0], false);
+    CHECK(reused > 100, "%llu", (unsigned long long)reused);
+    CHECK(model::records_while_capturing == 0);
+    c->synchronize_all();
+}
+static void cached_blocks_change_streams_after_their_use() { cached_blocks(false); }
+static void cached_blocks_under_a_capture() { cached_blocks(true); }
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
@@ -298,6 +356,8 @@ int main(int argc, char** argv) {
         {"encrypted_products_stay_within_their_estimate", encrypted_products_stay_within_their_estimate},
         {"served_requests_are_admitted_by_what_they_hold", served_requests_are_admitted_by_what_they_hold},
         {"allocation_hook_counts_by_size", allocation_hook_counts_by_size},
+        {"cached_blocks_change_streams_after_their_use", cached_blocks_change_streams_after_their_use},
+        {"cached_blocks_under_a_capture", cached_blocks_under_a_capture},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -83,6 +83,7 @@ uint64_t launches = 0;
 bool refuse_launch = false;
 float elapsed_ms = 1.0f;
 uint64_t records_while_capturing = 0;
+uint64_t destroyed_graphs = 0;
 size_t free_bytes = (size_t)1 << 40;
 
 std::function<void()> on_launch;
@@ -274,7 +275,10 @@ hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, c
 }
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { OK; }
 hipError_t hipGraphDestroy(hipGraph_t) { OK; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t) { OK; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) {
+    ++model::destroyed_graphs;
+    OK;
+}
 }
 
 // ------------------------------------------------------------------ the library's kernels

@@ -25,6 +25,7 @@ extern uint64_t launches;               // kernel launches so far
 extern bool refuse_launch;              // the next kernel launch is refused (and the flag cleared)
 extern float elapsed_ms;                // what hipEventElapsedTime reports
 extern uint64_t records_while_capturing;  // event records on a stream that a caller captures
+extern uint64_t destroyed_graphs;       // executable graphs destroyed so far
 extern size_t free_bytes;               // what hipMemGetInfo reports
 
 extern std::function<void()> on_launch;  // called at every kernel launch

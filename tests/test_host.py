@@ -43,6 +43,8 @@ def exe(tmp_path_factory):
     "encrypted_products_stay_within_their_estimate",
     "served_requests_are_admitted_by_what_they_hold",
     "allocation_hook_counts_by_size",
+    "cached_blocks_change_streams_after_their_use",
+    "cached_blocks_under_a_capture",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
