@@ -113,7 +113,8 @@ Context::Context(int ordinal, const ckh_params& p, u32 n_streams) {
 Context::~Context() {
     (void)hipSetDevice(device);
     for (auto s : streams_) (void)hipStreamSynchronize(s);
-    for (auto& b : ring_busy_) (void)hipEventDestroy(b.ev);
+    for (auto& b : ring_busy_)
+        if (b.ev) (void)hipEventDestroy(b.ev);
     for (auto e : ring_events_) (void)hipEventDestroy(e);
     if (ring_) (void)hipHostFree(ring_);
     for (auto& pl : plans_) {
@@ -427,47 +428,68 @@ BufPtr Context::upload_blob(const void* host, size_t bytes, hipStream_t s) {
     return b;
 }
 
+// Whether b's event stands: recorded when its run was closed or, for a stream that a caller was capturing
+// then, at the first call after the capture has ended.
+bool Context::ring_event(Staged& b) {
+    if (b.ev) return true;
+    if (capturing(b.s)) return false;
+    hipEvent_t ev;
+    if (ring_events_.empty()) {
+        hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
+    } else {
+        ev = ring_events_.back();
+        ring_events_.pop_back();
+    }
+    b.ev = ev;
+    hip_check(hipEventRecord(ev, b.s), "event");
+    return true;
+}
+
 // One completion event per stream that copied from the open run; the run's slots are busy until all
 // of them have completed.
 void Context::ring_close_run() {
     for (hipStream_t s : run_streams_) {
-        hipEvent_t ev;
-        if (ring_events_.empty()) {
-            hip_check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event");
-        } else {
-            ev = ring_events_.back();
-            ring_events_.pop_back();
-        }
-        hip_check(hipEventRecord(ev, s), "event");
-        ring_busy_.push_back({run_off_, run_len_, ev});
+        ring_busy_.push_back({run_off_, run_len_, nullptr, s});
+        ring_event(ring_busy_.back());
     }
     run_streams_.clear();
     run_len_ = 0;
 }
 
 // A ring slot of len bytes: slots are handed out in address order, wrapping at the end; a run
-// still read by an unfinished copy (the oldest busy runs, from the previous lap) is waited for.
+// still read by an unfinished copy (the oldest busy runs, from the previous lap) is waited for, one
+// whose stream is being captured passed over.
 size_t Context::ring_reserve(size_t len) {
     len = (len + 255) & ~(size_t)255;
-    if (ring_head_ + len > ring_cap_) {
-        ring_close_run();
-        ring_head_ = 0;
-    }
-    const size_t off = ring_head_;
-    ring_head_ += len;
-    if (run_streams_.empty()) run_off_ = off;
-    run_len_ = ring_head_ - run_off_;
-    while (!ring_busy_.empty()) {
-        Staged& b = ring_busy_.front();
-        const bool overlaps = b.off < off + len && off < b.off + b.len;
-        if (!overlaps && hipEventQuery(b.ev) != hipSuccess) break;
-        if (overlaps) hip_check(hipEventSynchronize(b.ev), "staging ring");
-        ring_events_.push_back(b.ev);
+    while (!ring_busy_.empty() && ring_event(ring_busy_.front()) && hipEventQuery(ring_busy_.front().ev) == hipSuccess) {
+        ring_events_.push_back(ring_busy_.front().ev);
         ring_busy_.pop_front();
     }
-    for (const Staged& b : ring_busy_)  // a later busy run can overlap only after a wrap
-        if (b.off < off + len && off < b.off + b.len) hip_check(hipEventSynchronize(b.ev), "staging ring");
-    return off;
+    for (u32 laps = 0;;) {
+        if (ring_head_ + len > ring_cap_) {
+            if (++laps == 3) fail(CKH_ERR_DEVICE, "the staging ring is held by streams being captured");
+            ring_close_run();
+            ring_head_ = 0;
+        }
+        const size_t off = ring_head_;
+        size_t past = 0;
+        for (Staged& b : ring_busy_)
+            if (b.off < off + len && off < b.off + b.len) {
+                if (ring_event(b))
+                    hip_check(hipEventSynchronize(b.ev), "staging ring");
+                else
+                    past = std::max(past, b.off + b.len);
+            }
+        if (past) {
+            ring_close_run();
+            ring_head_ = past;
+            continue;
+        }
+        ring_head_ += len;
+        if (run_streams_.empty()) run_off_ = off;
+        run_len_ = ring_head_ - run_off_;
+        return off;
+    }
 }
 
 void Context::h2d(void* dst, const void* src, size_t bytes, hipStream_t s) {

@@ -391,7 +391,8 @@ class Context : public std::enable_shared_from_this<Context> {
     // RING_RUN bytes, then takes one event per stream that copied from it.
     struct Staged {
         size_t off, len;
-        hipEvent_t ev;
+        hipEvent_t ev;  // null: not recorded yet, the stream was being captured
+        hipStream_t s;
     };
     static constexpr size_t RING_RUN = (size_t)1 << 20;
     std::mutex ring_mu_;
@@ -408,6 +409,7 @@ class Context : public std::enable_shared_from_this<Context> {
     std::deque<Staged> ring_busy_;
     std::vector<hipEvent_t> ring_events_;
     size_t ring_reserve(size_t len);
+    bool ring_event(Staged& b);
     void ring_close_run();
     struct Plan {
         hipStream_t s = nullptr;

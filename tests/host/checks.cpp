@@ -347,6 +347,53 @@ static void cached_blocks(bool capture) {
 static void cached_blocks_change_streams_after_their_use() { cached_blocks(false); }
 static void cached_blocks_under_a_capture() { cached_blocks(true); }
 
+// Staged uploads of two streams arrive whole over many laps of the ring, at random steps of both streams; with
+// `capture`, while a caller captures the first stream from time to time.
+static void staged_uploads(bool capture) {
+    auto c = make(12, 6, 2, 3, 2);
+    std::mt19937 g(6);
+    hipStream_t s[2];
+    for (u32 i = 0; i < 2; ++i) {
+        c->set_stream(i);
+        s[i] = c->stream();
+    }
+    struct Sent {
+        BufPtr b;
+        size_t words;
+        u64 tag;
+        u32 stream;
+    };
+    std::vector<Sent> sent;
+    bool capturing = false;
+    auto verify = [&] {
+        for (u32 i = 0; i < 2; ++i) CHECK(hipStreamSynchronize(s[i]) == hipSuccess);
+        for (const Sent& x : sent)
+            for (size_t w = 0; w < x.words; ++w) CHECK(x.b->ptr[w] == x.tag + w, "word %zu of upload %llu", w, (unsigned long long)x.tag);
+        sent.clear();
+    };
+    size_t total = 0;
+    for (u32 round = 0; total < ((size_t)400 << 20); ++round) {
+        if (capture && g() % 24 == 0) model::set_capturing(s[0], capturing = !capturing);
+        const u32 i = capturing ? 1 : g() % 2;
+        c->set_stream(i);
+        const size_t words = g() % 8 == 0 ? 1 + g() % 700000 : 1 + g() % 20000;
+        std::vector<u64> src(words);
+        const u64 tag = (u64)round << 32;
+        for (size_t w = 0; w < words; ++w) src[w] = tag + w;
+        BufPtr b = c->alloc(words);
+        c->h2d(b->ptr, src.data(), words * 8, s[i]);
+        total += words * 8;
+        sent.push_back({b, words, tag, i});
+        for (u32 k = g() % 3; k > 0; --k) model::step(s[g() % 2]);
+        if (!capturing && g() % 200 == 0) verify();
+    }
+    if (capturing) model::set_capturing(s[0], false);
+    verify();
+    CHECK(model::records_while_capturing == 0);
+}
+static void staged_uploads_of_two_streams() { staged_uploads(false); }
+static void staged_uploads_under_a_capture() { staged_uploads(true); }
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
@@ -358,6 +405,8 @@ int main(int argc, char** argv) {
         {"allocation_hook_counts_by_size", allocation_hook_counts_by_size},
         {"cached_blocks_change_streams_after_their_use", cached_blocks_change_streams_after_their_use},
         {"cached_blocks_under_a_capture", cached_blocks_under_a_capture},
+        {"staged_uploads_of_two_streams", staged_uploads_of_two_streams},
+        {"staged_uploads_under_a_capture", staged_uploads_under_a_capture},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -45,6 +45,8 @@ def exe(tmp_path_factory):
     "allocation_hook_counts_by_size",
     "cached_blocks_change_streams_after_their_use",
     "cached_blocks_under_a_capture",
+    "staged_uploads_of_two_streams",
+    "staged_uploads_under_a_capture",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
