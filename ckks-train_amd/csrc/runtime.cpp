@@ -124,6 +124,7 @@ Context::~Context() {
     }
     plans_.clear();
     for (auto& pl : retired_) {  // every stream was synchronized above
+        if (pl->desc) (void)hipFreeAsync(pl->desc, pl->s);
         if (pl->done) (void)hipEventDestroy(pl->done);
         if (pl->exec) (void)hipGraphExecDestroy(pl->exec);
     }
@@ -787,28 +788,37 @@ void Context::execute(const Program& p, hipStream_t s) {
     run(p, (const uint8_t*)d->ptr, s);
 }
 
-// Evicts plan i without waiting: its descriptor buffer returns to the pool in its stream's
-// order (after the last replay), and the executable graph and event are destroyed once that
-// replay has finished (retired until then, swept by later calls).
+// Queues an evicted plan's end on its stream: its descriptor buffer returns to the pool after the last replay, and
+// an event tells when that replay has finished. False while a caller is capturing the stream.
+bool Context::retire_plan(Plan& pl) {
+    if (capturing(pl.s)) return false;
+    if (pl.desc) (void)hipFreeAsync(pl.desc, pl.s);
+    pl.desc = nullptr;
+    if (pl.exec && (hipEventCreateWithFlags(&pl.done, hipEventDisableTiming) != hipSuccess ||
+                    hipEventRecord(pl.done, pl.s) != hipSuccess)) {
+        (void)hipGetLastError();
+        (void)hipStreamSynchronize(pl.s);
+    }
+    pl.retired = true;
+    return true;
+}
+
+// Evicts plan i without waiting: the executable graph and event are destroyed once the last replay
+// has finished (retired until then, swept by later calls).
 void Context::drop_plan(size_t i) {
     std::unique_ptr<Plan> pl = std::move(plans_[i]);
     plans_.erase(plans_.begin() + i);
-    if (pl->desc) (void)hipFreeAsync(pl->desc, pl->s);
-    pl->desc = nullptr;
-    if (!pl->exec) return;
-    if (hipEventCreateWithFlags(&pl->done, hipEventDisableTiming) != hipSuccess || hipEventRecord(pl->done, pl->s) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipStreamSynchronize(pl->s);
-    }
-    retired_.push_back(std::move(pl));
+    if (!retire_plan(*pl) || pl->exec) retired_.push_back(std::move(pl));
 }
 
-// Destroys the retired plans whose last replay has finished (wait: all of them, after it).
+// Destroys the retired plans whose last replay has finished (wait: all of them, after it, but for those whose
+// stream is being captured).
 void Context::sweep_retired(bool wait) {
     for (size_t i = 0; i < retired_.size();) {
         Plan& pl = *retired_[i];
-        if (wait && pl.done) (void)hipEventSynchronize(pl.done);
-        if (wait || !pl.done || hipEventQuery(pl.done) != hipErrorNotReady) {
+        const bool marked = pl.retired || retire_plan(pl);
+        if (marked && wait && pl.done) (void)hipEventSynchronize(pl.done);
+        if (marked && (wait || !pl.done || hipEventQuery(pl.done) != hipErrorNotReady)) {
             if (pl.done) (void)hipEventDestroy(pl.done);
             if (pl.exec) (void)hipGraphExecDestroy(pl.exec);
             retired_.erase(retired_.begin() + i);

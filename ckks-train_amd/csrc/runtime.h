@@ -419,6 +419,7 @@ class Context : public std::enable_shared_from_this<Context> {
                                // context alive)
         hipGraphExec_t exec = nullptr;
         hipEvent_t done = nullptr;  // recorded when the plan is evicted, after its last replay
+        bool retired = false;       // evicted and its end queued
         u64 last_use = 0;
     };
     std::mutex plan_mu_;
@@ -428,6 +429,7 @@ class Context : public std::enable_shared_from_this<Context> {
     void sweep_retired(bool wait);
     u64 plan_clock_ = 0;
     bool execute_graph(const Program& p, hipStream_t s);
+    bool retire_plan(Plan& pl);
     void drop_plan(size_t i);
 
    public:

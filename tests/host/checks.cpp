@@ -394,6 +394,37 @@ static void staged_uploads(bool capture) {
 static void staged_uploads_of_two_streams() { staged_uploads(false); }
 static void staged_uploads_under_a_capture() { staged_uploads(true); }
 
+// A plan evicted while a caller captures its stream leaves nothing in that capture, and goes once it has ended.
+static void plans_evicted_under_a_capture() {
+    auto c = make(12, 6, 2, 3, 2);
+    c->set_tuning("graph_cache", 1);
+    KskPtr key = ksk_uniform(*c, 5, 0, 1);
+    std::vector<PolyPtr> ps;
+    std::vector<const Poly*> in;
+    for (u32 i = 0; i < 4; ++i) {
+        ps.push_back(poly_uniform(*c, 5, 0, true, i, 0));
+        in.push_back(ps.back().get());
+    }
+    c->set_stream(0);
+    hipStream_t s0 = c->stream();
+    for (u32 k = 0; k < 3; ++k) ks_switch_batch(*c, in, *key);  // seen, captured, replayed
+    CHECK(c->graph_launches == 2);
+    const uint64_t queued = model::pending(s0);
+    model::set_capturing(s0, true);
+    c->set_stream(1);
+    for (u32 k = 0; k < 3; ++k) ks_switch_batch(*c, in, *key);
+    CHECK(c->graph_launches == 4);
+    CHECK(model::records_while_capturing == 0 && model::pending(s0) == queued);
+    CHECK(model::destroyed_graphs == 0);
+    model::set_capturing(s0, false);
+    for (u32 k = 0; k < 3; ++k) {  // swept once its stream has finished
+        c->synchronize_all();
+        ks_switch_batch(*c, in, *key);
+    }
+    CHECK(model::destroyed_graphs == 1);
+    c->set_stream(0);
+}
+
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {
         {"upload_launch_checked", upload_launch_checked},
@@ -407,6 +438,7 @@ int main(int argc, char** argv) {
         {"cached_blocks_under_a_capture", cached_blocks_under_a_capture},
         {"staged_uploads_of_two_streams", staged_uploads_of_two_streams},
         {"staged_uploads_under_a_capture", staged_uploads_under_a_capture},
+        {"plans_evicted_under_a_capture", plans_evicted_under_a_capture},
     };
     auto it = argc == 2 ? checks.find(argv[1]) : checks.end();
     if (it == checks.end()) {

@@ -47,6 +47,7 @@ def exe(tmp_path_factory):
     "cached_blocks_under_a_capture",
     "staged_uploads_of_two_streams",
     "staged_uploads_under_a_capture",
+    "plans_evicted_under_a_capture",
 ])
 def test_host(exe, check):
     r = subprocess.run([exe, check], capture_output=True, text=True, timeout=300)
