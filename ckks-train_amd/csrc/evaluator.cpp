@@ -286,11 +286,18 @@ u64 ks_scratch_words(const Context& c, u32 level, bool with_digits, bool with_ac
     return c.n * (L + (with_digits ? c.ndigits(level) * (L + k) : 0) + (with_acc ? 2 * (L + k) : 0) + 2 * k + 2 * L);
 }
 
-// Whether a batch of switches of `limbs` limbs in all takes the apply stage that leaves acc unused.
-bool ks_without_acc(const Context& c, u64 limbs) {
-    const bool small = limbs <= c.small_limbs;
-    if ((small ? c.fuse_ip_s : c.fuse_ip) && c.fuse_ip_possible()) return false;
-    return c.narrow_apply(2 * limbs, small ? c.conv_variant_s : c.md_variant());
+// How a batch of switches of `limbs` limbs in all runs: decided once, so that its scratch and its program agree
+// whatever another thread tunes meanwhile. narrow: the apply stage that leaves acc unused.
+struct KsRoute {
+    bool small, fuse, narrow;
+    u32 conv, md;  // conversion kernel variants of ModUp and mod_down
+};
+KsRoute ks_route(const Context& c, u64 limbs) {
+    KsRoute r{limbs <= c.small_limbs, false, false, c.conv_variant, c.md_variant()};
+    if (r.small) r.conv = r.md = c.conv_variant_s;
+    r.fuse = (r.small ? c.fuse_ip_s : c.fuse_ip) && c.fuse_ip_possible();
+    r.narrow = !r.fuse && c.narrow_apply(2 * limbs, r.md);
+    return r;
 }
 
 struct KsReq {
@@ -310,14 +317,16 @@ void check_switch(const Context& c, const Poly& d, const Ksk& key) {
     use(c, key);
 }
 
-// The program of a batch of requests (decompose + apply, one launch per stage), its scratch laid
-// out from base (ks_scratch_words per request, in request order; acc only with with_acc).
-static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
-                          const std::vector<AutJob>* pre = nullptr, bool with_acc = true, bool compact = false) {
+u64 limbs_of(const std::vector<KsReq>& reqs) {
     u64 limbs = 0;
     for (auto& r : reqs) limbs += r.d->level + 1;
-    const bool small = limbs <= c.small_limbs;
-    const bool fuse = (small ? c.fuse_ip_s : c.fuse_ip) && c.fuse_ip_possible();
+    return limbs;
+}
+
+// The program of a batch of requests (decompose + apply, one launch per stage), its scratch laid
+// out from base (ks_scratch_words per request, in request order; acc only with with_acc).
+static Program ks_program(Context& c, const std::vector<KsReq>& reqs, const KsRoute& route, u64* base, bool with_acc,
+                          const std::vector<AutJob>* pre = nullptr, bool compact = false) {
     std::vector<DecTask> dec;
     std::vector<ApplyTask> app;
     u64* p = base;
@@ -329,27 +338,29 @@ static Program ks_program(Context& c, const std::vector<KsReq>& reqs, u64* base,
         u64* y = acc + (with_acc ? 2 * (L + k) * c.n : 0);
         u64* z = y + 2 * k * c.n;
         p = z + 2 * L * c.n;
-        dec.push_back({r.d->data(), r.d->level, dig, x, false, fuse});
-        app.push_back({dig, r.d->level, 0, r.key, r.out_b, r.out_a, r.add_b, r.add_a, acc, y, z, r.d->data(), fuse});
+        dec.push_back({r.d->data(), r.d->level, dig, x, false, route.fuse});
+        app.push_back({dig, r.d->level, 0, r.key, r.out_b, r.out_a, r.add_b, r.add_a, acc, y, z, r.d->data(), route.fuse});
     }
     Program prog;  // one program (one graph when captured) per batched switch
     prog.compact = compact;
     if (pre) prog.step(S_AUTOMORPH, prog.add(*pre), (u32)pre->size());
-    c.prog_decompose(prog, dec, small ? c.conv_variant_s : c.conv_variant);
-    c.prog_apply(prog, app, small ? c.conv_variant_s : c.md_variant());
-    if (small) prog.set_conv_schedule(c.conv_variant_s, c.conv_tg_s);
+    c.prog_decompose(prog, dec, route.conv);
+    if (route.narrow && !compact)
+        c.prog_apply_narrow(prog, app);
+    else
+        c.prog_apply_wide(prog, app, route.md);
+    if (route.small) prog.set_conv_schedule(route.conv, c.conv_tg_s);
     return prog;
 }
 
 // decompose + apply for a batch of requests, in one launch per stage.
 static void run_ks_on(Context& c, const std::vector<KsReq>& reqs, hipStream_t s,
                       const std::vector<AutJob>* pre = nullptr) {
-    u64 total = 0, limbs = 0;
-    for (auto& r : reqs) limbs += r.d->level + 1;
-    const bool with_acc = !ks_without_acc(c, limbs);
-    for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true, with_acc);
+    const KsRoute route = ks_route(c, limbs_of(reqs));
+    u64 total = 0;
+    for (auto& r : reqs) total += ks_scratch_words(c, r.d->level, true, !route.narrow);
     BufPtr scratch = c.alloc(total, s);
-    c.execute(ks_program(c, reqs, scratch->ptr, pre, with_acc), s);
+    c.execute(ks_program(c, reqs, route, scratch->ptr, !route.narrow, pre), s);
     hip_check(hipGetLastError(), "key switch");
 }
 
@@ -471,10 +482,11 @@ void ks_switch_batch_static(Context& c, const std::vector<const Poly*>& ds, cons
         reqs.push_back({ds[i], &key, nullptr, nullptr, kb[i]->data(), ka[i]->data()});
     }
     // Workspace: the switches' scratch from the start, the descriptor bytes after it.
-    Program prog = ks_program(c, reqs, (u64*)c.static_scratch);
+    const KsRoute route = ks_route(c, limbs_of(reqs));
+    Program prog = ks_program(c, reqs, route, (u64*)c.static_scratch, true);
     const u64 desc_off = (scratch_bytes + 255) & ~(u64)255;
     if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)  // the last bytes of the workspace
-        prog = ks_program(c, reqs, (u64*)c.static_scratch, nullptr, true, true);
+        prog = ks_program(c, reqs, route, (u64*)c.static_scratch, true, nullptr, true);
     if (desc_off + prog.bytes.size() > CKH_STATIC_SCRATCH_BYTES)
         fail(CKH_ERR_INVALID_PARAMS, "batch needs more than the static workspace");
     hipStream_t s = c.stream();
@@ -1464,7 +1476,7 @@ u64 Evaluator::matvec_enc_workspace_bytes(u32 level, u32 baby, u32 giant) const 
 size_t Evaluator::enc_blocks_at_once(u32 level, u32 baby, u32 giant, u64 copies, u64 blocks, u64 rotated) const {
     const u64 q = level + 1, xs = 2 * q * copies;
     const u64 room = matvec_enc_workspace_bytes(level, baby, giant) / (ctx.n * 8);
-    auto scratch = [&](u64 m) { return m * ks_scratch_words(ctx, level, true, !ks_without_acc(ctx, m * q)) / ctx.n; };
+    auto scratch = [&](u64 m) { return m * ks_scratch_words(ctx, level, true, !ks_route(ctx, m * q).narrow) / ctx.n; };
     if (std::max({xs + 3 * q * blocks, 3 * q * blocks + scratch(blocks), 3 * q * blocks + 4 * q * rotated + scratch(rotated)}) <=
         room)
         return blocks;

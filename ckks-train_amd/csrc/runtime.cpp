@@ -992,18 +992,26 @@ void Context::prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 
 // keyswitch::apply_key (keyswitch.rs:230-309) for a batch: the inner product over Q_l * P, then
 // mod_down of both sums.
 void Context::prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const {
-    std::vector<IpJob> ip;
-    u32 max_l = 0;
-    std::vector<const Ksk*> keys;
     u64 targets = 0;
     bool any_fused = false;
     for (const ApplyTask& t : tasks) {
-        max_l = std::max(max_l, t.level + 1);
-        keys.push_back(t.key);
         targets += 2 * (t.level + 1);
         any_fused |= t.fused;
     }
-    if (!any_fused && !p.compact && narrow_apply(targets, md_variant)) return prog_apply_narrow(p, tasks);
+    if (!any_fused && narrow_apply(targets, md_variant))
+        prog_apply_narrow(p, tasks);
+    else
+        prog_apply_wide(p, tasks, md_variant);
+}
+
+void Context::prog_apply_wide(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const {
+    std::vector<IpJob> ip;
+    u32 max_l = 0;
+    std::vector<const Ksk*> keys;
+    for (const ApplyTask& t : tasks) {
+        max_l = std::max(max_l, t.level + 1);
+        keys.push_back(t.key);
+    }
     // Several tasks, each under a key of its own: the key words are read once. (A single switch may
     // be followed by another under the same key, which a cached copy serves.)
     std::sort(keys.begin(), keys.end());

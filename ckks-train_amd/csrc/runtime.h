@@ -282,8 +282,10 @@ class Context : public std::enable_shared_from_this<Context> {
     // variant: the conversion kernel variant the program's ModUp conversion will run with (it
     // decides whether the inverse NTT leaves the y form, tuning key "conv_yform").
     void prog_decompose(Program& p, const std::vector<DecTask>& tasks, u32 variant) const;
-    // md_variant: the conversion kernel variant of mod_down.
+    // md_variant: the conversion kernel variant of mod_down. prog_apply chooses between the two forms by the
+    // size (narrow_apply).
     void prog_apply(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const;
+    void prog_apply_wide(Program& p, const std::vector<ApplyTask>& tasks, u32 md_variant) const;
     void prog_apply_narrow(Program& p, const std::vector<ApplyTask>& tasks) const;
     void prog_mod_down(Program& p, const std::vector<MdTask>& tasks, u32 md_variant) const;
     void prog_rescale(Program& p, const std::vector<RescaleTask>& tasks) const;
@@ -306,8 +308,8 @@ class Context : public std::enable_shared_from_this<Context> {
     // (all of them: the sources are read once; 8 per workgroup took 17.54 against 16.83 ms per step of
     // 256 switches at N = 2^16, 3.65 against 3.60 ms for the 32 x 32 product at 2^15)
     // The variant of mod_down's conversions (P -> Q) in batched programs (tuning key
-    // "conv_variant_md"; 3 = conv_variant). 0 and 1 are the same vector kernel, 2 the matrix-core
-    // kernel (15.90 against 16.85 ms for 256 switches at N = 2^16).
+    // "conv_variant_md"; 3 = conv_variant). 0 and 1 are the same vector kernel (16.2 ms for 256 switches at
+    // N = 2^16), 2 the matrix-core kernel (17.0).
     u32 conv_variant_md = 1;
     u32 md_variant() const { return conv_variant_md < 3 ? conv_variant_md : conv_variant; }
     // Batched key switches of at most small_limbs input limbs in all (a single switch, a few
@@ -336,7 +338,9 @@ class Context : public std::enable_shared_from_this<Context> {
     // "graphs" (1 = on) and "graph_cache" (plans kept per context, least recently used evicted).
     u32 use_graphs = 1, graph_cache_max = 64;
     // Programs of at most this many launches are launched directly: a graph launch takes about 20 us
-    // of the host whatever it holds, a kernel launch 2.4 us.
+    // of the host whatever it holds, a kernel launch 2.4 us. By those figures the line would lie at 8,
+    // the launches of a single switch (32.1 us launched, 37.3 replayed at N = 2^12); it lies below them
+    // because a switch is counted on to be captured and replayed (ckh_graph_stats).
     static constexpr u32 DIRECT_LAUNCHES = 6;
     // The one-launch NTTs (tuning key "ntt_fused", 1 = on where the device's XCD layout was
     // verified at creation, off by default: measured no faster than the two launches on the key

@@ -290,6 +290,29 @@ static void allocation_hook_counts_by_size() {
     }
 }
 
+// A tuning changed by another thread between the sizing of a switch's scratch and its program does not change the
+// program's form: the one sized for (here without room for the sums) is the one that runs.
+static void a_switch_keeps_the_route_it_was_sized_for() {
+    auto c = make(12, 6, 2, 3);
+    c->set_tuning("graphs", 0);
+    KskPtr key = ksk_uniform(*c, 5, 0, 1);
+    PolyPtr d = poly_uniform(*c, 5, 0, true, 2, 0);
+    for (u32 which = 0; which < 2; ++which) {
+        model::ip_launches = model::ip_finish_launches = 0;
+        u32 at = 0;
+        model::on_malloc = [&](size_t) {  // the outputs, then the scratch
+            if (++at == 2) (which ? c->conv_yform : c->conv_cols) = 0;
+        };
+        ks_switch(*c, *d, *key);
+        model::on_malloc = nullptr;
+        CHECK(c->conv_cols == 0 || c->conv_yform == 0);
+        CHECK(model::ip_finish_launches == 1 && model::ip_launches == 0);
+        c->conv_cols = 1;
+        c->conv_yform = 7;
+        c->trim_pool(0);  // the next switch allocates again
+    }
+}
+
 // Memory written by copies still queued on one stream goes to no other stream's buffer, at random steps of both
 // streams; with `capture`, while a caller captures the first stream from time to time.
 static void cached_blocks(bool capture) {
@@ -434,6 +457,7 @@ int main(int argc, char** argv) {
         {"encrypted_products_stay_within_their_estimate", encrypted_products_stay_within_their_estimate},
         {"served_requests_are_admitted_by_what_they_hold", served_requests_are_admitted_by_what_they_hold},
         {"allocation_hook_counts_by_size", allocation_hook_counts_by_size},
+        {"a_switch_keeps_the_route_it_was_sized_for", a_switch_keeps_the_route_it_was_sized_for},
         {"cached_blocks_change_streams_after_their_use", cached_blocks_change_streams_after_their_use},
         {"cached_blocks_under_a_capture", cached_blocks_under_a_capture},
         {"staged_uploads_of_two_streams", staged_uploads_of_two_streams},

@@ -84,6 +84,7 @@ bool refuse_launch = false;
 float elapsed_ms = 1.0f;
 uint64_t records_while_capturing = 0;
 uint64_t destroyed_graphs = 0;
+uint64_t ip_launches = 0, ip_finish_launches = 0;
 size_t free_bytes = (size_t)1 << 40;
 
 std::function<void()> on_launch;
@@ -312,7 +313,10 @@ void ntt_fast_forward_rows_finish(const NttTables&, const LimbRef*, const Finish
 void ntt_fast_forward_fused(const NttTables&, const LimbRef*, u32, const FinishJob*, u32*, const FusedCfg&, hipStream_t) { K; }
 void ntt_fast_inverse_fused(const NttTables&, const LimbRef*, u32, u32*, const FusedCfg&, hipStream_t) { K; }
 void narrow_ip_inverse(const NttTables&, const IpInvJob*, const LimbRef*, u32, const YForm*, hipStream_t) { K; }
-void narrow_ip_finish(const NttTables&, const IpFinJob*, u32, hipStream_t) { K; }
+void narrow_ip_finish(const NttTables&, const IpFinJob*, u32, hipStream_t) {
+    ++model::ip_finish_launches;
+    K;
+}
 void rows_ip_launch(const NttTables&, const RowIpJob*, u32, hipStream_t) { K; }
 void rows_ip_fin_launch(const NttTables&, const RowIpFinJob*, u32, hipStream_t) { K; }
 void conv_cols_launch(const ConvTables&, const NttTables&, const ConvColRef*, u32, u32, hipStream_t) { K; }
@@ -322,7 +326,10 @@ void mul_sum_launch(const MulSumJob*, const MulSumTerm*, u32, const PrimeConst*,
 void tensor_sum_launch(const TensorJob*, const TensorTerm*, u32, const PrimeConst*, u32, hipStream_t) { K; }
 void tensor_launch(const TensorTerm&, u64*, u32, const PrimeConst*, u32, hipStream_t) { K; }
 void add_sum_launch(const AddSumJob*, const u64* const*, u32, const PrimeConst*, u32, hipStream_t) { K; }
-void inner_product_launch(const IpJob*, u32, const PrimeConst*, u32, bool, hipStream_t) { K; }
+void inner_product_launch(const IpJob*, u32, const PrimeConst*, u32, bool, hipStream_t) {
+    ++model::ip_launches;
+    K;
+}
 void stream_copy_launch(const void*, void*, u64, hipStream_t) { K; }
 void copy_launch(const LimbRef*, u32, u32, hipStream_t) { K; }
 void pointwise_launch(PwOp, const u64*, const u64*, u64*, u32, u32, const PrimeConst*, u32, hipStream_t) { K; }

@@ -28,6 +28,7 @@ extern uint64_t records_while_capturing;  // event records on a stream that a ca
 extern uint64_t destroyed_graphs;       // executable graphs destroyed so far
 extern size_t free_bytes;               // what hipMemGetInfo reports
 
+extern uint64_t ip_launches, ip_finish_launches;  // of the inner product, and of the one inside the finish
 extern std::function<void()> on_launch;  // called at every kernel launch
 extern std::function<void(size_t)> on_malloc;  // called with the bytes of every device allocation
 

@@ -43,6 +43,7 @@ def exe(tmp_path_factory):
     "encrypted_products_stay_within_their_estimate",
     "served_requests_are_admitted_by_what_they_hold",
     "allocation_hook_counts_by_size",
+    "a_switch_keeps_the_route_it_was_sized_for",
     "cached_blocks_change_streams_after_their_use",
     "cached_blocks_under_a_capture",
     "staged_uploads_of_two_streams",
