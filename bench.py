@@ -462,7 +462,7 @@ def main():
         return
     levels = workload_levels()
     # --batched-only runs without the autotuner, at the choices it makes on this workload
-    tuning = ({"ntt_chunk_fwd": 0, "ntt_chunk_inv": 0, "conv_variant": 0, "conv_tg": 24, "fuse_ip": 1,
+    tuning = ({"ntt_chunk_fwd": 0, "ntt_chunk_inv": 0, "conv_variant": 0, "conv_tg": 32, "fuse_ip": 1,
                "conv_variant_md": 1} if args.batched_only else ctx.autotune())
     if args.batched_only:
         for kv in args.tune:

@@ -69,12 +69,18 @@ struct ConvTgt {
 };
 
 enum : u32 { TGT_INT = 0, TGT_FP = 1, TGT_SPLIT = 2 };
+// k = rint(F) has to be within 2 of T / r (WRAP_SMALL) or of T / (2^11 r) (WRAP_LARGE). In units of 1, with at
+// most 8 terms y c, c centered (|c| < r / 2) and its quotient rounded to nearest:
 // WRAP_SMALL: every source below 2^50, any r. The sums run over y_j - 2^49 (the constant takes
-// 2^49 sum_j c_j): the partial sums of F stay below 2^51, their roundings, those of the c_j / r and
-// of the e term add up to less than 0.9 for 6 sources and 1.2 for 8, so with rint |T - k r| < 2 r.
-// WRAP_LARGE: r below 2^50, sources below 2^60: F, in units of 2^11, is off by at most 1.7 with
-// its rounding (8 sources: 2,400 from the sums and their factors, 1,024 from rint, of 4,096), so
-// |T - 2^11 k r| < 2^12 r < 2^62; a second quotient of that remainder by r gives the residue.
+// 2^49 sum_j c_j), so |y_j - 2^49| <= 2^49 and F grows by at most 2^48 per term, to 2^51 (where adding
+// 1.5 2^52 still rounds to an integer). Errors: each c_j / r is off by 2^-55 at most, 2^-6 in its
+// term, 1/8 in all; the FMAs round to half an ulp of 2^48 .. 2^51, 1/32 + 1/16 + 1/16 + 1/8 for the
+// first four and 1/8 for each further one (1/4 where the last crosses 2^51), 0.91 in all; the e term
+// 2^-50; rint 1/2. That is 1.53 for 8 sources (1.13 for 6), so |T - k r| < 2 r.
+// WRAP_LARGE: r below 2^50, sources below 2^60, c_j / (2^11 r) at most 2^-12: F grows by 2^48 per
+// term, the rounding of y_j to f64 (2^6) adds 2^-6 per term to the same errors, and the terms left
+// out of F (e, the constant: below 5 r, 2^-8): 1.66 for 8 sources, so |T - 2^11 k r| < 2^12 r < 2^62;
+// a second quotient of that remainder by r gives the residue.
 enum : u32 { WRAP_NONE = 0, WRAP_SMALL = 1, WRAP_LARGE = 2 };
 constexpr u64 WRAP_CENTER = 1ull << 49;
 constexpr double WRAP_ROUND = 6755399441055744.0;        // 1.5 2^52: adding it rounds to an integer
@@ -229,7 +235,8 @@ CKH_DEV u64 conv_dot60(const Tgt& g, const PrimeConst& C, const u64 (&y)[MAXS], 
 // output words of targets [t0, t1). MAXS bounds the plan's sources. Per-target constants are read
 // through cst (the scalar cache on the device). Bound by VALU before the single-quotient form, now
 // by memory and latency: ModUp conversions of 256 switches at N = 2^16 (50-bit sources) 2.92 ->
-// 1.64 ms, mod_down's (60-bit sources) 2.12 -> 0.98 ms per step.
+// 1.64 ms, mod_down's (60-bit sources) 2.12 -> 0.98 ms per step. (The unnamed parameter chose between two
+// forms of the sums that are both gone; the replay still names it.)
 template <u32 MAXS, bool = false>
 CKH_DEV void conv_coeff(const ConvSrc* srcs, const ConvTgt* tgts, const PrimeConst* pcs, const ConvPlan& P,
                         const u64* in_p, u64* out_p, u32 n, u32 c, u32 t0, u32 t1, bool yform) {

@@ -89,19 +89,20 @@ void *ckh_stream_handle(ckh_context *ctx);
  * the batched key-switch schedule, and the small-batch schedule on one top-level switch); writes
  * a JSON report (candidates and choices) to report (may be NULL). */
 ckh_status ckh_autotune(ckh_context *ctx, char *report, size_t report_len);
-/* The autotuner's key-switch candidates (conversion kernel variant, row-pass fusion, then the
- * inverse-NTT chunk against none) timed on the caller's own batch: n NTT-form polynomials switched under key (no counterpart in the
- * reference). Keeps the fastest; writes the timings as JSON to report (may be NULL). */
+/* The autotuner's key-switch candidates (conversion kernel variant, targets per workgroup, row-pass fusion,
+ * then the inverse-NTT chunk against none) timed on the caller's own batch: n NTT-form polynomials switched
+ * under key (no counterpart in the reference). Keeps the fastest, the present choice unless another beats it;
+ * writes the timings as JSON to report (may be NULL). */
 ckh_status ckh_autotune_ks(ckh_context *ctx, uint32_t n, const ckh_poly *const *d, const ckh_ksk *key,
                            char *report, size_t report_len);
 /* Forces one tuning value: "ntt_chunk_fwd", "ntt_chunk_inv" (limbs per launch, 0 = all);
  * "graphs" (1 = replay repeated launch sequences from captured hipGraphs, the default; 0 = launch
  * directly); "graph_cache" (captured sequences kept per context); "conv_variant" (base conversion:
- * 0 or 1 = vector kernel, 2 = int8 matrix-core kernel); "conv_variant_md" (the variant of mod_down's conversions in batched
- * switches, default 1; 3 = conv_variant); "conv_tg" (targets per base-conversion
- * workgroup); "conv_cols" (1, the default: base conversions of few sources or few targets fused with
- * their targets' column pass); "fuse_ip" (1 = row pass fused into the inner product); "fuse_fin" (1, the default:
- * with fuse_ip, mod_down's finish of the Q limbs in the same kernel, so the inner-product sums
+ * 0 or 1 = vector kernel, 2 = int8 matrix-core kernel); "conv_variant_md" (the variant of mod_down's
+ * conversions in batched switches, default 1; 3 = conv_variant); "conv_tg" (targets per base-conversion
+ * workgroup, default 32); "conv_cols" (1, the default: base conversions of few sources or few targets fused
+ * with their targets' column pass); "fuse_ip" (1 = row pass fused into the inner product); "fuse_fin" (1, the
+ * default: with fuse_ip, mod_down's finish of the Q limbs in the same kernel, so the inner-product sums
  * never reach memory); "conv_yform" (a mask of the conversions whose inverse NTT ends with the
  * conversion's first product, [x + h] (Q/q_j)^-1, folded into its last stage: 1 = ModUp on the
  * vector kernel, 2 = mod_down, 4 = ModUp on the matrix-core kernel; default 7); "small_limbs" (batched
@@ -380,7 +381,9 @@ ckh_status ckh_slot_to_coeff(ckh_evaluator *ev, const ckh_ct *re, const ckh_ct *
 ckh_status ckh_matvec_enc_batch(ckh_evaluator *ev, uint32_t n, const ckh_ct *const *xs,
                                 const ckh_ct *const *const *entries, const ckh_bsgs_shape *shapes,
                                 ckh_ct **outs);
-/* CudaEvaluator::matvec_enc_workspace_bytes (evaluator.rs:403-410) for this engine. */
+/* CudaEvaluator::matvec_enc_workspace_bytes (evaluator.rs:403-410) for this engine: an upper estimate, in whole
+ * limbs, of what one product in the optimised form holds at its peak beyond its inputs; the product takes
+ * its giant blocks in as many groups as keep within it. */
 ckh_status ckh_matvec_enc_workspace_bytes(ckh_evaluator *ev, uint32_t level, uint32_t baby, uint32_t giant,
                                           uint64_t *bytes);
 /* n relinearizations in batched launches (bit-identical to n ckh_relinearize calls). */
