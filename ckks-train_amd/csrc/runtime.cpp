@@ -131,8 +131,10 @@ Context::~Context() {
     retired_.clear();
     for (auto s : streams_) (void)hipStreamSynchronize(s);
     cache_release(0);
-    for (auto& m : marks_)
-        if (m.second.ev) (void)hipEventDestroy(m.second.ev);
+    for (auto& m : marks_) {
+        for (auto& e : m.second.pending) (void)hipEventDestroy(e.first);
+        for (hipEvent_t e : m.second.spare) (void)hipEventDestroy(e);
+    }
     for (void* a : perm_allocs_) (void)hipFree(a);
     for (auto s : streams_) (void)hipStreamDestroy(s);
     if (capture_stream_) (void)hipStreamDestroy(capture_stream_);
@@ -173,28 +175,32 @@ static bool capturing(hipStream_t s) {
     return true;
 }
 
-// A mark covering every free queued on s so far (none while s is being captured).
-void Context::mark_record(Mark& m, hipStream_t s) {
-    if (capturing(s)) return;
-    if (!m.ev && hipEventCreateWithFlags(&m.ev, hipEventDisableTiming) != hipSuccess) {
+// A mark covering every free queued on s so far (none while s is being captured, or MARKS are under way).
+void Context::mark_record(Marks& m, hipStream_t s) {
+    if (m.pending.size() == MARKS || capturing(s)) return;
+    hipEvent_t ev = nullptr;
+    if (!m.spare.empty()) {
+        ev = m.spare.back();
+        m.spare.pop_back();
+    } else if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipGetLastError();
-        m.ev = nullptr;
         return;
     }
-    if (hipEventRecord(m.ev, s) != hipSuccess) {
+    if (hipEventRecord(ev, s) == hipSuccess) {
+        m.pending.push_back({ev, m.freed});
+    } else {
         (void)hipGetLastError();
-        return;
+        m.spare.push_back(ev);
     }
-    m.seq = m.freed;
-    m.pending = true;
 }
 
 // Whether the stream's seq-th free and the work before it have completed.
-bool Context::mark_covers(Mark& m, u64 seq) {
-    if (m.done >= seq) return true;
-    if (!m.pending || hipEventQuery(m.ev) != hipSuccess) return false;
-    m.done = m.seq;
-    m.pending = false;
+bool Context::mark_covers(Marks& m, u64 seq) {
+    while (m.done < seq && !m.pending.empty() && hipEventQuery(m.pending.front().first) == hipSuccess) {
+        m.done = std::max(m.done, m.pending.front().second);
+        m.spare.push_back(m.pending.front().first);
+        m.pending.pop_front();
+    }
     return m.done >= seq;
 }
 
@@ -207,18 +213,25 @@ void* Context::cache_take(size_t& cls, hipStream_t s) {
     // The class itself first, then larger classes up to twice its size (a fitting free block is
     // reused instead of growing the cache with another class); within a class, a block last used
     // on s, else one whose last use is known to have completed.
-    std::vector<hipStream_t> wanted;  // streams whose blocks could not be taken yet
+    std::vector<hipStream_t> wanted;  // streams still at work, whose blocks could not be taken yet
+    auto covered = [&](const Cached& b) {
+        Marks& m = marks_[b.s];
+        if (mark_covers(m, b.seq)) return true;
+        if (std::find(wanted.begin(), wanted.end(), b.s) != wanted.end()) return false;
+        if (!capturing(b.s) && hipStreamQuery(b.s) == hipSuccess) {  // idle: every free so far is covered
+            m.done = m.freed;
+            return true;
+        }
+        wanted.push_back(b.s);
+        return false;
+    };
     for (auto it = cache_.lower_bound(cls); it != cache_.end() && it->first <= 2 * cls; ++it) {
         std::vector<Cached>& v = it->second;
         size_t pick = v.size();
         for (size_t i = 0; i < v.size() && pick == v.size(); ++i)
             if (v[i].s == s) pick = i;
-        for (size_t i = 0; i < v.size() && pick == v.size(); ++i) {
-            if (mark_covers(marks_[v[i].s], v[i].seq))
-                pick = i;
-            else if (std::find(wanted.begin(), wanted.end(), v[i].s) == wanted.end())
-                wanted.push_back(v[i].s);
-        }
+        for (size_t i = 0; i < v.size() && pick == v.size(); ++i)
+            if (covered(v[i])) pick = i;
         if (pick == v.size()) continue;
         void* p = v[pick].p;
         v[pick] = v.back();
@@ -227,10 +240,7 @@ void* Context::cache_take(size_t& cls, hipStream_t s) {
         cache_bytes_ -= cls;
         return p;
     }
-    for (hipStream_t w : wanted) {  // for the next request
-        Mark& m = marks_[w];
-        if (!m.pending) mark_record(m, w);
-    }
+    for (hipStream_t w : wanted) mark_record(marks_[w], w);  // for the next request
     return nullptr;
 }
 
@@ -243,10 +253,13 @@ void Context::cache_put(void* p, size_t cls, hipStream_t s) {
         (void)hipFree(p);
         return;
     }
-    Mark& m = marks_[s];
+    Marks& m = marks_[s];
     cache_[cls].push_back({p, s, ++m.freed});
     cache_bytes_ += cls;
-    if (cache_multi_ && m.freed % MARK_EVERY == 0 && (!m.pending || mark_covers(m, m.seq))) mark_record(m, s);
+    if (cache_multi_ && m.freed % MARK_EVERY == 0) {
+        mark_covers(m, m.freed);  // takes back the events of completed marks
+        mark_record(m, s);
+    }
 }
 
 // Returns cached blocks to the driver, largest first, until at most keep_bytes stay cached.

@@ -442,31 +442,33 @@ class Context : public std::enable_shared_from_this<Context> {
 
     std::vector<hipStream_t> streams_;  // caller streams, then the service streams
     // The block cache of pool mode 1: free blocks per size class, each with the stream of its last use
-    // and its number among the blocks freed on that stream. Another stream may take a block once a
-    // mark (an event recorded after its free) has completed; a mark covers every earlier free of its
-    // stream. Marks are recorded only when another stream asks, and every MARK_EVERY frees once a
-    // second stream has allocated: an event per free took about 4.5 us of the stream each.
+    // and its number among the blocks freed on that stream. Another stream may take a block once that
+    // stream is idle, or a mark (an event recorded after the block's free) has completed; a mark covers
+    // every earlier free of its stream. Marks are recorded when another stream asks in vain, and every
+    // MARK_EVERY frees once a second stream has allocated, up to MARKS of them under way: an event per
+    // free took about 4.5 us of the stream each. (Sixty served bursts at N = 2^15 leave 4.5-5.1 GB cached,
+    // with an event per free 4.0-4.6; 9.4 with one mark under way and without asking whether a stream is idle.)
     struct Cached {
         void* p;
         hipStream_t s;
         u64 seq;
     };
-    struct Mark {
-        hipEvent_t ev = nullptr;
-        u64 freed = 0;    // blocks freed on the stream so far
-        u64 seq = 0;      // the pending mark covers frees up to here
-        u64 done = 0;     // frees known complete
-        bool pending = false;
+    struct Marks {  // of one stream
+        u64 freed = 0;  // blocks freed on it so far
+        u64 done = 0;   // frees known complete
+        std::deque<std::pair<hipEvent_t, u64>> pending;  // marks under way and the frees that each covers
+        std::vector<hipEvent_t> spare;
     };
     static constexpr u64 MARK_EVERY = 8;
+    static constexpr size_t MARKS = 32;
     std::mutex cache_mu_;
     std::map<size_t, std::vector<Cached>> cache_;
-    std::map<hipStream_t, Mark> marks_;
+    std::map<hipStream_t, Marks> marks_;
     hipStream_t cache_stream_ = nullptr;  // the first stream that allocated
     bool cache_multi_ = false;            // a second one has
     u64 cache_bytes_ = 0, cache_limit_ = ~0ull;
-    void mark_record(Mark& m, hipStream_t s);
-    bool mark_covers(Mark& m, u64 seq);
+    void mark_record(Marks& m, hipStream_t s);
+    bool mark_covers(Marks& m, u64 seq);
     // A free block of class cls or of a larger class up to 2 cls (cls is set to the block's).
     void* cache_take(size_t& cls, hipStream_t s);
     void cache_put(void* p, size_t cls, hipStream_t s);

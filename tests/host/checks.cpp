@@ -370,6 +370,53 @@ static void cached_blocks(bool capture) {
 static void cached_blocks_change_streams_after_their_use() { cached_blocks(false); }
 static void cached_blocks_under_a_capture() { cached_blocks(true); }
 
+// Another stream's blocks are taken as soon as that stream is idle, or has passed the frees of earlier batches
+// while a later one still runs: no block comes from the driver.
+static void blocks_of_finished_work_are_taken() {
+    auto c = make(12, 6, 2, 3, 2);
+    hipStream_t s[2];
+    for (u32 i = 0; i < 2; ++i) {
+        c->set_stream(i);
+        s[i] = c->stream();
+        c->alloc(16);  // both streams allocate
+    }
+    std::vector<u64> src(4096);
+    auto use_and_free = [&](u32 stream, u32 blocks) {
+        c->set_stream(stream);
+        std::vector<BufPtr> b;
+        for (u32 k = 0; k < blocks; ++k) {
+            b.push_back(c->alloc(src.size()));
+            model::queue_copy(b.back()->ptr, src.data(), src.size() * 8, s[stream]);
+        }
+    };
+    use_and_free(0, 4);
+    while (model::step(s[0])) {}
+    uint64_t before = c->stat_mallocs;
+    use_and_free(1, 4);  // stream 0 is idle
+    CHECK(c->stat_mallocs == before);
+    while (model::step(s[1])) {}
+
+    std::vector<size_t> queued;  // after each batch of 24 blocks
+    for (u32 batch = 0; batch < 3; ++batch) {
+        c->set_stream(0);
+        std::vector<BufPtr> b;
+        for (u32 k = 0; k < 24; ++k) b.push_back(c->alloc(src.size() << batch));  // a class of its own each
+        for (auto& x : b) model::queue_copy(x->ptr, src.data(), src.size() * 8, s[0]);
+        b.clear();
+        queued.push_back(model::pending(s[0]));
+    }
+    const size_t left = queued[2] - queued[1];  // the third batch still to run
+    while (model::pending(s[0]) > left) model::step(s[0]);
+    before = c->stat_mallocs;
+    for (u32 batch = 0; batch < 2; ++batch) {
+        c->set_stream(1);
+        std::vector<BufPtr> b;
+        for (u32 k = 0; k < 16; ++k) b.push_back(c->alloc(src.size() << batch));
+    }
+    CHECK(c->stat_mallocs == before, "%llu", (unsigned long long)(c->stat_mallocs - before));
+    c->synchronize_all();
+}
+
 // Staged uploads of two streams arrive whole over many laps of the ring, at random steps of both streams; with
 // `capture`, while a caller captures the first stream from time to time.
 static void staged_uploads(bool capture) {
@@ -460,6 +507,7 @@ int main(int argc, char** argv) {
         {"a_switch_keeps_the_route_it_was_sized_for", a_switch_keeps_the_route_it_was_sized_for},
         {"cached_blocks_change_streams_after_their_use", cached_blocks_change_streams_after_their_use},
         {"cached_blocks_under_a_capture", cached_blocks_under_a_capture},
+        {"blocks_of_finished_work_are_taken", blocks_of_finished_work_are_taken},
         {"staged_uploads_of_two_streams", staged_uploads_of_two_streams},
         {"staged_uploads_under_a_capture", staged_uploads_under_a_capture},
         {"plans_evicted_under_a_capture", plans_evicted_under_a_capture},

@@ -172,6 +172,11 @@ hipError_t hipStreamSynchronize(hipStream_t s) {
     drain(s, [] { return false; });
     OK;
 }
+hipError_t hipStreamQuery(hipStream_t s) {
+    LOCKED;
+    if (s->capturing) return fail_with(hipErrorStreamCaptureUnsupported);
+    return s->q.empty() ? hipSuccess : hipErrorNotReady;
+}
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* st) {
     LOCKED;
     *st = s->capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;

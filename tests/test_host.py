@@ -46,6 +46,7 @@ def exe(tmp_path_factory):
     "a_switch_keeps_the_route_it_was_sized_for",
     "cached_blocks_change_streams_after_their_use",
     "cached_blocks_under_a_capture",
+    "blocks_of_finished_work_are_taken",
     "staged_uploads_of_two_streams",
     "staged_uploads_under_a_capture",
     "plans_evicted_under_a_capture",
