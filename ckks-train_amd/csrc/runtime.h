@@ -235,7 +235,7 @@ class Context : public std::enable_shared_from_this<Context> {
     // (four per power of two), kept for reuse instead of returned to the driver (whose pools
     // released memory at synchronizations and stalled the host for the whole device queue when
     // growing under load); a freed block serves its own stream at once (stream order) and any
-    // other stream once an event recorded after its last use has completed; 0 = the device's
+    // other stream once its last use is known to have completed; 0 = the device's
     // default stream-ordered pool with the runtime's reuse rules (which may hand a block to
     // another stream before its free has run, behind a dependency the runtime inserts).
     BufPtr alloc(size_t words, hipStream_t s);
